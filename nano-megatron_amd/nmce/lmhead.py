@@ -13,9 +13,10 @@ with ``x`` the (already TP-mapped, model.py:188-191) hidden state and ``W`` the
 LM head's vocabulary shard ``[V/tp, H]``. The loss and its gradients with
 respect to ``x`` and ``W`` are those of the two-step reference, but the
 ``[tokens, V/tp]`` logits are never stored: the one-pass path holds the
-bf16 exponentials of one chunk of tokens at a time (by default at most a
-quarter of them and at most 2 GiB), the recomputing path two bf16 copies of
-one vocabulary chunk's logit gradient.
+bf16 exponentials of one chunk of tokens at a time (by default at most 2 GiB,
+and at most a quarter of the tokens unless every token at once takes no more
+memory), the recomputing path two bf16 copies of one vocabulary chunk's logit
+gradient.
 
 When a gradient is wanted (grad mode on, ``x`` or ``W`` requiring grad) the
 wrapper takes the one-pass path: the forward goes through the tokens in
@@ -72,7 +73,10 @@ DEFAULT_VOCAB_CHUNK = 32768
 # allocated. dW is then accumulated in fp32 across the chunks by the GEMM
 # epilogue (measured on one MI355X: [16384, 4096] x [128256, 4096] 3.4% slower
 # in four chunks of 4096 tokens than in one chunk, [16384, 3072] x
-# [256000, 3072] 1.6%).
+# [256000, 3072] 1.6%). The accumulator is 4 V H bytes whatever the tokens, so
+# with few tokens per unit of H it outgrows every token's exponentials: then
+# one chunk, which needs no accumulator, is the smaller workspace and the
+# faster pass (one_pass_token_chunk).
 CHUNK_BUDGET_BYTES = 2 << 30
 CHUNK_FRACTION = 4
 
@@ -85,6 +89,28 @@ def default_token_chunk(n_tokens: int, vocab_local: int) -> int:
     chunk = max(256, -(-quarter // 256) * 256)
     fit = max(256, CHUNK_BUDGET_BYTES // (2 * max(1, vocab_local)) // 256 * 256)
     return min(chunk, fit, max(n_tokens, 1))
+
+
+def one_pass_token_chunk(n_tokens: int, hidden: int, vocab_local: int) -> int:
+    """The chunk the one-pass path takes when the caller names none: every
+    token where that workspace is no larger than the one of
+    ``default_token_chunk``'s chunks, and else those chunks.
+
+    Against chunks of ``c`` tokens, one chunk of all ``n`` holds ``n - c`` more
+    tokens' exponentials (2 V bytes each), partial statistics (12 bytes per 128
+    vocabulary rows) and transposed hidden rows (2 H), and saves the fp32 dW
+    accumulator (4 V H): about n <= 2.6 H. It is also the faster side of the
+    line everywhere, since each further chunk reads and writes the accumulator
+    and shortens dW's K to the chunk ([4096, 4096] x [128256, 4096]: 12.9 ms
+    in four chunks, 10.7 in one; [2103, 1600] x [50257, 1600]: 1.60 ms in
+    three, 1.13 in one; [512, 768] x [50304, 768]: 0.54 in two, 0.32 in one). The line depends on sizes alone, so every tensor-parallel rank
+    takes the same chunks."""
+    chunk = default_token_chunk(n_tokens, vocab_local)
+    more = (n_tokens - chunk) * (2 * vocab_local + 12 * -(-vocab_local // 128) + 2 * hidden)
+    if more <= 4 * vocab_local * hidden and 2 * vocab_local * n_tokens <= CHUNK_BUDGET_BYTES:
+        return max(n_tokens, 1)
+    return chunk
+
 
 _ALIGN = 64  # hidden size granularity of the GEMM kernels
 
@@ -170,7 +196,7 @@ class _LMHeadVocabParallelCrossEntropyMean(torch.autograd.Function):
             ctx.weight_shape = weight.shape
             return torch.empty(0, dtype=torch.float32, device=dev).mean()
         ctx.empty = False
-        chunk = default_token_chunk(n, V) if token_chunk is None else int(token_chunk)
+        chunk = one_pass_token_chunk(n, hp, V) if token_chunk is None else int(token_chunk)
         L = _fused_layout(lib, n, hp, V, chunk)
         ws = _workspace(L["total"], dev)
         args = (x.data_ptr(), w.data_ptr(), _lib.NMCE_BF16, n, hp, V)
@@ -371,9 +397,9 @@ def lmhead_vocab_parallel_cross_entropy(
 
     When a gradient is wanted the forward is one pass (module docstring),
     going through ``token_chunk`` tokens at a time (default
-    ``default_token_chunk``: a quarter of the tokens, within
-    ``CHUNK_BUDGET_BYTES``; pass the token count to hold every token's
-    exponentials at once) and assuming the upstream value held by
+    ``one_pass_token_chunk``: a quarter of the tokens, or all of them where
+    that takes no more memory, within ``CHUNK_BUDGET_BYTES``; pass the token
+    count to hold every token's exponentials at once) and assuming the upstream value held by
     ``upstream_hint`` (a one-element fp32 device tensor; default: one per
     call site). ``one_pass=False`` selects the forward that keeps only the
     row statistics, with a backward that recomputes the logits in chunks of
@@ -456,7 +482,7 @@ class FusedParallelLMHead(torch.nn.Module):
         self.weight.tensor_parallel_sharded = True
         self.sequence_parallel = bool(getattr(config, "sequence_parallel", False))
         self.vocab_chunk = None  # backward chunk; None = DEFAULT_VOCAB_CHUNK
-        self.token_chunk = None  # one-pass chunk; None = default_token_chunk
+        self.token_chunk = None  # one-pass chunk; None = one_pass_token_chunk
         # The upstream value the one-pass forward assumes, per module and
         # device (created on first use on that device).
         self._hints: dict = {}

@@ -239,6 +239,37 @@ def test_one_pass_token_chunk_budget(lib):
     assert all(r % 256 == 0 for r in regions) and regions == sorted(regions)
 
 
+@pytest.mark.parametrize("n,h,v,whole", [(512, 768, 50304, True), (2103, 1600, 50257, True),
+                                         (4096, 4096, 128256, True), (8192, 4096, 128256, True),
+                                         (8704, 4096, 128256, False),   # 2 GiB of exponentials
+                                         (16384, 4096, 128256, False), (16384, 3072, 256000, False),
+                                         (2048, 512, 32000, False), (1280, 512, 32000, True),
+                                         (100, 64, 1000, True), (1, 64, 1, True)])
+def test_one_pass_chunk_holds_every_token_where_smaller(lib, n, h, v, whole):
+    """The one-pass path's own chunk is every token exactly where that
+    workspace is no larger than the quarter chunks' (their fp32 dW accumulator
+    against the further tokens' exponentials) and its exponentials fit the
+    budget; otherwise it is default_token_chunk's. The regions are the
+    library's layout, without the split dX product's partials (their count is
+    the device's)."""
+    import ctypes
+    from nmce import _lib as L
+    from nmce import lmhead
+    buf = (ctypes.c_int64 * L.NMCE_LMHEAD_FUSED_LAYOUT_FIELDS)()
+
+    def held(chunk):
+        assert lib.nmce_lmhead_ce_fused_layout(n, h, v, chunk, ctypes.addressof(buf)) == 0
+        return buf[0] - (buf[11] - buf[9])
+
+    quarter = lmhead.default_token_chunk(n, v)
+    chunk = lmhead.one_pass_token_chunk(n, h, v)
+    assert chunk == (n if whole else quarter)
+    if chunk != quarter:
+        # the rule counts whole tokens; the layout pads them to 64
+        assert held(chunk) <= held(quarter) + 64 * (2 * v + 2 * h) + 4096
+        assert 2 * v * chunk <= lmhead.CHUNK_BUDGET_BYTES
+
+
 def test_fused_dx_split_choice(lib):
     """A chunk's dX product (tokens x H tiles, K = the padded vocabulary) is
     split over K when its 256x256 tiles leave compute units idle; the fp32
