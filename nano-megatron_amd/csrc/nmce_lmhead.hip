@@ -1232,7 +1232,8 @@ __global__ __launch_bounds__(256) void lmhead_dz_rescale_kernel(
 // A product split over K (gemm_store_kernel, splits > 1) summed into bf16:
 // out[r * ldo + c] = bf16(sum_s part[s][r][c]) for r < M, c < N (N % 4 == 0),
 // with the partials [splits][M][N] fp32 contiguous. The splits are added in
-// order, so the result does not depend on how the GEMM was scheduled.
+// order, so the result does not depend on how the GEMM was scheduled; eight
+// ranges' loads are in flight at a time (up to 256 ranges are summed).
 __global__ __launch_bounds__(256) void split_sum_bf16_kernel(const float* __restrict__ part,
                                                              int splits, int64_t M, int64_t N,
                                                              uint16_t* __restrict__ out,
@@ -1242,6 +1243,7 @@ __global__ __launch_bounds__(256) void split_sum_bf16_kernel(const float* __rest
   if (i >= total) return;
   float a[4];
   Elem<float>::unpack(load_stream(reinterpret_cast<const u32x4*>(part + i)), a);
+#pragma unroll 8
   for (int sp = 1; sp < splits; ++sp) {
     float b[4];
     Elem<float>::unpack(load_stream(reinterpret_cast<const u32x4*>(part + sp * total + i)), b);
@@ -1506,12 +1508,26 @@ int device_cus() {
 // first `k_valid` k) whose rounds of tiles leave at most 5% of the compute
 // units idle, else the fewest with the least idle share. ks gets the range
 // length (a multiple of kBK).
-int choose_splits(int64_t tiles, int64_t K, int64_t k_valid, int cus, int64_t* ks) {
+//
+// Where even 8 ranges leave part of one round idle (fewer than 32 tiles on
+// 256 compute units: small batches, whose K is the whole vocabulary), the
+// product is one round of long serial K walks, and more ranges (up to one
+// round, each at least 1024 long) shorten them: a range costs kStageUs per
+// stage of its K, and the `out` partial values of each range a write and a
+// read at kPartialBytesPerUs. [512, 768] x [50304, 768] (6 tiles, K = 50432):
+// 126 + 5.6 us (product + sum) at 8 ranges, 43 + 9.4 at the model's 33.
+int choose_splits(int64_t tiles, int64_t out, int64_t K, int64_t k_valid, int cus, int64_t* ks) {
+  constexpr double kStageUs = 1.25;
+  constexpr double kPartialBytesPerUs = 4e6;
+  const auto valid = [&](int s, int64_t least) {
+    const int64_t len = round_up((K + s - 1) / s, kBK);
+    return s == 1 || (K / s >= least && (s - 1) * len < K && (s - 1) * len < k_valid);
+  };
   int best = 1;
+  int more = 1;
   double best_idle = 1e30;
   for (int s = 1; s <= 8; ++s) {
-    const int64_t len = round_up((K + s - 1) / s, kBK);
-    if (s > 1 && (K / s < 2048 || (s - 1) * len >= K || (s - 1) * len >= k_valid)) break;
+    if (!valid(s, 2048)) break;
     const int64_t t = tiles * s;
     const int64_t rounds = (t + cus - 1) / cus;
     const double idle = static_cast<double>(rounds * cus) / static_cast<double>(t);
@@ -1523,6 +1539,18 @@ int choose_splits(int64_t tiles, int64_t K, int64_t k_valid, int cus, int64_t* k
       best_idle = idle;
       best = s;
     }
+  }
+  if (tiles * 8 < cus) {
+    double best_us = 1e30;
+    for (int s = best; s <= cus / tiles && (s == best || valid(s, 1024)); ++s) {
+      const double us = kStageUs * static_cast<double>((K + s - 1) / s) / kBK +
+                        8.0 * static_cast<double>(out) * s / kPartialBytesPerUs;
+      if (us < best_us) {
+        best_us = us;
+        more = s;
+      }
+    }
+    best = more;
   }
   *ks = best == 1 ? K : round_up((K + best - 1) / best, kBK);
   return best;
@@ -1551,7 +1579,7 @@ FusedLayout fused_layout(int64_t n, int64_t h, int64_t v, int64_t token_chunk) {
   L.vpad = round_up(v, kBM);
   L.nb = fwd_partial_blocks(v);
   const int64_t dx_tiles = ((L.chunk + kBM - 1) / kBM) * ((h + kBN - 1) / kBN);
-  L.dx_splits = choose_splits(dx_tiles, L.vpad, v, device_cus(), &L.dx_ks);
+  L.dx_splits = choose_splits(dx_tiles, L.chunk * h, L.vpad, v, device_cus(), &L.dx_ks);
   int64_t off = 0;
   L.off_pt = off; off += align256(L.vpad * L.ldt * 2);
   L.off_part = off; off += align256(3 * L.nb * L.chunk * 4);

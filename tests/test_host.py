@@ -282,7 +282,11 @@ def test_fused_dx_split_choice(lib):
     buf = (ctypes.c_int64 * L.NMCE_LMHEAD_FUSED_LAYOUT_FIELDS)()
     for n, h, v, ch, splits in ((16384, 4096, 128256, 4096, 1), (16384, 3072, 256000, 4096, 4),
                                 (16384, 3072, 256000, 2048, 8), (16384, 3072, 256000, 16384, 1),
-                                (300, 128, 777, 256, 1)):
+                                (300, 128, 777, 256, 1),
+                                # fewer than 32 tiles: up to one round of ranges
+                                # of at least 1024
+                                (512, 768, 50304, 512, 33), (100, 64, 20000, 100, 19),
+                                (700, 1600, 50257, 700, 12), (256, 4096, 128256, 256, 16)):
         assert lib.nmce_lmhead_ce_fused_layout(n, h, v, ch, ctypes.addressof(buf)) == 0
         assert buf[10] == splits, (n, h, v, ch, buf[10])
         want = (splits * ch * h * 4 + 255) // 256 * 256 if splits > 1 else 0

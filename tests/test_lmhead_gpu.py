@@ -737,7 +737,7 @@ def test_one_pass_fused_against_oracle(n, h, v, chunk):
     chunk, several with a short last one, a hidden size padded to 64, a
     vocabulary of one row and one that ends a row into a 128-row block. The
     last two split a chunk's dX product over K (its tiles are too few for the
-    device): 8 equal ranges at V = 20000, and 3 at V = 7800 with a shorter last
+    device): 19 ranges at V = 20000, and 7 at V = 7800 with a shorter last
     range and a hidden size of 320 (a 64-column edge tile)."""
     import nmce
     print(f"[gpu] one-pass fused n={n} h={h} v={v} chunk={chunk}", flush=True)
@@ -751,6 +751,29 @@ def test_one_pass_fused_against_oracle(n, h, v, chunk):
     loss.backward()
     rl, _, rdx, rdw = fp64_reference(x, w, t)
     assert abs(loss.item() - rl.mean()) <= 1e-5 * abs(rl.mean()) + 1e-30
+    check_grad(xd.grad.float().cpu().numpy(), rdx, "dH")
+    check_grad(wd.grad.float().cpu().numpy(), rdw, "dW")
+
+
+@pytest.mark.parametrize("n,h,v", [(1, 64, 16640), (100, 64, 20000), (513, 320, 33001),
+                                   (257, 192, 9217)])
+def test_one_pass_fused_many_k_ranges(n, h, v):
+    """Few tokens: the dX product's K (the vocabulary) in as many ranges as one
+    round of compute units holds (16, 19, 26 and 9 with 256 of them; the ranges
+    past a multiple of eight are summed by the unrolled loop's remainder), the
+    last one shorter and ending in the vocabulary's padding, against the fp64
+    closed form."""
+    import nmce
+    print(f"[gpu] one-pass fused many ranges n={n} h={h} v={v}", flush=True)
+    x, w, t = make_inputs(n, h, v, seed=n + v, w_std=0.5)
+    xd = x.to(DEV).requires_grad_(True)
+    wd = w.to(DEV).requires_grad_(True)
+    loss = nmce.lmhead_vocab_parallel_cross_entropy(
+        xd, wd, t.to(DEV), 0, v, nmce.ParallelContext.single(),
+        upstream_hint=torch.ones(1, dtype=torch.float32, device=DEV))
+    loss.backward()
+    rl, _, rdx, rdw = fp64_reference(x, w, t)
+    assert abs(loss.item() - rl.mean()) <= 1e-5 * abs(rl.mean())
     check_grad(xd.grad.float().cpu().numpy(), rdx, "dH")
     check_grad(wd.grad.float().cpu().numpy(), rdw, "dW")
 
