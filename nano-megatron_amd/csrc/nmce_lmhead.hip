@@ -36,37 +36,35 @@
 // so 6 N V H flops in all, against 8 N V H for the recomputing backward, and
 // no copy of anything the size of the logits or the weight.
 //
-// Tokens are the MFMA N dimension in the loss GEMMs: the 32x32 accumulator
-// gives each lane 16 vocabulary rows of a single token, so the per-token
-// reductions are mostly in-register, with one cross-half shuffle.
+// Tokens are the MFMA N dimension in the loss GEMMs: the 16x16 accumulators
+// give each lane 32 vocabulary rows of each of 8 tokens, so the per-token
+// reductions are mostly in-register, with one merge over four lane groups.
 //
-// Main loop: a 256x256 output tile per 512-lane workgroup (eight waves, 2x4,
-// two per SIMD, each 128x64 = 8 accumulators of 32x32 held in AGPRs), K in
-// steps of 64.
-// Each wave reads its next fragments from LDS under the MFMAs of the current
-// ones (two register sets, one LDS read pinned after each MFMA). Operand tiles
-// move HBM/L2 -> LDS with 16-byte direct-to-LDS loads (MUBUF
-// buffer_load_dwordx4 ... lds, no VGPR staging), double-buffered. A
-// K-contiguous operand sits in rows of 128 bytes with the 16-byte chunks
-// XOR-swizzled by ((row >> 1) & 7). gfx950's LDS has 64 banks, so a
-// ds_read_b128 serves 16 lanes (16 consecutive rows of a fragment) per cycle;
-// this swizzle puts those 16 rows on 16 distinct 16-byte bank groups (row
-// parity picks the half of the banks, the swizzled chunk the group). An
-// MN-contiguous operand sits in 64 k-rows of 512 bytes and its fragments come
-// from gfx950's transposing LDS read, ds_read_b64_tr_b16, with the same
-// fragments, so the two layouts give the same bits. Workgroups are mapped to
-// tiles so that each XCD (one L2) owns a contiguous band of tiles walked in
-// groups that share operands.
+// Main loop: a 256x256 output tile per 256-lane workgroup (four waves, 2x2,
+// one per SIMD, each 128x128 = 64 accumulators of 16x16 held in AGPRs), K in
+// steps of 64. Each wave reads its next fragments from LDS under the MFMAs of
+// the current ones (two register sets), and the reads and the next stages'
+// loads have fixed places between the MFMAs. Operand tiles move HBM/L2 -> LDS
+// with 16-byte direct-to-LDS loads (MUBUF buffer_load_dwordx4 ... lds, no VGPR
+// staging), A triple- and B double-buffered. A K-contiguous operand sits in
+// rows of 128 bytes with the 16-byte chunks XOR-swizzled by ((row >> 1) & 7).
+// gfx950's LDS has 64 banks, so a ds_read_b128 serves 16 lanes (16 consecutive
+// rows of a fragment) per cycle; this swizzle puts those 16 rows on 16 distinct
+// 16-byte bank groups (row parity picks the half of the banks, the swizzled
+// chunk the group). An MN-contiguous operand sits in 64 k-rows of 512 bytes
+// and its fragments come from gfx950's transposing LDS read,
+// ds_read_b64_tr_b16, with the same fragments, so the two layouts give the
+// same bits. Workgroups are mapped to tiles so that each XCD (one L2) owns a
+// contiguous band of tiles walked in groups that share operands.
 //
 // The dZ epilogue stages the bf16 tile in the freed LDS with the token index
-// XOR-swizzled by the vocabulary-pair block, so that both output layouts leave
-// as coalesced 512-byte row segments.
+// XOR-swizzled by the vocabulary pair, so that both output layouts leave as
+// coalesced 512-byte row segments.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <mutex>
 #include <type_traits>
-
 
 #include "nmce.h"
 #include "nmce_device.h"
@@ -76,70 +74,228 @@ namespace nmce {
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 constexpr int kBM = 256;          // tile rows (GEMM M)
 constexpr int kBN = 256;          // tile columns (GEMM N)
 constexpr int kBK = 64;           // K per stage (128 bytes of bf16 per row)
-// Eight waves, two per SIMD, each 128 x 64 of the tile (2 x 4). One wave per
-// SIMD with 128 x 128 each leaves every load and LDS latency exposed without a
-// hand-scheduled instruction stream (measured 10-15% slower).
+// Four waves, one per SIMD, each 128 x 128 of the tile (2 x 2). Against eight
+// waves of 128 x 64 (two per SIMD) a wave reads a third less from LDS per
+// product, and that and the smaller MFMA (below) are what a chip at its power
+// cap turns into clock: 1190 -> 1525 TFLOP/s on 16384 x 16384 x 8192, 1175 ->
+// 1538 on 4096 x 4096 x 65536.
 constexpr int kWavesM = 2;
-constexpr int kWavesN = 4;
-constexpr int kThreads = 64 * kWavesM * kWavesN;
+constexpr int kWavesN = 2;
+constexpr int kWaves = kWavesM * kWavesN;
+constexpr int kThreads = 64 * kWaves;
 constexpr int kWaveM = kBM / kWavesM;  // 128
-constexpr int kWaveN = kBN / kWavesN;  // 64
-constexpr int kFM = kWaveM / 32;       // 4 accumulators down
-constexpr int kFN = kWaveN / 32;       // 2 accumulators across
-constexpr int kStageA = kBM * kBK * 2;  // bytes
-constexpr int kStageB = kBN * kBK * 2;
-constexpr int kStage = kStageA + kStageB;
-constexpr int kLdsBytes = 2 * kStage;  // dynamic LDS: 128 KiB of the 160 KiB per CU
-// 1 KiB LDS blocks (8 rows x 128 B) per stage and per wave.
-constexpr int kBlocksA = kBM / 8;
-constexpr int kBlocksB = kBN / 8;
-constexpr int kBlocksPerWave = (kBlocksA + kBlocksB) / (kWavesM * kWavesN);
-static_assert(kBlocksA % kBlocksPerWave == 0, "a wave loads blocks of one operand only");
-// Tile rows per raster group inside an XCD band (measured): groups of 4 for
-// the forward, which walks the whole weight shard (hundreds of tile rows),
-// and for the one-pass backward products (dX 1%, dW 1.5-2% faster than with
-// 8); groups of 8 for the chunked recomputation and the plain GEMM.
-constexpr int kGroupM = 8;
-constexpr int kGroupMStats = 4;
-constexpr int kGroupMProducts = 4;
+constexpr int kWaveN = kBN / kWavesN;  // 128
+constexpr int kF = kWaveM / 16;        // 8 fragments of 16 rows (columns) a side
+static_assert(kWaveM == kWaveN, "a wave's tile is square");
+constexpr int kStage = kBM * kBK * 2;  // bytes of one operand's stage: 32 KiB
+static_assert(kBM == kBN, "the operands' stages have one size");
+// A's stages in three buffers, B's in two: all of a compute unit's LDS. A
+// stage's A loads are then issued before the barrier that frees B's buffer,
+// which spreads a stage's loads over the whole K step (gemm_mainloop).
+constexpr int kBufsA = 3;
+constexpr int kBufsB = 2;
+constexpr int kLdsBytes = (kBufsA + kBufsB) * kStage;  // dynamic LDS: 160 KiB
+static_assert(kLdsBytes <= 160 * 1024, "the stages fit a compute unit's LDS");
+// 1 KiB LDS blocks per stage and operand, and per wave of them.
+constexpr int kBlocks = kStage / 1024;
+constexpr int kBlocksPerWave = kBlocks / kWaves;
+// Tile rows per raster group inside an XCD band: 4 of 2, 4 and 8 is the
+// fastest for the products of many tiles (16384 x 16384 x 8192: 1545 TFLOP/s
+// against 1476 with 8; the [16384, 4096] x [128256, 4096] step 39.3 ms against
+// 39.6 with 8 and 39.9 with 2) and no slower than 1.5% elsewhere.
+constexpr int kGroupM = 4;
 constexpr int kXcds = 8;
 constexpr float kMaxFloorL = -1.0e38f;
-
 
 // Partial statistics cover this many vocabulary rows (one wave's rows).
 constexpr int kPartialRows = kWaveM;
 
+// A wave's 128 x 128 results: c[i][j] is the 16 x 16 block of rows 16 i and
+// columns 16 j; lane l holds column l % 16, rows 4 (l / 16) + e of it.
 struct Acc {
-  f32x16_t c[kFM][kFN];
+  f32x4_t c[kF][kF];
 };
 
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// acc += A B^T of one 16 x 16 block, K = 32, as an instruction that updates
+// its accumulator registers in place. With the builtin the compiler gives 64
+// accumulators results in other registers than their inputs and moves them
+// back (360 moves per K step, 1055-1200 instead of 1440 TFLOP/s). The 16 x 16
+// form moves half the accumulator bytes per product that the 32 x 32 x 16 form
+// does, with the same sums: 1440 against 1240 TFLOP/s in the same loop.
+__device__ __forceinline__ void mfma_16x16x32(f32x4_t& c, const bf16x8_t& a, const bf16x8_t& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
 
 // Tile index for this workgroup. The dispatcher deals workgroups to the 8 XCDs
 // round-robin (block b runs on XCD b % 8); give each XCD a contiguous band of
-// tile ids, and inside the band walk groups of group_m tile rows column by
+// tile ids, and inside the band walk groups of kGroupM tile rows column by
 // column, so the tiles that run together on one L2 share A and B stripes.
-__device__ __forceinline__ void tile_coords(int group_m, int tiles_m, int tiles_n, int& tm,
-                                            int& tn) {
+__device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn) {
   const int total = tiles_m * tiles_n;
   const int b = blockIdx.x;
   const int xcd = b % kXcds;
   const int q = total / kXcds, r = total % kXcds;
   const int tid = xcd * q + (xcd < r ? xcd : r) + b / kXcds;
-  const int group = group_m * tiles_n;
+  const int group = kGroupM * tiles_n;
   const int g = tid / group;
-  const int first_m = g * group_m;
-  const int gm = (tiles_m - first_m) < group_m ? (tiles_m - first_m) : group_m;
+  const int first_m = g * kGroupM;
+  const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
   const int in_g = tid - g * group;
   tm = first_m + in_g % gm;
   tn = in_g / gm;
 }
+
+// The loads of one operand's stages (64 k each) into LDS by this wave: 1 KiB
+// blocks blk0 .. blk0 + 7, one MUBUF direct-to-LDS load each.
+//
+// K-contiguous (kMN = false): a block is 8 rows of 128 bytes; lane p writes
+// row p / 8, physical chunk p % 8, which holds logical chunk
+// (p % 8) ^ ((row >> 1) & 7). The K position goes in the scalar offset, so a
+// stage needs no per-lane arithmetic. MN-contiguous: a block is k-rows 2 b and
+// 2 b + 1 of 512 bytes; lane p writes row 2 b + p / 32, physical chunk p % 32,
+// which holds logical chunk (p % 32) ^ 4 (row & 3) ^ 2 ((row >> 3) & 1). The
+// resource's base moves by 64 rows per stage (the offset would pass 32 bits).
+//
+// The buffer resource has no stride and no range limit (every offset is
+// clamped in bounds) and gfx9's data format word.
+template <bool kMN>
+struct StageLoads {
+  i32x4_t rsrc;
+  const char* base;
+  int64_t row_bytes, krows;
+  uint32_t off[kBlocksPerWave];
+  int row0, last_chunk, lane, soff;
+
+  __device__ __forceinline__ void set_base(const char* p) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    rsrc[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(a & 0xffffffffu));
+    rsrc[1] = __builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32));
+  }
+  __device__ __forceinline__ int krow(int j) const { return row0 + 2 * j; }
+  __device__ __forceinline__ int chunk_bytes(int j) const {
+    int chunk = (lane & 31) ^ (4 * (krow(j) & 3)) ^ (2 * ((krow(j) >> 3) & 1));
+    if (chunk > last_chunk) chunk = last_chunk;
+    return chunk * 16;
+  }
+  // first: the operand's element at the tile's first row (column), k = 0;
+  // rows: the operand's rows (columns) from there on; krows_: its k-rows (kMN).
+  __device__ __forceinline__ void init(const uint16_t* first, int64_t ld, int64_t rows,
+                                       int64_t krows_, int wave, int lane_) {
+    lane = lane_;
+    base = reinterpret_cast<const char*>(first);
+    row_bytes = ld * 2;
+    krows = krows_;
+    soff = 0;
+    const int blk0 = wave * kBlocksPerWave;
+    if constexpr (kMN) {
+      row0 = 2 * blk0 + (lane >> 5);
+      const int64_t last = (rows + 7) / 8 - 1;  // >= 0
+      last_chunk = static_cast<int>(last < 31 ? last : 31);
+#pragma unroll
+      for (int j = 0; j < kBlocksPerWave; ++j)
+        off[j] = static_cast<uint32_t>(krow(j) * row_bytes + chunk_bytes(j));
+    } else {
+#pragma unroll
+      for (int j = 0; j < kBlocksPerWave; ++j) {
+        const int tile_row = (blk0 + j) * 8 + (lane >> 3);
+        const int chunk = (lane & 7) ^ ((tile_row >> 1) & 7);
+        const int64_t r = tile_row < rows ? tile_row : rows - 1;
+        off[j] = static_cast<uint32_t>(r * row_bytes + chunk * 16);
+      }
+    }
+    set_base(base);
+    rsrc[2] = -1;
+    rsrc[3] = 0x00020000;
+  }
+  // The number of leading stages whose k-rows all exist.
+  __device__ __forceinline__ int full_stages(int stages) const {
+    if constexpr (!kMN) return stages;
+    const int64_t f = krows / kBK;
+    return f < stages ? static_cast<int>(f) : stages;
+  }
+  // Stage kt (all of its k-rows exist) is the next one to be loaded.
+  __device__ __forceinline__ void at(int kt) {
+    if constexpr (kMN)
+      set_base(base + kt * (kBK * row_bytes));
+    else
+      soff = __builtin_amdgcn_readfirstlane(kt * (kBK * 2));
+  }
+  __device__ __forceinline__ void load(char* dst, int j) const {
+    raw_buffer_load_lds(rsrc, (lds_void_t*)(dst + j * 1024), 16, static_cast<int>(off[j]), soff, 0,
+                        0);
+  }
+  // A whole stage at once, whose k-rows may end before it does (kMN): those
+  // past the last are read as the last.
+  __device__ __forceinline__ void stage(char* dst, int kt) {
+    const int64_t k0 = static_cast<int64_t>(kt) * kBK;
+    if (kMN && k0 + kBK > krows) {
+      const int64_t b0 = k0 < krows ? k0 : krows - 1;
+      set_base(base + b0 * row_bytes);
+#pragma unroll
+      for (int j = 0; j < kBlocksPerWave; ++j) {
+        int64_t row = k0 + krow(j);
+        if (row > krows - 1) row = krows - 1;
+        raw_buffer_load_lds(rsrc, (lds_void_t*)(dst + j * 1024), 16,
+                            static_cast<int>((row - b0) * row_bytes) + chunk_bytes(j), 0, 0, 0);
+      }
+      return;
+    }
+    at(kt);
+#pragma unroll
+    for (int j = 0; j < kBlocksPerWave; ++j) load(dst, j);
+  }
+};
+
+// One operand's fragments of 16 rows (columns) and 32 k from its stage: lane l
+// gets row l % 16, k 8 (l / 16) .. + 7. K-contiguous: one ds_read_b128 of the
+// row's logical chunk 4 s + l / 16 (sub-step s); 16 consecutive rows of one
+// chunk are on distinct 16-byte bank groups. MN-contiguous: two
+// ds_read_b64_tr_b16, each giving a lane 4 consecutive k of its column (in a
+// group of 16 lanes, lanes 4 r .. 4 r + 3 read the 16 columns of k-row r and
+// lane j receives column j of the 4 rows). Lane 16 g + 4 r + u reads k-row
+// 8 g + r (+ 4 for the second, + 32 s), columns 4 u .. 4 u + 3 of the
+// fragment; the swizzle puts the 8 k-rows that half of the lanes read (rows
+// 0-3 and 8-11) on distinct 32 bytes of the 256 that the banks span.
+template <bool kMN>
+struct Frags {
+  int off0, off1;  // K-contiguous: the lane's byte offset in sub-step 0 and 1
+  int lane;
+  int col0;        // first row (column) of the wave's 128
+
+  __device__ __forceinline__ void init(int first, int lane_) {
+    lane = lane_;
+    col0 = first;
+    const int r = lane & 15, q = lane >> 4;
+    off0 = (first + r) * 128 + ((q ^ ((r >> 1) & 7)) << 4);
+    off1 = (first + r) * 128 + (((4 + q) ^ ((r >> 1) & 7)) << 4);
+  }
+  // K-contiguous: the whole fragment f of sub-step s.
+  __device__ __forceinline__ bf16x8_t read(const char* st, int s, int f) const {
+    return *reinterpret_cast<const bf16x8_t*>(st + (s ? off1 : off0) + f * 16 * 128);
+  }
+  // MN-contiguous: its half h (k 4 h .. 4 h + 3 of the lane's eight).
+  __device__ __forceinline__ s16x4_t read_half(const char* st, int s, int f, int h) const {
+    const int g = lane >> 4, r = (lane >> 2) & 3, u = lane & 3;
+    // k-rows 8 g + r and 8 g + 4 + r share the swizzle (row & 3 = r,
+    // (row >> 3) & 1 = g & 1); 32 s does not change it either.
+    const int chunk = (((col0 + 16 * f) >> 3) + (u >> 1)) ^ (4 * r) ^ (2 * (g & 1));
+    const char* p = st + (8 * g + r) * 512 + chunk * 16 + 8 * (u & 1) + s * (32 * 512);
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4_t*)(p + h * (4 * 512)));
+  }
+  static __device__ __forceinline__ bf16x8_t join(const s16x4_t& lo, const s16x4_t& hi) {
+    typedef short s16x8_t __attribute__((ext_vector_type(8)));
+    const s16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8_t, v);
+  }
+};
 
 // The main loop: acc = A[m0:m0+256, 0:K] * B[n0:n0+256, 0:K]^T, each operand
 // K-contiguous (A[m, k] at A + m * lda + k; kAMN = false) or MN-contiguous
@@ -154,15 +310,18 @@ __device__ __forceinline__ void tile_coords(int group_m, int tiles_m, int tiles_
 // 16-byte aligned A and B, and 256 * ld * 2 < 2^32 bytes (K-contiguous) or
 // 64 * ld * 2 < 2^32 bytes (MN-contiguous).
 //
-// LDS per stage and operand: 32 KiB. K-contiguous: 256 rows of 128 bytes (the
-// stage's 64 k), 16-byte chunks XOR-swizzled by (row >> 1) & 7, one
-// ds_read_b128 per fragment. MN-contiguous: 64 k-rows of 512 bytes (256
-// columns), chunk c of row k at c ^ 4 (k & 3); a fragment is two
-// ds_read_b64_tr_b16, each giving a lane 4 consecutive k of its column (in a
-// group of 16 lanes, lanes 4r .. 4r + 3 read 16 columns of k-row r and lane j
-// receives column j of the 4 rows), and the swizzle puts the 8 k-rows of one
-// read on distinct 16-byte bank groups, two rows per group.
-template <bool kAMN, bool kBMN, bool kStagger = true>
+// A K step is two sub-steps of 32 k, 64 MFMAs each. One wave per SIMD has
+// nothing else to hide a wait, so the stream is fixed: after every third MFMA
+// one fragment of the next sub-step is read from LDS (the 16 reads are done
+// by the 48th of 64 MFMAs, so none is waited for), and after every sixth one
+// of the stage's 16 loads is issued (issued together they fill the address
+// unit's queue and the wave stalls: 1370 against 1450 TFLOP/s with one every
+// second MFMA, 1525 spread over both sub-steps, on 16384 x 16384 x 8192).
+// Stage kt + 2's A goes into the buffer that stage kt - 1 had, during the first
+// sub-step of kt; its B into stage kt's buffer, after the barrier at which every
+// wave has read the last of stage kt. That barrier waits for all but the wave's
+// newest eight loads (stage kt + 2's A).
+template <bool kAMN, bool kBMN>
 __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda,
                                               int64_t M, const uint16_t* __restrict__ B,
                                               int64_t ldb, int64_t N, int64_t K, int64_t m0,
@@ -174,287 +333,196 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / kWavesN, wn = wave % kWavesN;
 
-#pragma unroll
-  for (int i = 0; i < kFM; ++i)
-#pragma unroll
-    for (int j = 0; j < kFN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc.c[i][j][e] = 0.0f;
+  StageLoads<kAMN> la;
+  StageLoads<kBMN> lb;
+  la.init(kAMN ? A + m0 : A + m0 * lda, lda, M - m0, ka_rows, wave, lane);
+  lb.init(kBMN ? B + n0 : B + n0 * ldb, ldb, N - n0, kb_rows, wave, lane);
+  Frags<kAMN> fa;
+  Frags<kBMN> fb;
+  fa.init(wm * kWaveM, lane);
+  fb.init(wn * kWaveN, lane);
 
-  // ---- load plan: this wave fills kBlocksPerWave 1 KiB blocks per stage ----
-  // K-contiguous: lane p of a block writes LDS bytes [16p, 16p+16): row p/8 of
-  // the block, physical chunk p%8, which holds logical chunk
-  // (p%8) ^ ((row >> 1) & 7). MN-contiguous: a block is k-rows 2b and 2b + 1,
-  // lane p writes row 2b + p/32, physical chunk p%32, which holds logical
-  // chunk (p%32) ^ 4 (row & 3).
-  const int first_block = wave * kBlocksPerWave;
-  const bool load_a = first_block < kBlocksA;
-  const bool mn_op = load_a ? kAMN : kBMN;
-  const char* gbase;
-  int64_t ld_op, rows_op, krows_op;
-  int lds_op;
-  int blk0;
-  if (load_a) {
-    gbase = reinterpret_cast<const char*>(kAMN ? A + m0 : A + m0 * lda);
-    ld_op = lda; rows_op = M - m0; krows_op = ka_rows; lds_op = 0; blk0 = first_block;
-  } else {
-    gbase = reinterpret_cast<const char*>(kBMN ? B + n0 : B + n0 * ldb);
-    ld_op = ldb; rows_op = N - n0; krows_op = kb_rows; lds_op = kStageA;
-    blk0 = first_block - kBlocksA;
+  char* const lds_b = lds + kBufsA * kStage;
+  const int lds_w = wave * (kBlocksPerWave * 1024);
+  const int kt_n = static_cast<int>(K / kBK);
+
+  la.stage(lds + lds_w, 0);
+  lb.stage(lds_b + lds_w, 0);
+  if (kt_n > 1) {
+    la.stage(lds + kStage + lds_w, 1);
+    lb.stage(lds_b + kStage + lds_w, 1);
   }
-  uint32_t goff[kBlocksPerWave];
-  // MN-contiguous: the lane's k-row within the stage and its (clamped)
-  // logical chunk, as a byte offset.
-  auto mn_row = [&](int j) { return 2 * (blk0 + j) + (lane >> 5); };
-  auto mn_chunk_bytes = [&](int j) {
-    const int last_chunk = static_cast<int>((rows_op + 7) / 8 - 1);  // >= 0
-    int chunk = (lane & 31) ^ (4 * (mn_row(j) & 3));
-    if (chunk > last_chunk) chunk = last_chunk;
-    return chunk * 16;
-  };
-  if ((kAMN || kBMN) && mn_op) {
 #pragma unroll
-    for (int j = 0; j < kBlocksPerWave; ++j)
-      goff[j] = static_cast<uint32_t>(mn_row(j) * ld_op * 2 + mn_chunk_bytes(j));
-  } else {
-    const int row_lane = lane >> 3;
+  for (int i = 0; i < kF; ++i)
 #pragma unroll
-    for (int j = 0; j < kBlocksPerWave; ++j) {
-      const int tile_row = (blk0 + j) * 8 + row_lane;
-      const int chunk = (lane & 7) ^ ((tile_row >> 1) & 7);
-      int64_t r = tile_row;
-      if (r > rows_op - 1) r = rows_op - 1;
-      goff[j] = static_cast<uint32_t>((r * ld_op + chunk * 8) * 2);
-    }
-  }
-
-  // Buffer resource on this wave's operand tile: base = the tile's first row,
-  // no stride, no range limit (every offset above is clamped in bounds), gfx9
-  // data format word. A K-contiguous operand's K position goes in the scalar
-  // offset, so a stage's loads need no per-lane address arithmetic; an
-  // MN-contiguous one moves the base by 64 rows per stage instead (the offset
-  // would pass 32 bits).
-  auto set_base = [](i32x4_t& r, const char* base) {
-    const uint64_t gaddr = reinterpret_cast<uint64_t>(base);
-    r[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(gaddr & 0xffffffffu));
-    r[1] = __builtin_amdgcn_readfirstlane(static_cast<int>(gaddr >> 32));
-  };
-  i32x4_t rsrc;
-  set_base(rsrc, gbase);
-  rsrc[2] = -1;
-  rsrc[3] = 0x00020000;
-  auto issue = [&](int stage, int64_t k0) {
-    char* l = lds + stage * kStage + lds_op + blk0 * 1024;
-    int soff = 0;
-    if ((kAMN || kBMN) && mn_op) {
-      if (k0 + kBK > krows_op) {
-        // The stage runs past the operand's k-rows: read from row
-        // min(k0, krows - 1) and clamp each lane's row to the last one.
-        const int64_t b0 = k0 < krows_op ? k0 : krows_op - 1;
-        set_base(rsrc, gbase + b0 * ld_op * 2);
+    for (int j = 0; j < kF; ++j) acc.c[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // The compiler does not know that mfma_16x16x32 reads them as an MFMA does:
+  // the zeros are written, and have settled, before the first one.
 #pragma unroll
-        for (int j = 0; j < kBlocksPerWave; ++j) {
-          int64_t row = k0 + mn_row(j);
-          if (row > krows_op - 1) row = krows_op - 1;
-          const int off = static_cast<int>((row - b0) * ld_op * 2) + mn_chunk_bytes(j);
-          raw_buffer_load_lds(rsrc, (lds_void_t*)(l + j * 1024), 16, off, 0, 0, 0);
-        }
-        return;
-      }
-      set_base(rsrc, gbase + k0 * ld_op * 2);
-    } else {
-      soff = __builtin_amdgcn_readfirstlane(static_cast<int>(k0 * 2));
-    }
+  for (int i = 0; i < kF; ++i)
 #pragma unroll
-    for (int j = 0; j < kBlocksPerWave; ++j)
-      raw_buffer_load_lds(rsrc, (lds_void_t*)(l + j * 1024), 16, static_cast<int>(goff[j]), soff,
-                          0, 0);
-  };
-
-  // ---- fragment plan: 32x32x16 operands, 8 bf16 per lane (k 8 * (lane / 32)
-  // .. + 7 of the sub-step, row or column lane % 32 of the fragment) --------
-  // K-contiguous A fragment fm, K sub-step s: row wm*128 + 32*fm + lane%32,
-  // logical chunk 2*s + lane/32 of that row (16 bytes).
-  const int frow = lane & 31;
-  const int fhalf = lane >> 5;
-  const int a_row_off = (wm * kWaveM + frow) * 128;
-  const int b_row_off = kStageA + (wn * kWaveN + frow) * 128;
-  int xo[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) xo[s] = (((2 * s + fhalf) ^ ((frow >> 1) & 7)) << 4);
-  // MN-contiguous: lane 16 g + 4 r + u reads k-row 8 (g / 2) + r (+ 16 s + 4 h
-  // for sub-step s and half h), columns 16 (g % 2) + 4 u .. + 3 of the
-  // fragment: chunk (fragment base) / 8 + 2 (g % 2) + u / 2, 8 bytes in.
-  const int tg = lane >> 4, tr = (lane >> 2) & 3, tu = lane & 3;
-  const int tr_lane = (8 * (tg >> 1) + tr) * 512 + 8 * (tu & 1);
-  auto tr_off = [&](int col0) {  // col0: first column of the fragment, multiple of 32
-    return tr_lane + ((((col0 >> 3) + 2 * (tg & 1) + (tu >> 1)) ^ (4 * tr)) << 4);
-  };
-  int a_tr[kFM], b_tr[kFN];
-#pragma unroll
-  for (int i = 0; i < kFM; ++i) a_tr[i] = tr_off(wm * kWaveM + 32 * i);
-#pragma unroll
-  for (int j = 0; j < kFN; ++j) b_tr[j] = kStageA + tr_off(wn * kWaveN + 32 * j);
-
-  typedef short s16x4_t __attribute__((ext_vector_type(4)));
-  typedef short s16x8_t __attribute__((ext_vector_type(8)));
-  auto read_tr = [](const char* p, int off) {
-    const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) s16x4_t*)(p + off));
-    const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) s16x4_t*)(p + off + 4 * 512));
-    const s16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(bf16x8_t, v);
-  };
-
-  // Fragments of one K sub-step; two sets alternate so that the LDS reads of
-  // sub-step s+1 are in flight under the 16 MFMAs of sub-step s.
-  struct Frags {
-    bf16x8_t a[kFM];
-    bf16x8_t b[kFN];
-  };
-  auto read_a = [&](const char* st, int s, Frags& f, int i) {
-    if constexpr (kAMN)
-      f.a[i] = read_tr(st + 16 * s * 512, a_tr[i]);
-    else
-      f.a[i] = *reinterpret_cast<const bf16x8_t*>(st + a_row_off + i * 32 * 128 + xo[s]);
-  };
-  auto read_b = [&](const char* st, int s, Frags& f, int j) {
-    if constexpr (kBMN)
-      f.b[j] = read_tr(st + 16 * s * 512, b_tr[j]);
-    else
-      f.b[j] = *reinterpret_cast<const bf16x8_t*>(st + b_row_off + j * 32 * 128 + xo[s]);
-  };
-  auto load_frags = [&](const char* st, int s, Frags& f) {
-    if constexpr (kAMN || kBMN) {
-      // In the order the MFMAs first use them (B0 A0, B1, A1, A2, ...), so
-      // that each MFMA of the next sub-step waits only for its own reads:
-      // +3% on the product with both operands MN-contiguous (two transposing
-      // reads per fragment), +0.3% with one; -0.4% with none, which keeps
-      // the A-first order.
-      constexpr int kMax = kFM > kFN ? kFM : kFN;
-#pragma unroll
-      for (int i = 0; i < kMax; ++i) {
-        if (i < kFN) read_b(st, s, f, i);
-        if (i < kFM) read_a(st, s, f, i);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kFM; ++i) read_a(st, s, f, i);
-#pragma unroll
-      for (int j = 0; j < kFN; ++j) read_b(st, s, f, j);
-    }
-  };
-  auto mma = [&](const Frags& f) {
-#pragma unroll
-    for (int i = 0; i < kFM; ++i)
-#pragma unroll
-      for (int j = 0; j < kFN; ++j) {
-        acc.c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i], f.b[j], acc.c[i][j], 0, 0, 0);
-        // Keep the accumulators in AGPRs: the MFMAs then read and write them
-        // there and the arch VGPRs serve the fragment reads alone.
-        asm volatile("" : "+a"(acc.c[i][j]));
-      }
-  };
-
-  // One sub-step of the pipeline: the LDS reads of the next fragments
-  // interleaved with the 8 MFMAs of the current ones (one read per MFMA, two
-  // for the first MFMAs when an operand takes two reads per fragment), so
-  // that the compiler neither serialises them nor reuses registers early.
-  constexpr int kReads = (kAMN ? 2 : 1) * kFM + (kBMN ? 2 : 1) * kFN;
-  constexpr int kMfmas = kFM * kFN;
-  static_assert(kReads <= 2 * kMfmas, "at most two reads per MFMA");
-  auto step = [&](const char* st_next, int s_next, Frags& next, const Frags& cur) {
-    load_frags(st_next, s_next, next);
-    mma(cur);
-    if constexpr (kReads <= kMfmas) {
-#pragma unroll
-      for (int i = 0; i < kReads; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kReads, 0);
-    } else {
-#pragma unroll
-      for (int i = 0; i < kReads - kMfmas; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // 2 LDS reads
-      }
-#pragma unroll
-      for (int i = 0; i < 2 * kMfmas - kReads; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
-      }
-    }
-  };
-
-  // Stage kt lives in LDS buffer kt & 1. Loads run one stage ahead: stage
-  // kt+2 is issued into buffer kt & 1 as soon as every wave has its last
-  // fragments of stage kt in registers. Past the end of K the loads repeat the
-  // last stage (in bounds, never read), which keeps the loop free of branches.
-  const int64_t kt_n = K / kBK;
-  auto k_at = [&](int64_t kt) { return (kt < kt_n ? kt : kt_n - 1) * kBK; };
-  issue(0, 0);
-  issue(1, k_at(1));
-  wait_vmem();
+    for (int j = 0; j < kF; ++j) asm volatile("" : "+a"(acc.c[i][j]));
+  asm volatile("s_nop 7" ::: "memory");
+  if (kt_n > 1)
+    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  Frags f0, f1;
-  load_frags(lds, 0, f0);
-  for (int64_t kt = 0; kt + 1 < kt_n; ++kt) {
-    const char* st = lds + static_cast<int>(kt & 1) * kStage;
-    step(st, 1, f1, f0);
-    step(st, 2, f0, f1);
-    step(st, 3, f1, f0);
-    // Own loads of stage kt+1 done; the barrier then also covers every other
-    // wave's loads and every wave's LDS reads of stage kt.
-    wait_vmem();
-    __syncthreads();
-    // With kStagger, the two waves of a SIMD (w and w + 4) issue their loads
-    // one sub-step apart: while one wave is issuing its eight
-    // buffer_load ... lds, the other still has MFMAs to issue, so the SIMD's
-    // MFMA pipe does not drain after every barrier (measured: every product
-    // of the one-pass fused step about 2% faster, the c4 step 1.5% and c5
-    // 1.8%; delaying waves 1, 3, 5, 7 or 2, 3, 6, 7 instead, so that both
-    // waves of a SIMD still issue together, is about 1% slower than no delay).
-    // The later half of the loads then has one sub-step less to arrive, which
-    // costs the recomputing path's products (operand rows 32-256 KiB apart)
-    // 1.5-9% and its dZ kernel 0.7%: they are built without it.
-    if constexpr (kStagger) {
-      const bool late = (wave & 4) != 0;
-      if (!late) issue(static_cast<int>(kt & 1), k_at(kt + 2));
-      step(lds + static_cast<int>((kt + 1) & 1) * kStage, 0, f0, f1);
-      if (late) issue(static_cast<int>(kt & 1), k_at(kt + 2));
+
+  struct Set {
+    bf16x8_t a[kF], b[kF];
+  };
+  // Fragment q of a sub-step in the order the MFMAs first use them, b0 a0 b1
+  // a1 ...: part 1 completes it, part 0 reads a transposed one's first half.
+  s16x4_t half;
+  auto read = [&](const char* pa, const char* pb, int s, Set& f, int q, int part) {
+    if (q & 1) {
+      if constexpr (!kAMN) {
+        if (part == 1) f.a[q >> 1] = fa.read(pa, s, q >> 1);
+      } else if (part == 0) {
+        half = fa.read_half(pa, s, q >> 1, 0);
+      } else {
+        f.a[q >> 1] = fa.join(half, fa.read_half(pa, s, q >> 1, 1));
+      }
     } else {
-      issue(static_cast<int>(kt & 1), k_at(kt + 2));
-      step(lds + static_cast<int>((kt + 1) & 1) * kStage, 0, f0, f1);
+      if constexpr (!kBMN) {
+        if (part == 1) f.b[q >> 1] = fb.read(pb, s, q >> 1);
+      } else if (part == 0) {
+        half = fb.read_half(pb, s, q >> 1, 0);
+      } else {
+        f.b[q >> 1] = fb.join(half, fb.read_half(pb, s, q >> 1, 1));
+      }
     }
+  };
+  // One sub-step: the 64 MFMAs of `cur`, the 16 fragment reads of the next
+  // sub-step after every third of them (a transposed fragment's two halves
+  // after the second and the third), and kLoads loads, six MFMAs apart, after
+  // MFMAs that no read follows: an MFMA's 16 cycles hide about three other
+  // instructions.
+  constexpr int kLoadGap = 6;
+  auto step = [&](const char* pa, const char* pb, int s, Set& next, const Set& cur, auto loads,
+                  auto&& load) {
+    constexpr int kLoads = decltype(loads)::value;
+#pragma unroll
+    for (int x = 0; x < kF * kF; ++x) {
+      const int i = x / kF, j = (i & 1) ? kF - 1 - x % kF : x % kF;
+      mfma_16x16x32(acc.c[i][j], cur.a[i], cur.b[j]);
+      if (x % 3 != 0 && x / 3 < 2 * kF) read(pa, pb, s, next, x / 3, x % 3 - 1);
+      if (x % kLoadGap == 0 && x / kLoadGap < kLoads) load(x / kLoadGap);
+      if (kAMN || kBMN || x % 3 == 2) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using NoLoads = std::integral_constant<int, 0>;
+  using Loads = std::integral_constant<int, kBlocksPerWave>;
+  auto none = [](int) {};
+
+  Set f0, f1;
+#pragma unroll
+  for (int q = 0; q < 2 * kF; ++q) {
+    read(lds, lds_b, 0, f0, q, 0);
+    read(lds, lds_b, 0, f0, q, 1);
   }
-  {
-    const char* st = lds + static_cast<int>((kt_n - 1) & 1) * kStage;
-    step(st, 1, f1, f0);
-    step(st, 2, f0, f1);
-    step(st, 3, f1, f0);
-    mma(f1);
+  int a_cur = 0;               // byte offset of stage kt's A buffer
+  auto next_a = [](int o) { return o == (kBufsA - 1) * kStage ? 0 : o + kStage; };
+  auto prev_a = [](int o) { return o == 0 ? (kBufsA - 1) * kStage : o - kStage; };
+  // Stages [0, full) have all their k-rows: their loads run inside the
+  // sub-steps. The last one or two steps load with clamped rows, or nothing.
+  const int full_a = la.full_stages(kt_n), full_b = lb.full_stages(kt_n);
+  const int full = full_a < full_b ? full_a : full_b;
+  int kt = 0;
+  for (; kt + 2 < full; ++kt) {
+    const int a_nxt = next_a(a_cur);
+    const int b_cur = (kt & 1) * kStage;
+    char* da = lds + prev_a(a_cur) + lds_w;
+    la.at(kt + 2);
+    step(lds + a_cur, lds_b + b_cur, 1, f1, f0, Loads{}, [&](int l) { la.load(da, l); });
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    char* db = lds_b + b_cur + lds_w;
+    lb.at(kt + 2);
+    step(lds + a_nxt, lds_b + (kStage - b_cur), 0, f0, f1, Loads{},
+         [&](int l) { lb.load(db, l); });
+    a_cur = a_nxt;
   }
-  wait_vmem();
+  static_assert(kBlocksPerWave == 8, "the loop's wait leaves one stage's A loads in flight");
+  for (; kt + 1 < kt_n; ++kt) {
+    const int a_nxt = next_a(a_cur);
+    const int b_cur = (kt & 1) * kStage;
+    if (kt + 2 < kt_n) la.stage(lds + prev_a(a_cur) + lds_w, kt + 2);
+    step(lds + a_cur, lds_b + b_cur, 1, f1, f0, NoLoads{}, none);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + 2 < kt_n) lb.stage(lds_b + b_cur + lds_w, kt + 2);
+    step(lds + a_nxt, lds_b + (kStage - b_cur), 0, f0, f1, NoLoads{}, none);
+    a_cur = a_nxt;
+  }
+  step(lds + a_cur, lds_b + (kt & 1) * kStage, 1, f1, f0, NoLoads{}, none);
+#pragma unroll
+  for (int x = 0; x < kF * kF; ++x) mfma_16x16x32(acc.c[x / kF][x % kF], f1.a[x / kF], f1.b[x % kF]);
+  // The compiler does not know the MFMAs' latency: let the last ones finish
+  // before anything reads the accumulators.
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < kF; ++i)
+#pragma unroll
+    for (int j = 0; j < kF; ++j) asm volatile("" : "+a"(acc.c[i][j]));
 }
 
-// Row (within the wave's 128 rows) of accumulator fm, element e, for this lane:
-// the 32x32 result gives lane l column l%32 and rows 8*(e/4) + 4*(l/32) + e%4.
-__device__ __forceinline__ int acc_row(int fm, int e, int fhalf) {
-  return 32 * fm + 8 * (e >> 2) + 4 * fhalf + (e & 3);
-}
+// Row (within the wave's 128 rows) of accumulator row block i, element e, for
+// a lane in 16-lane group g: the 16x16 result gives lane l column l % 16 and
+// rows 4 (l / 16) + e.
+__device__ __forceinline__ int acc_row(int i, int e, int g) { return 16 * i + 4 * g + e; }
 
 // The epilogues stage a 256 x 256 bf16 tile in LDS as words of two rows: word
-// (vp, c) at vp * kBN + (c ^ 4 ((vp >> 2) & 15)) holds rows 2 vp and 2 vp + 1
-// of column c. Accumulator fm, element group q (elements 4q .. 4q + 3) of a
-// lane covers row pairs vp and vp + 1 with vp = wm * 64 + 16 fm + 4 q +
-// 2 fhalf, so vp >> 2 = 16 wm + 4 fm + q and the swizzle is a constant per
-// (fm, q): from the lane's base P + (wm * 64 + 2 fhalf) * kBN, the word of
-// column c is at a constant row offset and c XOR a constant.
-__device__ __forceinline__ uint32_t* stage_word(uint32_t* lane_base, int fm, int q, int c) {
-  return lane_base + (16 * fm + 4 * q) * kBN + (c ^ (((4 * fm + q) & 15) << 2));
+// (vp, c) at vp * kBN + (c ^ stage_swz(vp)) holds rows 2 vp and 2 vp + 1 of
+// column c. The swizzle keeps groups of 4 columns together (16-byte reads).
+// Its bits 4 and 5 take vp's bits 1 and 2, so that the four row groups of a
+// 16x16 block (lanes 16 g ..: vp = 8 i + 2 g) are written to the four 16-bank
+// groups; bits 2, 3 and (again) 4 take vp's bits 3, 4 and 5, so that one
+// column read at every fourth vp (lmhead_dz_kernel) spreads over 16 of the 64
+// banks, two rows to a bank.
+__device__ __forceinline__ int stage_swz(int vp) {
+  return ((((vp >> 1) ^ (vp >> 5)) & 1) << 4) | (((vp >> 2) & 1) << 5) | (((vp >> 3) & 3) << 2);
 }
+
+// Word of rows 16 i + 4 g + 2 h, + 1 (of wave row wm) and tile column c.
+__device__ __forceinline__ uint32_t* stage_word(uint32_t* P, int wm, int i, int g, int h, int c) {
+  // stage_swz(64 wm + 8 i + 2 g + h), the lane's part and the block's apart.
+  const int lane_swz = ((g & 1) << 4) | ((g >> 1) << 5);
+  const int block_swz = ((i & 3) << 2) | ((i >> 2) << 4);
+  return P + (wm * (kWaveM / 2) + 2 * g) * kBN + (8 * i + h) * kBN + ((c ^ lane_swz) ^ block_swz);
+}
+
+// Stage the wave's results as bf16.
+__device__ __forceinline__ void stage_bf16(const Acc& acc, uint32_t* P, int wm, int wn, int lane) {
+  const int g = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < kF; ++j) {
+    const int c = wn * kWaveN + 16 * j + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < kF; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *stage_word(P, wm, i, g, h, c) =
+            pack_bf16x2(acc.c[i][j][2 * h], acc.c[i][j][2 * h + 1]);
+  }
+}
+
+// 8 columns t0 .. t0 + 7 of staged rows 2 vp (lo) and 2 vp + 1 (hi), bf16.
+__device__ __forceinline__ void staged_rows(const uint32_t* P, int vp, int t0, u32x4& lo,
+                                            u32x4& hi) {
+  const int swz = stage_swz(vp);
+  const u32x4 a = *reinterpret_cast<const u32x4*>(P + vp * kBN + (t0 ^ swz));
+  const u32x4 b = *reinterpret_cast<const u32x4*>(P + vp * kBN + ((t0 + 4) ^ swz));
+  lo = u32x4{(a.x & 0xffffu) | (a.y << 16), (a.z & 0xffffu) | (a.w << 16),
+             (b.x & 0xffffu) | (b.y << 16), (b.z & 0xffffu) | (b.w << 16)};
+  hi = u32x4{(a.x >> 16) | (a.y & 0xffff0000u), (a.z >> 16) | (a.w & 0xffff0000u),
+             (b.x >> 16) | (b.y & 0xffff0000u), (b.z >> 16) | (b.w & 0xffff0000u)};
+}
+// The staged tile leaves 32 lanes to a pair of rows, 8 columns a lane.
+constexpr int kStagedIters = (kBM / 2) * (kBN / 8) / kThreads;
 
 // max(a, b, c) as one v_max3_f32 (two IEEE maxNum steps: a quiet NaN operand
 // is ignored). fmaxf gives the same value, but the compiler quiets every
@@ -475,22 +543,172 @@ __device__ __forceinline__ float bit_select(uint32_t mask, float a, float b) {
   return r;
 }
 
-// The element of accumulator fm, column fn, that holds wave row `row` in
-// this lane, when row lies in block fm and row bit 2 is the lane's half (the
-// caller selects among blocks and checks the half): e = 4 * (row bits 3-4) +
-// row bits 0-1. A select tree on the row's bits, 15 v_bfi_b32.
-__device__ __forceinline__ float acc_in_block(const Acc& acc, int fm, int fn, int row) {
-  const uint32_t m0 = 0u - (row & 1), m1 = 0u - ((row >> 1) & 1);
-  const uint32_t m3 = 0u - ((row >> 3) & 1), m4 = 0u - ((row >> 4) & 1);
-  float a[8];
+// Merge of a value over the four 16-lane groups of a wave (the lanes that hold
+// one column's rows), every lane getting the result: lanes 16-31 against 0-15
+// and 48-63 against 32-47, then the halves, by gfx950's row and half swaps.
+template <typename Op>
+__device__ __forceinline__ float merge_groups(float v, Op op) {
+  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+  const uint32_t w = __float_as_uint(v);
+  const auto r16 = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  const float x = op(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+  const uint32_t u = __float_as_uint(x);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return op(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+}
+__device__ __forceinline__ float max_op(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ float add_op(float a, float b) { return a + b; }
+
+// One column's statistics over the wave's 128 rows.
+struct ColumnStats {
+  float max, sum_m1, pick;
+};
+
+// The per-token statistics of kCols columns j0 .. of the wave's results
+// (Z^T: rows are vocabulary rows, columns tokens): maximum, sum exp(z - max)
+// - 1 and the target row's z (0 when tl[.] < 0, the target row within the
+// wave's rows otherwise), over the rows < valid_rows (kFull: all 128). The
+// terms of the sum that equal 1 (the maximum and its ties) are counted apart:
+// fract zeroes exactly those, so the maximum's 1 never enters a rounded sum
+// with the small terms. `keep(jj, i, p)` gets the four exponentials of row
+// block i of column j0 + jj (0 for rows past valid_rows).
+//
+// VALU work with the MFMA pipe idle, at every tile, so full tiles drop the
+// per-element row masks, take the maximum two values per v_max3_f32, and find
+// the target's element by a select tree on its row, only where a lane of the
+// wave has one (the wave's 128 rows of V hold few of its tokens' targets).
+// Both forms give the same bits. The columns go together so that their
+// merges' latencies overlap.
+template <int kCols, bool kFull, typename Keep>
+__device__ __forceinline__ void column_stats(const Acc& acc, int j0, int g, int valid_rows,
+                                             const int* tl, ColumnStats* out, Keep&& keep) {
+  float mx[kCols];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) a[i] = bit_select(m0, acc.c[fm][fn][2 * i + 1], acc.c[fm][fn][2 * i]);
-  float b[4];
+  for (int jj = 0; jj < kCols; ++jj) {
+    mx[jj] = kMaxFloorL;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) b[i] = bit_select(m1, a[2 * i + 1], a[2 * i]);
-  const float c0 = bit_select(m3, b[1], b[0]);
-  const float c1 = bit_select(m3, b[3], b[2]);
-  return bit_select(m4, c1, c0);
+    for (int i = 0; i < kF; ++i) {
+      const f32x4_t z = acc.c[i][j0 + jj];
+      if constexpr (kFull) {
+        mx[jj] = max3_hw(max3_hw(mx[jj], z[0], z[1]), z[2], z[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (acc_row(i, e, g) < valid_rows) mx[jj] = fmaxf(mx[jj], z[e]);
+      }
+    }
+  }
+#pragma unroll
+  for (int jj = 0; jj < kCols; ++jj) mx[jj] = merge_groups(mx[jj], max_op);
+#pragma unroll
+  for (int jj = 0; jj < kCols; ++jj) {
+    float pick = 0.0f;
+    if (__builtin_amdgcn_ballot_w64(tl[jj] >= 0)) {
+      // Element (i, e) of row 16 i + 4 g + e: a tree on the row's bits 0, 1,
+      // 4, 5 and 6, then the lane group that holds bits 2 and 3.
+      const int row = tl[jj];
+      const uint32_t m0 = 0u - (row & 1), m1 = 0u - ((row >> 1) & 1);
+      const uint32_t m4 = 0u - ((row >> 4) & 1), m5 = 0u - ((row >> 5) & 1);
+      const uint32_t m6 = 0u - ((row >> 6) & 1);
+      float b[kF];
+#pragma unroll
+      for (int i = 0; i < kF; ++i) {
+        const f32x4_t z = acc.c[i][j0 + jj];
+        b[i] = bit_select(m1, bit_select(m0, z[3], z[2]), bit_select(m0, z[1], z[0]));
+      }
+      const float c0 = bit_select(m4, b[1], b[0]), c1 = bit_select(m4, b[3], b[2]);
+      const float c2 = bit_select(m4, b[5], b[4]), c3 = bit_select(m4, b[7], b[6]);
+      const float z = bit_select(m6, bit_select(m5, c3, c2), bit_select(m5, c1, c0));
+      pick = merge_groups((row >= 0 && ((row >> 2) & 3) == g) ? z : 0.0f, add_op);
+    }
+    out[jj].pick = pick;
+  }
+  float se[kCols], sr[kCols];
+#pragma unroll
+  for (int jj = 0; jj < kCols; ++jj) {
+    se[jj] = sr[jj] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kF; ++i) {
+      const f32x4_t z = acc.c[i][j0 + jj];
+      float p[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        p[e] = (kFull || acc_row(i, e, g) < valid_rows) ? exp_shift(z[e], mx[jj]) : 0.0f;
+        se[jj] += p[e];
+        sr[jj] += __builtin_amdgcn_fractf(p[e]);
+      }
+      keep(jj, i, p);
+    }
+  }
+#pragma unroll
+  for (int jj = 0; jj < kCols; ++jj) {
+    const float e = merge_groups(se[jj], add_op), r = merge_groups(sr[jj], add_op);
+    const float ones = rintf(e - r);  // at least the maximum's own 1
+    out[jj].max = mx[jj];
+    out[jj].sum_m1 = (ones - 1.0f) + r;
+  }
+}
+
+// Columns whose statistics are formed together: two columns' 64 values and
+// their exponentials fit the registers beside the accumulators.
+constexpr int kStatCols = 2;
+
+// The partial statistics of the wave's 128 rows x 128 tokens, written for the
+// rows' 128-row block: pmax[blk * N + t], psum1[blk * N + t] and ptgt[blk * N +
+// t]. `keep(j, i, p)` as in column_stats, with the column block's index.
+template <typename Keep>
+__device__ __forceinline__ void wave_stats(const Acc& acc, int64_t vrow0, int64_t V, int64_t tok0,
+                                           int64_t N, const int64_t* __restrict__ target,
+                                           int64_t vstart, float* __restrict__ pmax,
+                                           float* __restrict__ psum1, float* __restrict__ ptgt,
+                                           int lane, Keep&& keep) {
+  const int g = lane >> 4;
+  const int64_t blk = vrow0 / kPartialRows;
+  const int64_t vr = V - vrow0;
+  // rows >= valid_rows of this wave's 128 are padding (possibly all of them)
+  const int valid_rows = static_cast<int>(vr < 0 ? 0 : (vr < kWaveM ? vr : kWaveM));
+  auto columns = [&](auto full_tag, int j0) {
+    constexpr bool kFull = decltype(full_tag)::value;
+    int tl[kStatCols];
+    ColumnStats st[kStatCols];
+#pragma unroll
+    for (int jj = 0; jj < kStatCols; ++jj) {
+      const int64_t tok = tok0 + 16 * (j0 + jj) + (lane & 15);
+      tl[jj] = -1;  // target row within this wave's valid rows, or -1
+      if (kFull || tok < N) {
+        // Rows past the shard's end pad the last block (they repeat its last
+        // row); a target there belongs to the next shard and picks nothing.
+        const int64_t t = target[tok] - vstart - vrow0;
+        tl[jj] = (t >= 0 && t < valid_rows) ? static_cast<int>(t) : -1;
+      }
+    }
+    column_stats<kStatCols, kFull>(acc, j0, g, valid_rows, tl, st, [&](int jj, int i, float* p) {
+      if (!kFull && tok0 + 16 * (j0 + jj) + (lane & 15) >= N) p[0] = p[1] = p[2] = p[3] = 0.0f;
+      keep(j0 + jj, i, p);
+    });
+#pragma unroll
+    for (int jj = 0; jj < kStatCols; ++jj) {
+      const int64_t tok = tok0 + 16 * (j0 + jj) + (lane & 15);
+      if (g == 0 && (kFull || tok < N) && valid_rows > 0) {
+        pmax[blk * N + tok] = st[jj].max;
+        psum1[blk * N + tok] = st[jj].sum_m1;
+        ptgt[blk * N + tok] = st[jj].pick;
+      }
+    }
+  };
+  if (valid_rows == kWaveM && tok0 + kWaveN <= N) {
+#pragma unroll
+    for (int j0 = 0; j0 < kF; j0 += kStatCols) {
+      columns(std::true_type{}, j0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+#pragma unroll
+    for (int j0 = 0; j0 < kF; j0 += kStatCols) {
+      columns(std::false_type{}, j0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -499,7 +717,7 @@ __device__ __forceinline__ float acc_in_block(const Acc& acc, int fm, int fn, in
 //   block's valid rows; ptgt[b*N + t] = z of the target row if it lies in the
 //   block, else 0. (cross_entropy.py:21, :28-36, :40-41 restricted to the block.)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void lmhead_stats_kernel(
+__global__ __launch_bounds__(kThreads, 1) void lmhead_stats_kernel(
     const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, int64_t V, int64_t N,
     int64_t H, const int64_t* __restrict__ target, int64_t vstart, float* __restrict__ pmax,
     float* __restrict__ psum1, float* __restrict__ ptgt) {
@@ -507,7 +725,7 @@ __global__ __launch_bounds__(kThreads) void lmhead_stats_kernel(
   const int tiles_m = static_cast<int>((V + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(kGroupMStats, tiles_m, tiles_n, tm, tn);
+  tile_coords(tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
   gemm_mainloop<false, false>(W, H, V, X, H, N, H, m0, n0, lds, acc);
@@ -515,58 +733,10 @@ __global__ __launch_bounds__(kThreads) void lmhead_stats_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int fhalf = lane >> 5;
   const int64_t vrow0 = m0 + wm * kWaveM;  // first vocabulary row of this wave
   if (vrow0 >= V) return;
-  const int64_t blk = vrow0 / kPartialRows;
-  // rows >= valid_rows of this wave's 128 are padding
-  const int valid_rows = static_cast<int>((V - vrow0) < kWaveM ? (V - vrow0) : kWaveM);
-#pragma unroll
-  for (int fn = 0; fn < kFN; ++fn) {
-    const int64_t tok = n0 + wn * kWaveN + 32 * fn + (lane & 31);
-    const bool tok_ok = tok < N;
-    int tl = -1;  // target row within this wave's valid rows, or -1
-    if (tok_ok) {
-      // Rows past the shard's end pad the last block (they repeat its last
-      // row); a target there belongs to the next shard and picks nothing here.
-      const int64_t t = target[tok] - vstart - vrow0;
-      tl = (t >= 0 && t < valid_rows) ? static_cast<int>(t) : -1;
-    }
-    float mx = kMaxFloorL;
-    float pick = 0.0f;
-#pragma unroll
-    for (int fm = 0; fm < kFM; ++fm)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = acc_row(fm, e, fhalf);
-        const float z = acc.c[fm][fn][e];
-        if (r < valid_rows) mx = fmaxf(mx, z);
-        pick = (r == tl) ? z : pick;
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // sum exp(z - mx) - 1 with the terms equal to 1 (the maximum and its
-    // ties) counted apart: fract zeroes exactly those, so the maximum's 1
-    // never enters a rounded sum with the small terms.
-    float se = 0.0f, sr = 0.0f;
-#pragma unroll
-    for (int fm = 0; fm < kFM; ++fm)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = acc_row(fm, e, fhalf);
-        const float p = r < valid_rows ? exp_shift(acc.c[fm][fn][e], mx) : 0.0f;
-        se += p;
-        sr += __builtin_amdgcn_fractf(p);
-      }
-    se += __shfl_xor(se, 32);
-    sr += __shfl_xor(sr, 32);
-    pick += __shfl_xor(pick, 32);
-    const float ones = rintf(se - sr);  // at least the maximum's own 1
-    if (fhalf == 0 && tok_ok) {
-      pmax[blk * N + tok] = mx;
-      psum1[blk * N + tok] = (ones - 1.0f) + sr;
-      ptgt[blk * N + tok] = pick;
-    }
-  }
+  wave_stats(acc, vrow0, V, n0 + wn * kWaveN, N, target, vstart, pmax, psum1, ptgt, lane,
+             [](int, int, const float*) {});
 }
 
 // Merge the partial statistics of nb vocabulary blocks into shard statistics:
@@ -636,7 +806,7 @@ __global__ __launch_bounds__(kRedTokens * kRedSlices) void lmhead_reduce_partial
 // of the two GEMMs that follow). The tile goes through LDS so that both
 // layouts leave as coalesced 16-byte stores.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
+__global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
     const uint16_t* __restrict__ Wc, const uint16_t* __restrict__ X, int64_t Mvalid,
     int64_t Mpad, int64_t N, int64_t H, const int64_t* __restrict__ target, int64_t vfirst,
     const float* __restrict__ gmax, const float* __restrict__ gsum1,
@@ -646,15 +816,15 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
   const int tiles_m = static_cast<int>(Mpad / kBM);
   const int tiles_n = static_cast<int>((ldt + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(kGroupM, tiles_m, tiles_n, tm, tn);
+  tile_coords(tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
-  gemm_mainloop<false, false, /*kStagger=*/false>(Wc, H, Mvalid, X, H, N, H, m0, n0, lds, acc);
+  gemm_mainloop<false, false>(Wc, H, Mvalid, X, H, N, H, m0, n0, lds, acc);
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int fhalf = lane >> 5;
+  const int g4 = lane >> 4;
   const int64_t vrow0 = m0 + wm * kWaveM;
   const int64_t vr = Mvalid - vrow0;
   const int valid_rows = static_cast<int>(vr < 0 ? 0 : (vr < kWaveM ? vr : kWaveM));
@@ -662,14 +832,9 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
   // fragments; the 256x256 bf16 tile of dZ (128 KiB) is staged there.
   __syncthreads();
   uint32_t* P = reinterpret_cast<uint32_t*>(lds);
-  // Word (vp, t) of the tile sits at P[vp * kBN + pcol(vp, t)]: the token
-  // index is XOR-swizzled in its bits 2..5 by the block of 4 vocabulary pairs,
-  // so a column read (32 lanes, one token, 32 blocks) spreads over the banks
-  // (at most 2-way), while 4 consecutive tokens stay one aligned 16-byte group.
-  auto pcol = [](int vp, int t) { return t ^ (((vp >> 2) & 15) << 2); };
 #pragma unroll
-  for (int fn = 0; fn < kFN; ++fn) {
-    const int tloc = wn * kWaveN + 32 * fn + (lane & 31);
+  for (int j = 0; j < kF; ++j) {
+    const int tloc = wn * kWaveN + 16 * j + (lane & 15);
     const int64_t tok = n0 + tloc;
     const bool tok_ok = tok < N;
     float M = 0.0f, scale = 0.0f, g = 0.0f, T1 = 0.0f;
@@ -688,29 +853,25 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
     // its softmax is at most 1/2 and the plain form loses nothing.
     float zt = 0.0f;
 #pragma unroll
-    for (int fm = 0; fm < kFM; ++fm)
+    for (int i = 0; i < kF; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) zt = (acc_row(fm, e, fhalf) == tl) ? acc.c[fm][fn][e] : zt;
+      for (int e = 0; e < 4; ++e) zt = (acc_row(i, e, g4) == tl) ? acc.c[i][j][e] : zt;
     const float dt = zt == M ? -T1 / (1.0f + T1) * g : (exp_shift(zt, M) / (1.0f + T1) - 1.0f) * g;
 #pragma unroll
-    for (int fm = 0; fm < kFM; ++fm) {
-      float d[16];
+    for (int i = 0; i < kF; ++i) {
+      float d[4];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = acc_row(fm, e, fhalf);
-        float p = exp_shift(acc.c[fm][fn][e], M) * scale;
+      for (int e = 0; e < 4; ++e) {
+        const int r = acc_row(i, e, g4);
+        float p = exp_shift(acc.c[i][j][e], M) * scale;
         p = (r == tl) ? dt : p;
         d[e] = (tok_ok && r < valid_rows) ? p : 0.0f;
       }
-      // Into the LDS tile as (even, odd) vocabulary-row pairs of one token:
-      // word P[v/2][t] = bf16(d[v]) | bf16(d[v+1]) << 16, tile-local v and t.
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t* w = stage_word(P + (wm * kWaveM / 2 + 2 * fhalf) * kBN, fm, q, tloc);
-        w[0] = pack_bf16x2(d[4 * q], d[4 * q + 1]);
-        w[kBN] = pack_bf16x2(d[4 * q + 2], d[4 * q + 3]);
-      }
+      // Into the LDS tile as (even, odd) vocabulary-row pairs of one token.
+      *stage_word(P, wm, i, g4, 0, tloc) = pack_bf16x2(d[0], d[1]);
+      *stage_word(P, wm, i, g4, 1, tloc) = pack_bf16x2(d[2], d[3]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
   // dz [N, ldz]: 32 lanes per token row, each 8 consecutive vocabulary rows
@@ -721,23 +882,21 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
     const int t = lin / (kBM / 8);
     const int L = lin % (kBM / 8);  // vocabulary rows 8L .. 8L+7, pairs 4L .. 4L+3
     const int64_t tok = n0 + t;
-    const uint32_t* col = P + 4 * L * kBN + pcol(4 * L, t);
-    const u32x4 w = {col[0], col[kBN], col[2 * kBN], col[3 * kBN]};
+    uint32_t c4[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c4[u] = P[(4 * L + u) * kBN + (t ^ stage_swz(4 * L + u))];
+    const u32x4 w = {c4[0], c4[1], c4[2], c4[3]};
     if (tok < N) *reinterpret_cast<u32x4*>(dz + tok * ldz + m0 + 8 * L) = w;
   }
   // dz^T [Vc, ldt]: 32 lanes cover one pair of vocabulary rows (256 tokens);
   // each reads 8 words (8 tokens of both rows) and writes 16 bytes to each row.
 #pragma unroll 2
-  for (int it = 0; it < (kBM / 2) * (kBN / 8) / kThreads; ++it) {
+  for (int it = 0; it < kStagedIters; ++it) {
     const int lin = it * kThreads + static_cast<int>(threadIdx.x);
     const int vp = lin / (kBN / 8);
     const int t0 = 8 * (lin % (kBN / 8));
-    const u32x4 a = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, t0));
-    const u32x4 b = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, t0 + 4));
-    const u32x4 lo = {(a.x & 0xffffu) | (a.y << 16), (a.z & 0xffffu) | (a.w << 16),
-                      (b.x & 0xffffu) | (b.y << 16), (b.z & 0xffffu) | (b.w << 16)};
-    const u32x4 hi = {(a.x >> 16) | (a.y & 0xffff0000u), (a.z >> 16) | (a.w & 0xffff0000u),
-                      (b.x >> 16) | (b.y & 0xffff0000u), (b.z >> 16) | (b.w & 0xffff0000u)};
+    u32x4 lo, hi;
+    staged_rows(P, vp, t0, lo, hi);
     const int64_t tok0 = n0 + t0;
     if (tok0 < ldt) {
       *reinterpret_cast<u32x4*>(dzt + (m0 + 2 * vp) * ldt + tok0) = lo;
@@ -747,15 +906,15 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
 }
 
 // The fp32 epilogues (modes 1-3 of gemm_store_kernel). The 256x256 fp32 tile
-// goes through the freed LDS in two passes of 128 rows: pass q takes
-// accumulators fm = 2q, 2q + 1 of every wave, i.e. tile rows 64 q .. 64 q + 63
+// goes through the freed LDS in two passes of 128 rows: pass q takes row
+// blocks i = 4q .. 4q + 3 of every wave, i.e. tile rows 64 q .. 64 q + 63
 // and 128 + 64 q .. 128 + 64 q + 63, so each pass reads its own half of the
 // accumulator registers. Staged row r (1 KiB) is tile row
-// 128 (r >> 6) + 64 q + (r & 63); its 16-byte chunk c sits at c ^ 8 ((r >> 2)
-// & 1), which puts the two rows one ds_write_b32 covers (r and r + 4) on
-// opposite halves of the banks. Every thread then moves 16 chunks: staged row
-// 8 p + wave, chunk lane, so a wave's access is one 1 KiB row segment of Cf
-// (or 512 bytes of C).
+// 128 (r >> 6) + 64 q + (r & 63); its 16-byte chunk c sits at c ^ 4 ((r >> 2)
+// & 3), which puts the four rows one ds_write_b32 covers (r, r + 4, r + 8,
+// r + 12) on the four 16-bank groups. Every thread then moves 32 chunks:
+// staged row 4 p + wave, chunk lane, so a wave's access is one 1 KiB row
+// segment of Cf (or 512 bytes of C).
 // kVec (N % 4 == 0, ldc % 4 == 0, Cf 16-byte and C 8-byte aligned, 512 rows
 // within 32-bit offsets): buffer resources on the wave's first row, the
 // lane's column in the one offset register and the row step in the scalar
@@ -765,9 +924,9 @@ __global__ __launch_bounds__(kThreads) void lmhead_dz_kernel(
 // a lane whose columns lie past N gets the resource's size as its offset: its
 // accesses are out of range (no memory access, a load reads 0, a store is
 // dropped) whether or not the row step takes part in the check. Every access
-// left is inside the matrix. In modes 2 and 3 half of the 16 loads of Cf
+// left is inside the matrix. In modes 2 and 3 half of the 32 loads of Cf
 // are issued before the pass is staged, so their latency runs under the
-// staging, and the other half right after it. Cf is streamed (non-temporal)
+// staging, and each of the others as an earlier row leaves. Cf is streamed (non-temporal)
 // both ways. Without kVec the pass leaves element by element.
 //   kMode 1: Cf = acc;  kMode 2: Cf += acc;  kMode 3: C = bf16(Cf + acc)
 template <int kMode, bool kVec>
@@ -775,22 +934,22 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
                                                uint16_t* __restrict__ C, int64_t ldc, int64_t M,
                                                int64_t N, int64_t m0, int64_t n0) {
   static_assert(kMode >= 1 && kMode <= 3, "fp32 epilogue modes");
-  static_assert(kBN == 256 && kWavesM == 2 && kFM == 4 && 128 * kBN * 4 <= kLdsBytes,
+  static_assert(kBN == 256 && kWavesM == 2 && kF == 8 && 128 * kBN * 4 <= kLdsBytes,
                 "two passes of 128 rows fit the stages");
-  constexpr int kRowsPerPass = kThreads / 64;  // 8
-  constexpr int kPasses = 128 / kRowsPerPass;  // 16
+  constexpr int kRowsPerPass = kThreads / 64;  // 4
+  constexpr int kPasses = 128 / kRowsPerPass;  // 32
   constexpr int kNt = 2;                       // cache policy: non-temporal
-  // Loads of Cf issued before a pass is staged (the staging needs registers
-  // for the accumulators it moves); the rest follow right after it.
-  constexpr int kEarly = 8;
+  // Loads of Cf in flight (the staging needs registers for the accumulators
+  // it moves).
+  constexpr int kEarly = 16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int fhalf = lane >> 5;
+  const int g = lane >> 4;
   float* S = reinterpret_cast<float*>(lds);
   const bool col_ok = n0 + 4 * lane < N;
-  // Tile rows of staged rows 8 p + wave, relative to the pass's first row.
-  auto row_off = [](int p) { return 8 * p + 64 * (p >> 3); };
+  // Tile rows of staged rows 4 p + wave, relative to the pass's first row.
+  auto row_off = [](int p) { return 4 * p + 64 * (p >> 4); };
   __syncthreads();  // every wave is done with the operand buffers
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
@@ -804,7 +963,7 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
     const uint32_t vf = col_ok ? static_cast<uint32_t>(lane) * 16u
                                : static_cast<uint32_t>(lim * ldc * 4);
     float* cf_base = Cf + (np > 0 ? row0 : 0) * ldc + n0;
-    u32x4 old[kPasses];
+    u32x4 old[kEarly];  // row p's values of Cf in old[p % kEarly], kEarly rows ahead
     __amdgpu_buffer_rsrc_t rf;
     if constexpr (kVec) {
       rf = __builtin_amdgcn_make_buffer_rsrc(cf_base, 0, static_cast<int>(lim * ldc * 4),
@@ -819,30 +978,21 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
       }
     }
 #pragma unroll
-    for (int fn = 0; fn < kFN; ++fn) {
-      const int c = wn * kWaveN + 32 * fn + (lane & 31);
+    for (int j = 0; j < kF; ++j) {
+      const int c = wn * kWaveN + 16 * j + (lane & 15);
 #pragma unroll
-      for (int f = 0; f < 2; ++f)
+      for (int f = 0; f < 4; ++f)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int r = wm * 64 + 32 * f + 8 * (e >> 2) + 4 * fhalf + (e & 3);
-          S[r * kBN + ((((c >> 2) ^ (fhalf << 3)) << 2) | (c & 3))] = acc.c[2 * q + f][fn][e];
+        for (int e = 0; e < 4; ++e) {
+          const int r = wm * 64 + 16 * f + 4 * g + e;
+          S[r * kBN + (c ^ (g << 4))] = acc.c[4 * q + f][j][e];
         }
     }
     __syncthreads();
-    if constexpr (kVec && kMode >= 2) {
-#pragma unroll
-      for (int p = kEarly; p < kPasses; ++p) {
-        if (p < np)
-          old[p] = __builtin_amdgcn_raw_buffer_load_b128(
-              rf, vf, static_cast<uint32_t>(row_off(p) * ldc * 4), kNt);
-      }
-    }
-    const int sw = ((wave >> 2) & 1) << 3;  // chunk swizzle of staged rows 8 p + wave
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
       const int r = p * kRowsPerPass + wave;
-      const u32x4 sv = *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ sw) << 2));
+      const u32x4 sv = *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ ((p & 3) << 2)) << 2));
       if constexpr (!kVec) {
         const int64_t row = row0 + row_off(p);
         const float sf[4] = {__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z),
@@ -861,7 +1011,10 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
         if constexpr (kMode == 1) {
           buffer_store_b128<kNt>(sv, rf, vf + so);
         } else {
-          const u32x4 o = old[p];
+          const u32x4 o = old[p % kEarly];
+          if (p + kEarly < np)
+            old[p % kEarly] = __builtin_amdgcn_raw_buffer_load_b128(
+                rf, vf, static_cast<uint32_t>(row_off(p + kEarly) * ldc * 4), kNt);
           const float v0 = __uint_as_float(sv.x) + __uint_as_float(o.x);
           const float v1 = __uint_as_float(sv.y) + __uint_as_float(o.y);
           const float v2 = __uint_as_float(sv.z) + __uint_as_float(o.z);
@@ -888,44 +1041,40 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
 }
 
 // bf16 out through the freed LDS, as lmhead_p_kernel stages P^T: words of two
-// rows (vp = row / 2) per column, columns XOR-swizzled by the row pair, then
-// 16-byte stores of 512-byte row segments. Tiles that reach past N, and
-// outputs that are not 16-byte aligned, store element by element.
+// rows (vp = row / 2) per column, then 16-byte stores of 512-byte row
+// segments. Tiles that reach past N, and outputs that are not 16-byte
+// aligned, store element by element.
 __device__ __forceinline__ void store_bf16_tile(const Acc& acc, char* lds,
                                                 uint16_t* __restrict__ C, int64_t ldc, int64_t M,
                                                 int64_t N, int64_t m0, int64_t n0) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int fhalf = lane >> 5;
   const bool vec_ok = (ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   __syncthreads();  // every wave is done with the operand buffers
   uint32_t* P = reinterpret_cast<uint32_t*>(lds);
-  auto pcol = [](int vp, int t) { return t ^ (((vp >> 2) & 15) << 2); };
-#pragma unroll
-  for (int fn = 0; fn < kFN; ++fn) {
-    const int cloc = wn * kWaveN + 32 * fn + (lane & 31);
-#pragma unroll
-    for (int fm = 0; fm < kFM; ++fm)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t* w = stage_word(P + (wm * kWaveM / 2 + 2 * fhalf) * kBN, fm, q, cloc);
-        w[0] = pack_bf16x2(acc.c[fm][fn][4 * q], acc.c[fm][fn][4 * q + 1]);
-        w[kBN] = pack_bf16x2(acc.c[fm][fn][4 * q + 2], acc.c[fm][fn][4 * q + 3]);
-      }
-  }
+  stage_bf16(acc, P, wm, wn, lane);
   __syncthreads();
+  const int vp0 = static_cast<int>(threadIdx.x) / (kBN / 8);
+  const int c0 = 8 * (static_cast<int>(threadIdx.x) % (kBN / 8));
+  constexpr int kVpStep = kThreads / (kBN / 8);
+  if (vec_ok && m0 + kBM <= M && n0 + kBN <= N) {  // every store in bounds: no tests
+    uint16_t* dst = C + (m0 + 2 * vp0) * ldc + n0 + c0;
+#pragma unroll 4
+    for (int it = 0; it < kStagedIters; ++it) {
+      u32x4 lo, hi;
+      staged_rows(P, vp0 + it * kVpStep, c0, lo, hi);
+      *reinterpret_cast<u32x4*>(dst) = lo;
+      *reinterpret_cast<u32x4*>(dst + ldc) = hi;
+      dst += 2 * kVpStep * ldc;
+    }
+    return;
+  }
 #pragma unroll 2
-  for (int it = 0; it < (kBM / 2) * (kBN / 8) / kThreads; ++it) {
-    const int lin = it * kThreads + static_cast<int>(threadIdx.x);
-    const int vp = lin / (kBN / 8);
-    const int c0 = 8 * (lin % (kBN / 8));
-    const u32x4 a = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, c0));
-    const u32x4 b = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, c0 + 4));
-    const u32x4 lo = {(a.x & 0xffffu) | (a.y << 16), (a.z & 0xffffu) | (a.w << 16),
-                      (b.x & 0xffffu) | (b.y << 16), (b.z & 0xffffu) | (b.w << 16)};
-    const u32x4 hi = {(a.x >> 16) | (a.y & 0xffff0000u), (a.z >> 16) | (a.w & 0xffff0000u),
-                      (b.x >> 16) | (b.y & 0xffff0000u), (b.z >> 16) | (b.w & 0xffff0000u)};
+  for (int it = 0; it < kStagedIters; ++it) {
+    const int vp = vp0 + it * kVpStep;
+    u32x4 lo, hi;
+    staged_rows(P, vp, c0, lo, hi);
     const int64_t col0 = n0 + c0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -958,18 +1107,17 @@ __device__ __forceinline__ void store_bf16_tile(const Acc& acc, char* lds,
 // accesses (the host checks them); otherwise the half tiles leave element by
 // element.
 // ---------------------------------------------------------------------------
-template <int kMode, bool kAMN = false, bool kBMN = false, bool kVec = true,
-          bool kStagger = true>
-__global__ __launch_bounds__(kThreads) void gemm_store_kernel(
+template <int kMode, bool kAMN = false, bool kBMN = false, bool kVec = true>
+__global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
     const uint16_t* __restrict__ A, int64_t lda, int64_t M, const uint16_t* __restrict__ B,
     int64_t ldb, int64_t N, int64_t K, uint16_t* __restrict__ C, float* __restrict__ Cf,
-    int64_t ldc, int group_m, int64_t ka_rows, int64_t kb_rows, int splits, int64_t ks,
+    int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits, int64_t ks,
     int64_t split_stride) {
   extern __shared__ __align__(16) char lds[];
   const int tiles_m = static_cast<int>((M + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tmv, tn;
-  tile_coords(group_m, tiles_m * splits, tiles_n, tmv, tn);
+  tile_coords(tiles_m * splits, tiles_n, tmv, tn);
   const int split = tmv / tiles_m;
   const int tm = tmv - split * tiles_m;
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
@@ -981,8 +1129,8 @@ __global__ __launch_bounds__(kThreads) void gemm_store_kernel(
   const uint16_t* Bs = kBMN ? B + k0 * ldb : B + k0;
   Cf += split * split_stride;
   Acc acc;
-  gemm_mainloop<kAMN, kBMN, kStagger>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
-                                      ka_rows - k0, kb_rows - k0);
+  gemm_mainloop<kAMN, kBMN>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc, ka_rows - k0,
+                            kb_rows - k0);
   if constexpr (kMode != 0)
     store_f32_tile<kMode, kVec>(acc, lds, Cf, C, ldc, M, N, m0, n0);
   else
@@ -999,7 +1147,7 @@ __global__ __launch_bounds__(kThreads) void gemm_store_kernel(
 // the logits never need to be recomputed. pt leaves through LDS as 512-byte
 // row segments, as in lmhead_dz_kernel.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void lmhead_p_kernel(
+__global__ __launch_bounds__(kThreads, 1) void lmhead_p_kernel(
     const uint16_t* __restrict__ W, const uint16_t* __restrict__ X, int64_t V, int64_t N,
     int64_t H, const int64_t* __restrict__ target, int64_t vstart, float* __restrict__ pmax,
     float* __restrict__ psum1, float* __restrict__ ptgt, uint16_t* __restrict__ pt,
@@ -1008,7 +1156,7 @@ __global__ __launch_bounds__(kThreads) void lmhead_p_kernel(
   const int tiles_m = static_cast<int>((V + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(kGroupMStats, tiles_m, tiles_n, tm, tn);
+  tile_coords(tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
   gemm_mainloop<false, false>(W, H, V, X, H, N, H, m0, n0, lds, acc);
@@ -1016,128 +1164,27 @@ __global__ __launch_bounds__(kThreads) void lmhead_p_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
-  const int fhalf = lane >> 5;
-  const int64_t vrow0 = m0 + wm * kWaveM;  // first vocabulary row of this wave
-  const int64_t blk = vrow0 / kPartialRows;
-  const int64_t vr = V - vrow0;
-  // rows >= valid_rows of this wave's 128 are padding (possibly all of them)
-  const int valid_rows = static_cast<int>(vr < 0 ? 0 : (vr < kWaveM ? vr : kWaveM));
+  const int g = lane >> 4;
   __syncthreads();  // every wave is done with the operand buffers
   uint32_t* P = reinterpret_cast<uint32_t*>(lds);
-  auto pcol = [](int vp, int t) { return t ^ (((vp >> 2) & 15) << 2); };
-  // One token column (fn) of the wave's 128 rows. This is VALU work with the
-  // MFMA pipe idle, at every tile, so full tiles (all 128 rows of the wave
-  // valid, every token < N: all but the last tile row and column) drop the
-  // per-element row and token masks, take the maximum two values per
-  // v_max3_f32 and find the target's element by a select tree on its row
-  // rather than a compare per element. Both forms give the same bits.
-  auto column = [&](auto full_tag, int fn) {
-    constexpr bool kFull = decltype(full_tag)::value;
-    const int tloc = wn * kWaveN + 32 * fn + (lane & 31);
-    const int64_t tok = n0 + tloc;
-    const bool tok_ok = kFull || tok < N;
-    int tl = -1;  // target row within this wave's valid rows, or -1
-    if (tok_ok) {
-      const int64_t t = target[tok] - vstart - vrow0;
-      tl = (t >= 0 && t < valid_rows) ? static_cast<int>(t) : -1;
-    }
-    float mx = kMaxFloorL;
-    float pick = 0.0f;
-    if constexpr (kFull) {
-      float m4[kFM];
-#pragma unroll
-      for (int fm = 0; fm < kFM; ++fm) {
-        m4[fm] = kMaxFloorL;
-#pragma unroll
-        for (int e = 0; e < 16; e += 2)
-          m4[fm] = max3_hw(m4[fm], acc.c[fm][fn][e], acc.c[fm][fn][e + 1]);
-      }
-      mx = max3_hw(m4[0], m4[1], max3_hw(m4[2], m4[3], kMaxFloorL));
-      // A wave's 64 tokens of this column have a target among its 128 rows
-      // only about once in 16 (128 of V rows): skip the tree otherwise.
-      if (__builtin_amdgcn_ballot_w64(tl >= 0)) {
-        float z4[kFM];
-#pragma unroll
-        for (int fm = 0; fm < kFM; ++fm) z4[fm] = acc_in_block(acc, fm, fn, tl);
-        const float za = (tl & 32) ? z4[1] : z4[0];
-        const float zb = (tl & 32) ? z4[3] : z4[2];
-        const float z = (tl & 64) ? zb : za;
-        pick = (tl >= 0 && ((tl >> 2) & 1) == fhalf) ? z : 0.0f;
-      }
-    } else {
-#pragma unroll
-      for (int fm = 0; fm < kFM; ++fm)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int r = acc_row(fm, e, fhalf);
-          const float z = acc.c[fm][fn][e];
-          if (r < valid_rows) mx = fmaxf(mx, z);
-          pick = (r == tl) ? z : pick;
-        }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // sum exp(z - mx) - 1 with the terms equal to 1 counted apart (as in
-    // lmhead_stats_kernel); each exponential also goes to the LDS tile.
-    float se = 0.0f, sr = 0.0f;
-#pragma unroll
-    for (int fm = 0; fm < kFM; ++fm) {
-      float d[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = acc_row(fm, e, fhalf);
-        const float p = (kFull || r < valid_rows) ? exp_shift(acc.c[fm][fn][e], mx) : 0.0f;
-        se += p;
-        sr += __builtin_amdgcn_fractf(p);
-        d[e] = tok_ok ? p : 0.0f;
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t* w = stage_word(P + (wm * kWaveM / 2 + 2 * fhalf) * kBN, fm, q, tloc);
-        w[0] = pack_bf16x2(d[4 * q], d[4 * q + 1]);
-        w[kBN] = pack_bf16x2(d[4 * q + 2], d[4 * q + 3]);
-      }
-    }
-    se += __shfl_xor(se, 32);
-    sr += __shfl_xor(sr, 32);
-    pick += __shfl_xor(pick, 32);
-    const float ones = rintf(se - sr);
-    if (fhalf == 0 && tok_ok && valid_rows > 0) {
-      pmax[blk * N + tok] = mx;
-      psum1[blk * N + tok] = (ones - 1.0f) + sr;
-      ptgt[blk * N + tok] = pick;
-    }
-  };
-  // One column at a time: both at once would need every accumulator in
-  // VGPRs together and spill.
-  if (valid_rows == kWaveM && n0 + kBN <= N) {
-#pragma unroll
-    for (int fn = 0; fn < kFN; ++fn) {
-      column(std::true_type{}, fn);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
-#pragma unroll
-    for (int fn = 0; fn < kFN; ++fn) {
-      column(std::false_type{}, fn);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
+  wave_stats(acc, m0 + wm * kWaveM, V, n0 + wn * kWaveN, N, target, vstart, pmax, psum1, ptgt,
+             lane, [&](int j, int i, const float* p) {
+               const int c = wn * kWaveN + 16 * j + (lane & 15);
+               *stage_word(P, wm, i, g, 0, c) = pack_bf16x2(p[0], p[1]);
+               *stage_word(P, wm, i, g, 1, c) = pack_bf16x2(p[2], p[3]);
+             });
   __syncthreads();
   // pt [Mpad, ldt]: 32 lanes cover one pair of vocabulary rows (256 tokens).
   // Non-temporal stores: pt (N V bf16, gigabytes) is read back only by the
   // rescale kernel, so it should not take L2 lines from the operand stripes
   // the next tiles of this XCD read (measured: the kernel 2% faster).
 #pragma unroll 2
-  for (int it = 0; it < (kBM / 2) * (kBN / 8) / kThreads; ++it) {
+  for (int it = 0; it < kStagedIters; ++it) {
     const int lin = it * kThreads + static_cast<int>(threadIdx.x);
     const int vp = lin / (kBN / 8);
     const int t0 = 8 * (lin % (kBN / 8));
-    const u32x4 a = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, t0));
-    const u32x4 b = *reinterpret_cast<const u32x4*>(P + vp * kBN + pcol(vp, t0 + 4));
-    const u32x4 lo = {(a.x & 0xffffu) | (a.y << 16), (a.z & 0xffffu) | (a.w << 16),
-                      (b.x & 0xffffu) | (b.y << 16), (b.z & 0xffffu) | (b.w << 16)};
-    const u32x4 hi = {(a.x >> 16) | (a.y & 0xffff0000u), (a.z >> 16) | (a.w & 0xffff0000u),
-                      (b.x >> 16) | (b.y & 0xffff0000u), (b.z >> 16) | (b.w & 0xffff0000u)};
+    u32x4 lo, hi;
+    staged_rows(P, vp, t0, lo, hi);
     const int64_t tok0 = n0 + t0;
     if (tok0 < ldt) {
       store_stream(reinterpret_cast<u32x4*>(pt + (m0 + 2 * vp) * ldt + tok0), lo);
@@ -1344,24 +1391,24 @@ inline bool operand_ok(const void* p, int64_t ld) {
 }
 
 // The product kernels by output mode and operand layout: K-contiguous A, and
-// B K-contiguous (b_mn = false) or MN-contiguous with kb_rows k-rows (b_mn;
-// then A may be MN-contiguous too, a_mn, in modes 0 and 1 only).
-template <int kMode, bool kAMN, bool kBMN, bool kVec, bool kStagger = true>
+// B K-contiguous (b_mn = false) or MN-contiguous with kb_rows k-rows (b_mn,
+// in mode 0; with A MN-contiguous too, a_mn, in modes 0 and 1).
+template <int kMode, bool kAMN, bool kBMN, bool kVec>
 int launch_store(dim3 grid, hipStream_t stream, const uint16_t* A, int64_t lda, int64_t M,
                  const uint16_t* B, int64_t ldb, int64_t N, int64_t K, uint16_t* C, float* Cf,
-                 int64_t ldc, int group_m, int64_t ka_rows, int64_t kb_rows, int splits,
+                 int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits,
                  int64_t ks, int64_t split_stride) {
   static bool lds_set = false;  // the attribute is set once per process and kernel
   if (!lds_set) {
     const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&gemm_store_kernel<kMode, kAMN, kBMN, kVec, kStagger>),
+        reinterpret_cast<const void*>(&gemm_store_kernel<kMode, kAMN, kBMN, kVec>),
         hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess) return static_cast<int>(e);
     lds_set = true;
   }
-  hipLaunchKernelGGL((gemm_store_kernel<kMode, kAMN, kBMN, kVec, kStagger>), grid, dim3(kThreads),
-                     kLdsBytes, stream, A, lda, M, B, ldb, N, K, C, Cf, ldc, group_m, ka_rows,
-                     kb_rows, splits, ks, split_stride);
+  hipLaunchKernelGGL((gemm_store_kernel<kMode, kAMN, kBMN, kVec>), grid, dim3(kThreads),
+                     kLdsBytes, stream, A, lda, M, B, ldb, N, K, C, Cf, ldc, ka_rows, kb_rows,
+                     splits, ks, split_stride);
   return NMCE_OK;
 }
 
@@ -1369,80 +1416,46 @@ int launch_store(dim3 grid, hipStream_t stream, const uint16_t* A, int64_t lda, 
 // the last one may be shorter), partial products at Cf + s * split_stride.
 int launch_gemm_store(int mode, const uint16_t* A, int64_t lda, int64_t M, const uint16_t* B,
                       int64_t ldb, int64_t N, int64_t K, uint16_t* C, float* Cf, int64_t ldc,
-                      hipStream_t stream, int group_m = kGroupM, bool a_mn = false,
+                      hipStream_t stream, bool a_mn = false,
                       bool b_mn = false, int64_t ka_rows = 0, int64_t kb_rows = 0,
-                      int splits = 1, int64_t ks = 0, int64_t split_stride = 0,
-                      bool stagger = true) {
+                      int splits = 1, int64_t ks = 0, int64_t split_stride = 0) {
   if (splits < 1 || (splits > 1 && (mode != 1 || ks <= 0 || ks % kBK != 0 ||
                                     (splits - 1) * ks >= K)))
     return NMCE_EINVAL_SHAPE;
   if (splits == 1) ks = K;
   const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN) * splits;
   const dim3 grid(static_cast<unsigned>(tiles));
-  if (a_mn && (!b_mn || mode > 1)) return NMCE_EINVAL_SHAPE;
+  if ((a_mn && (!b_mn || mode > 1)) || (b_mn && !a_mn && mode > 0)) return NMCE_EINVAL_SHAPE;
   // The fp32 epilogues' 16-byte form: whole 16-byte chunks, aligned outputs,
-  // and every offset (a pass's 185 rows, plus as much again for a lane past
+  // and every offset (a pass's 189 rows, plus as much again for a lane past
   // N) within 32 bits.
   const bool vec = (N & 3) == 0 && (ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(Cf) & 15) == 0 &&
                    (mode != 3 || (reinterpret_cast<uintptr_t>(C) & 7) == 0) &&
                    ldc * 4 * 512 < (int64_t{1} << 32);
   int st = NMCE_OK;
-#define NMCE_STORE(MODE, AMN, BMN)                                                           \
-  st = vec ? launch_store<MODE, AMN, BMN, true>(grid, stream, A, lda, M, B, ldb, N, K, C, Cf, \
-                                                ldc, group_m, ka_rows, kb_rows, splits, ks,   \
-                                                split_stride)                                 \
-           : launch_store<MODE, AMN, BMN, false>(grid, stream, A, lda, M, B, ldb, N, K, C, Cf, \
-                                                 ldc, group_m, ka_rows, kb_rows, splits, ks,  \
-                                                 split_stride)
-  // Both operands K-contiguous, loads issued together (stagger = false).
-#define NMCE_STORE_FLAT(MODE)                                                                   \
-  st = vec ? launch_store<MODE, false, false, true, false>(grid, stream, A, lda, M, B, ldb, N, K, \
-                                                           C, Cf, ldc, group_m, ka_rows, kb_rows, \
-                                                           splits, ks, split_stride)              \
-           : launch_store<MODE, false, false, false, false>(grid, stream, A, lda, M, B, ldb, N,   \
-                                                            K, C, Cf, ldc, group_m, ka_rows,      \
-                                                            kb_rows, splits, ks, split_stride)
-  if (!stagger && (a_mn || b_mn)) return NMCE_EINVAL_SHAPE;  // built for K-contiguous only
+  // (mode 0 has one form: its epilogue tests its own alignment)
+#define NMCE_STORE(MODE, AMN, BMN)                                                                \
+  st = vec ? launch_store<MODE, AMN, BMN, true>(grid, stream, A, lda, M, B, ldb, N, K, C, Cf,      \
+                                                ldc, ka_rows, kb_rows, splits, ks, split_stride)   \
+           : launch_store<MODE, AMN, BMN, MODE == 0>(grid, stream, A, lda, M, B, ldb, N, K, C, Cf, \
+                                                     ldc, ka_rows, kb_rows, splits, ks,            \
+                                                     split_stride)
   if (a_mn) {
     if (mode == 0) NMCE_STORE(0, true, true);
     else NMCE_STORE(1, true, true);
   } else if (b_mn) {
-    switch (mode) {
-      case 0: NMCE_STORE(0, false, true); break;
-      case 1: NMCE_STORE(1, false, true); break;
-      case 2: NMCE_STORE(2, false, true); break;
-      default: NMCE_STORE(3, false, true); break;
-    }
-  } else if (stagger) {
+    NMCE_STORE(0, false, true);
+  } else {
     switch (mode) {
       case 0: NMCE_STORE(0, false, false); break;
       case 1: NMCE_STORE(1, false, false); break;
       case 2: NMCE_STORE(2, false, false); break;
       default: NMCE_STORE(3, false, false); break;
     }
-  } else {
-    switch (mode) {
-      case 0: NMCE_STORE_FLAT(0); break;
-      case 1: NMCE_STORE_FLAT(1); break;
-      case 2: NMCE_STORE_FLAT(2); break;
-      default: NMCE_STORE_FLAT(3); break;
-    }
   }
-#undef NMCE_STORE_FLAT
 #undef NMCE_STORE
   if (st) return st;
   return launch_status();
-}
-
-// A product with both operands K-contiguous whose stage loads are issued by
-// all waves together (gemm_mainloop's kStagger off): the recomputing path's
-// products, whose operand rows lie far apart.
-int launch_gemm_store_unstaggered(int mode, const uint16_t* A, int64_t lda, int64_t M,
-                                  const uint16_t* B, int64_t ldb, int64_t N, int64_t K,
-                                  uint16_t* C, float* Cf, int64_t ldc, hipStream_t stream) {
-  return launch_gemm_store(mode, A, lda, M, B, ldb, N, K, C, Cf, ldc, stream, kGroupM,
-                           /*a_mn=*/false, /*b_mn=*/false, 0, 0, /*splits=*/1, 0, 0,
-                           /*stagger=*/false);
 }
 
 int launch_transpose(const uint16_t* in, int64_t R, int64_t C, int64_t ldi, uint16_t* out,
@@ -1853,8 +1866,8 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
                      grad_output, gout_stride, c, L, ws, s)))
       return st;
     // dW rows [v0, v0 + mvalid) = dZ^T_c X  (K = tokens, padded with zeros).
-    if ((st = launch_gemm_store_unstaggered(0, dzt, L.ldt, mvalid, xt, L.ldt, H, L.ldt,
-                                            dW + v0 * H, nullptr, H, s)))
+    if ((st = launch_gemm_store(0, dzt, L.ldt, mvalid, xt, L.ldt, H, L.ldt, dW + v0 * H, nullptr, H,
+                                s)))
       return st;
     // dX (+)= dZ_c W_c  (K = the chunk's padded vocabulary rows).
     int mode;
@@ -1862,8 +1875,7 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
     else if (c == 0) mode = 1;
     else if (c + 1 < L.n_chunks) mode = 2;
     else mode = 3;
-    if ((st = launch_gemm_store_unstaggered(mode, dz, L.chunk, n_rows, wt + v0, L.vpad, H, mpad,
-                                            dX, acc, H, s)))
+    if ((st = launch_gemm_store(mode, dz, L.chunk, n_rows, wt + v0, L.vpad, H, mpad, dX, acc, H, s)))
       return st;
   }
   return NMCE_OK;
@@ -2000,12 +2012,12 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
   uint16_t* dx_rows = static_cast<uint16_t*>(grad_hidden) + t0 * H;
   if (L.dx_splits == 1) {
     if ((st = launch_gemm_store(0, pt, L.ldt, nc, W, H, H, L.vpad, dx_rows, nullptr, H, s,
-                                kGroupMProducts, true, true, L.vpad, V)))
+                                true, true, L.vpad, V)))
       return st;
   } else {
     float* part = reinterpret_cast<float*>(ws + L.off_dxp);
     if ((st = launch_gemm_store(1, pt, L.ldt, nc, W, H, H, L.vpad, nullptr, part, H, s,
-                                kGroupMProducts, true, true, L.vpad, V,
+                                true, true, L.vpad, V,
                                 static_cast<int>(L.dx_splits), L.dx_ks, nc * H)))
       return st;
     const int64_t quads = nc * H / 4;
@@ -2029,7 +2041,7 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
   if ((st = launch_transpose(X + t0 * H, nc, H, H, xt, L.ldt, s))) return st;
   return launch_gemm_store(mode, pt, L.ldt, V, xt, L.ldt, H, L.ldt,
                            static_cast<uint16_t*>(grad_weight),
-                           reinterpret_cast<float*>(ws + L.off_acc), H, s, kGroupMProducts);
+                           reinterpret_cast<float*>(ws + L.off_acc), H, s);
 }
 
 }  // extern "C"
@@ -2067,6 +2079,6 @@ extern "C" int nmce_gemm_mn_bf16(int a_mn, const void* a, int64_t lda, const voi
   if (st) return st;
   return launch_gemm_store(0, static_cast<const uint16_t*>(a), lda, m,
                            static_cast<const uint16_t*>(b), ldb, n, k, static_cast<uint16_t*>(c),
-                           nullptr, ldc, static_cast<hipStream_t>(stream), kGroupM, a_mn != 0,
+                           nullptr, ldc, static_cast<hipStream_t>(stream), a_mn != 0,
                            true, k, k);
 }
