@@ -236,6 +236,23 @@ int nmce_ce_grad_rescale_unless(void* grad, int dtype, int64_t n_rows, int64_t v
                                 float* observed, void* stream);
 
 /*
+ * The two calls above for rows of any width and alignment: `vocab` up to the
+ * same limit, logits and grad aligned to their element. In
+ * nmce_ce_fwd_bwd_ragged every grad row must share its logits row's offset
+ * from a 16-byte boundary (logits - grad a multiple of 16 bytes, ld - ld_grad
+ * a multiple of 16 bytes' elements). Same results, bit for bit, as
+ * nmce_ce_fwd followed by nmce_ce_bwd_scaled.
+ */
+int nmce_ce_fwd_bwd_ragged(const void* logits, void* grad, int dtype, int64_t n_rows,
+                           int64_t vocab, int64_t ld, int64_t ld_grad, const int64_t* target,
+                           float* loss, float* g_max, float* g_sumexp_m1,
+                           const float* grad_expected, float* grad_assumed,
+                           const int32_t* target_bad, float gout_div, void* stream);
+int nmce_ce_grad_rescale_unless_ragged(void* grad, int dtype, int64_t n_rows, int64_t vocab,
+                                       int64_t ld_grad, const float* grad_output,
+                                       const float* assumed, float* observed, void* stream);
+
+/*
  * Measurement support (no counterpart in the reference): a plain copy of
  * `bytes` (multiple of 16, both pointers 16-byte aligned) with the loss
  * kernels' access pattern -- 16-byte non-temporal loads and stores. Its HBM

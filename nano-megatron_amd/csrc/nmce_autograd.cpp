@@ -89,9 +89,17 @@ void timed(const char* name, hipStream_t st, Launch&& launch) {
   check(status, name);
 }
 
+// Rows off the 16-byte grid or of a ragged width take the ragged entries.
+bool is_ragged(const at::Tensor& t, int64_t V, int64_t ld) {
+  const int64_t es = t.element_size();
+  return (V * es) % 16 != 0 || (ld * es) % 16 != 0 ||
+         reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0;
+}
+
 struct OnePassMean : public torch::autograd::Function<OnePassMean> {
-  // logits [..., V] viewable as [rows, V] (16-byte aligned rows, V a whole
-  // number of 16-byte vectors within the kernel's width; the wrapper checked),
+  // logits [..., V] viewable as [rows, V], V within the kernel's width (for a
+  // separate gradient buffer, rows that share its rows' offsets from a 16-byte
+  // boundary; the wrapper checked),
   // target the flat contiguous int64 targets, hint the one-element fp32
   // upstream value to assume, bad_flag the address of the target check's
   // device word (0 without a check; not an autograd input), inplace whether
@@ -113,12 +121,12 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
     at::Tensor assumed = at::empty({1}, out.options());
     hipStream_t st = stream_of(rows);
     float* stats = out.data_ptr<float>();
-    timed("nmce_ce_fwd_bwd", st, [&] {
-      return nmce_ce_fwd_bwd(rows.data_ptr(), grad.data_ptr(), code, n, V, ld, ldg,
-                             target.data_ptr<int64_t>(), stats, stats + n, stats + 2 * n,
-                             hint.data_ptr<float>(), assumed.data_ptr<float>(),
-                             reinterpret_cast<const int32_t*>(bad_flag),
-                             static_cast<float>(n), st);
+    const bool ragged = is_ragged(rows, V, ld);
+    timed(ragged ? "nmce_ce_fwd_bwd_ragged" : "nmce_ce_fwd_bwd", st, [&] {
+      return (ragged ? nmce_ce_fwd_bwd_ragged : nmce_ce_fwd_bwd)(
+          rows.data_ptr(), grad.data_ptr(), code, n, V, ld, ldg, target.data_ptr<int64_t>(), stats,
+          stats + n, stats + 2 * n, hint.data_ptr<float>(), assumed.data_ptr<float>(),
+          reinterpret_cast<const int32_t*>(bad_flag), static_cast<float>(n), st);
     });
     ctx->saved_data["inplace"] = inplace;
     ctx->saved_data["ld"] = ld;
@@ -158,10 +166,11 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
       at::Tensor grad = ctx->saved_data["grad_buf"].toTensor();
       const int64_t n = target.numel();
       hipStream_t st = stream_of(grad);
-      timed("nmce_ce_grad_rescale_unless", st, [&] {
-        return nmce_ce_grad_rescale_unless(grad.data_ptr(), dtype_code(grad), n, V, ld,
-                                           go.data_ptr<float>(), assumed.data_ptr<float>(),
-                                           hint.data_ptr<float>(), st);
+      const bool ragged = is_ragged(grad, V, ld);
+      timed(ragged ? "nmce_ce_grad_rescale_unless_ragged" : "nmce_ce_grad_rescale_unless", st, [&] {
+        return (ragged ? nmce_ce_grad_rescale_unless_ragged : nmce_ce_grad_rescale_unless)(
+            grad.data_ptr(), dtype_code(grad), n, V, ld, go.data_ptr<float>(),
+            assumed.data_ptr<float>(), hint.data_ptr<float>(), st);
       });
       ctx->saved_data["handed_out"] = true;
       ctx->saved_data["grad_buf"] = at::Tensor();

@@ -801,6 +801,104 @@ def test_one_pass_falls_back():
         assert torch.equal(grads[0], grads[1])
 
 
+RAGGED_WIDTHS = {torch.bfloat16: (1, 7, 9, 1001, 8191, 32767, 50257, 65535, 65537, 100277, 131071),
+                 torch.float32: (1, 3, 5, 1001, 4095, 16385, 32767, 32769, 50257, 65535)}
+
+
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_pass_ragged_rows(dtype, inplace):
+    """Rows of odd widths (every row starts at another offset from a 16-byte
+    boundary) through the one-pass kernel's ragged form, both sides of each
+    register-slot count and of the wide kernel, against the two-pass path: the
+    loss and the gradient for upstream 1.0 bit for bit; a miss (0.5, a
+    power-of-two ratio) too. Targets at the row's first and last columns (the
+    edge elements) and at the body's ends."""
+    import nmce
+    ctx = nmce.ParallelContext.single()
+    for v in RAGGED_WIDTHS[dtype]:
+        n = 600 if v <= 1001 else 37
+        print(f"[gpu] ragged one-pass v={v} {dtype} inplace={inplace}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(v)
+        x = (torch.randn(n, v, device=DEV, generator=g) * 3.0).to(dtype)
+        t = torch.randint(0, v, (n,), device=DEV, generator=g)
+        ends = torch.tensor([0, v - 1, min(7, v - 1), max(0, v - 8), min(8, v - 1)], device=DEV)
+        t[:min(n, 30)] = ends[torch.arange(min(n, 30), device=DEV) % 5]
+        x[1, :] = -1.0e30  # a row far below any floor's neighbourhood
+        x[2, 0], x[3, v - 1] = float("-inf"), float("inf") if v > 1 else 0.0
+        hint = torch.ones(1, device=DEV)
+        for upstream in (1.0, 0.5):
+            got = []
+            for one_pass in (True, False):
+                leaf = x.clone().requires_grad_(True)
+                hint.fill_(1.0)
+                loss = nmce.vocab_parallel_cross_entropy(leaf * 1.0, t, 0, v, ctx,
+                                                         inplace=inplace, one_pass=one_pass,
+                                                         upstream_hint=hint)
+                name = type(loss.grad_fn).__name__
+                assert ("OnePassMean" in loss.grad_fn.name()) == one_pass, name
+                (loss * upstream).backward()
+                got.append((loss.detach(), leaf.grad))
+            (l1, g1), (l2, g2) = got
+            assert torch.equal(l1, l2) or (l1.isnan() and l2.isnan()), (v, upstream)
+            ok = ((g1 == g2) | (g1.isnan() & g2.isnan())).all()
+            assert ok, f"gradient differs at v={v} upstream={upstream}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_pass_ragged_in_place_strided(dtype):
+    """In place into rows with a padded stride and a base off the 16-byte grid
+    (a view of a larger buffer): the loss and gradient bits of the two-pass
+    path, the rescale after a miss, a bad target leaving the logits as they
+    were, and nothing written outside the rows."""
+    import nmce
+    ctx = nmce.ParallelContext.single()
+    n, v, pad, off = 300, 999, 14, 3
+    g = torch.Generator(device=DEV).manual_seed(3)
+    store = torch.randn(n * (v + pad) + off, device=DEV, generator=g).to(dtype)
+    t = torch.randint(0, v, (n,), device=DEV, generator=g)
+
+    def rows(buf):
+        return buf[off:].as_strided((n, v), (v + pad, 1))
+
+    outside = torch.ones_like(store, dtype=torch.bool)
+    outside[off:].as_strided((n, v), (v + pad, 1)).fill_(False)
+    for upstream in (1.0, 0.25):
+        grads = []
+        for one_pass in (True, False):
+            buf = store.clone()
+            leaf = torch.zeros(1, device=DEV, dtype=dtype, requires_grad=True)
+            # a non-leaf alias of the rows, as a matmul's output would be
+            logits = _Alias.apply(leaf, rows(buf))
+            hint = torch.ones(1, device=DEV)
+            loss = nmce.vocab_parallel_cross_entropy(logits, t, 0, v, ctx, inplace=True,
+                                                     one_pass=one_pass, upstream_hint=hint)
+            (loss * upstream).backward()
+            assert torch.equal(buf[outside], store[outside])
+            grads.append((loss.detach(), rows(buf).clone()))
+        assert torch.equal(grads[0][0], grads[1][0])
+        assert torch.equal(grads[0][1], grads[1][1]), f"upstream {upstream}"
+    buf = store.clone()
+    logits = _Alias.apply(torch.zeros(1, device=DEV, dtype=dtype, requires_grad=True), rows(buf))
+    bad = t.clone()
+    bad[17] = v
+    with pytest.raises(ValueError, match="outside the model vocabulary"):
+        nmce.vocab_parallel_cross_entropy(logits, bad, 0, v, ctx, inplace=True)
+    assert torch.equal(buf, store)
+
+
+class _Alias(torch.autograd.Function):
+    """Hands a buffer on as a non-leaf tensor; its backward ends the graph."""
+
+    @staticmethod
+    def forward(ctx, anchor, buf):
+        return buf.view_as(buf)
+
+    @staticmethod
+    def backward(ctx, grad):
+        return torch.zeros(1, device=grad.device, dtype=grad.dtype), None
+
+
 class _HitRecorder:
     """Records (assumed, received) upstream values of every one-pass loss's
     backward: the value its forward assumed (saved by the autograd node) and

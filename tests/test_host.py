@@ -394,6 +394,46 @@ def test_one_pass_route_edges(lib):
     assert take(torch.zeros(0, 1000, dtype=torch.bfloat16), 1) is None
 
 
+def test_one_pass_ragged_route(lib):
+    """Which of the rows left out above take the one-pass kernel's ragged form:
+    any width up to the limit, and into a new buffer only rows that share its
+    rows' offsets from a 16-byte boundary. The C entries refuse what they
+    cannot address (CPU: argument errors only)."""
+    from nmce import cross_entropy as ce
+    bf = torch.bfloat16
+    take = ce._one_pass_ragged
+    assert take(torch.zeros(2, 1001, dtype=bf), 1, False)
+    assert take(torch.zeros(2, 1001), 1, False)
+    assert take(torch.zeros(2, 3, 131071, dtype=bf), 1, False)
+    assert not take(torch.zeros(2, 131073, dtype=bf), 1, True)
+    assert not take(torch.zeros(2, 65537), 1, True)
+    assert not take(torch.zeros(2, 1001, dtype=bf), 2, True)
+    assert not take(torch.zeros(2, 1001, dtype=torch.float16), 1, True)
+    assert not take(torch.zeros(0, 1001, dtype=bf), 1, True)
+    padded = torch.zeros(4, 1009, dtype=bf)[:, :1001]  # stride 8 past the width
+    assert take(padded, 1, False) and take(padded, 1, True)
+    odd = torch.zeros(4, 1007, dtype=bf)[:, :1001]     # stride 6 past the width
+    assert not take(odd, 1, False) and take(odd, 1, True)
+    shifted = torch.zeros(1 + 4 * 1001, dtype=bf)[1:].view(4, 1001)
+    assert not take(shifted, 1, False) and take(shifted, 1, True)
+    p = 1 << 20
+    fb = lib.nmce_ce_fwd_bwd_ragged
+    args = (p, p, p, p, p, p, None)
+    assert fb(p, p, 5, 4, 9, 9, 9, *args, 4.0, None) == -1
+    assert fb(p, p, 1, 4, 131073, 131073, 131073, *args, 4.0, None) == -2
+    assert fb(p, p, 1, 4, 9, 8, 9, *args, 4.0, None) == -2
+    assert fb(p, p, 1, 4, 9, 10, 9, *args, 4.0, None) == -2         # in place: one stride
+    assert fb(p, p + 2, 1, 4, 9, 9, 9, *args, 4.0, None) == -3      # offsets differ
+    assert fb(p + 1, p + 1, 1, 4, 9, 9, 9, *args, 4.0, None) == -3
+    assert fb(p, p + 4096, 1, 4, 9, 11, 9, *args, 4.0, None) == -3  # strides differ by 4 bytes
+    assert fb(p, None, 1, 4, 9, 9, 9, *args, 4.0, None) == -4
+    rs = lib.nmce_ce_grad_rescale_unless_ragged
+    assert rs(p, 5, 4, 9, 9, p, p, None, None) == -1
+    assert rs(p, 1, 4, 9, 8, p, p, None, None) == -2
+    assert rs(p + 1, 1, 4, 9, 9, p, p, None, None) == -3
+    assert rs(p, 1, 4, 9, 9, None, p, None, None) == -4
+
+
 def test_wide_buffer_stores_go_through_the_helper():
     """Buffer stores wider than 8 bytes are issued only by buffer_store_b128,
     which keeps the scalar offset the constant 0: with a register scalar
