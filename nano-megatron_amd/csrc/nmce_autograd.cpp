@@ -25,6 +25,7 @@
 #include <atomic>
 #include <chrono>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <tuple>
@@ -233,25 +234,30 @@ at::Tensor flag_word(const at::Tensor& like, hipStream_t st) {
   return it->second;
 }
 
-// Pinned count words with their events, pooled and reused once a check has
-// been waited for (the kernel writes the word through its host mapping).
+// Pinned count words with their events, pooled per device (an event belongs
+// to one) and reused once a check has been waited for (the kernel writes the
+// word through its host mapping).
 struct CheckSlot {
   at::Tensor host;
   hipEvent_t event = nullptr;
+  int device = 0;
 };
 std::mutex g_slot_lock;
-std::vector<CheckSlot> g_slots;
+std::map<int, std::vector<CheckSlot>> g_slots;
 
-CheckSlot take_slot() {
+// The caller has made `device` the current one.
+CheckSlot take_slot(int device) {
   {
     std::lock_guard<std::mutex> g(g_slot_lock);
-    if (!g_slots.empty()) {
-      CheckSlot s = g_slots.back();
-      g_slots.pop_back();
+    std::vector<CheckSlot>& free = g_slots[device];
+    if (!free.empty()) {
+      CheckSlot s = free.back();
+      free.pop_back();
       return s;
     }
   }
   CheckSlot s;
+  s.device = device;
   s.host = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
   TORCH_CHECK(hipEventCreateWithFlags(&s.event, hipEventDisableTiming) == hipSuccess,
               "nmce: hipEventCreateWithFlags failed");
@@ -285,12 +291,66 @@ class CheckGuard {
   ~CheckGuard() {
     if (recorded_) (void)hipEventSynchronize(slot_.event);
     std::lock_guard<std::mutex> g(g_slot_lock);
-    g_slots.push_back(std::move(slot_));
+    g_slots[slot_.device].push_back(std::move(slot_));
   }
 
  private:
   CheckSlot slot_;
   bool recorded_ = false;
+};
+
+// The check of flat contiguous targets on the current stream of their device,
+// its event recorded behind it; `flag` is that stream's device word.
+std::unique_ptr<CheckGuard> launch_check(const at::Tensor& target, int64_t vocab_total,
+                                         const at::Tensor& flag, hipStream_t st) {
+  auto guard = std::make_unique<CheckGuard>(take_slot(target.device().index()));
+  timed("nmce_validate_targets_once", st, [&] {
+    return nmce_validate_targets_once(target.data_ptr<int64_t>(), target.numel(), vocab_total,
+                                      guard->host(), flag.data_ptr<int32_t>(), st);
+  });
+  if (hipEventRecord(guard->event(), st) != hipSuccess) {
+    // The check may still write the slot's word: let it finish first.
+    (void)hipStreamSynchronize(st);
+    TORCH_CHECK(false, "nmce: hipEventRecord failed");
+  }
+  guard->recorded();
+  return guard;
+}
+
+// The device word of checks that no kernel reads the result of (their callers
+// write nothing until the host has it), one per device: apart from the words
+// that one-pass kernels read, which another thread's check on the same stream
+// must not touch.
+at::Tensor unread_word(const at::Tensor& like) {
+  static std::map<int, at::Tensor> words;
+  std::lock_guard<std::mutex> g(g_flag_lock);
+  at::Tensor& w = words[static_cast<int>(like.device().index())];
+  if (!w.defined()) w = at::empty({1}, like.options().dtype(at::kInt));
+  return w;
+}
+
+// A target check in flight, for the callers that launch their loss kernels
+// from Python meanwhile: wait() gives the count of bad targets (once the check
+// is over) and the slot back; so does the end of its life.
+class TargetCheck {
+ public:
+  TargetCheck(const at::Tensor& target, int64_t vocab_total) {
+    const c10::DeviceGuard device_guard(target.device());
+    hipStream_t st = stream_of(target);
+    guard_ = launch_check(target, vocab_total, unread_word(target), st);
+  }
+  bool query() const { return !guard_ || hipEventQuery(guard_->event()) == hipSuccess; }
+  int32_t wait() {
+    if (guard_) {
+      count_ = guard_->wait();
+      guard_.reset();
+    }
+    return count_;
+  }
+
+ private:
+  std::unique_ptr<CheckGuard> guard_;
+  int32_t count_ = 0;
 };
 
 at::Tensor one_pass_mean(const at::Tensor& logits, const at::Tensor& target,
@@ -311,20 +371,11 @@ at::Tensor one_pass_mean_checked(const at::Tensor& logits, const at::Tensor& tar
   const c10::DeviceGuard device_guard(logits.device());
   hipStream_t st = stream_of(logits);
   const at::Tensor flag = flag_word(logits, st);
-  CheckGuard guard(take_slot());
-  check(nmce_validate_targets_once(target.data_ptr<int64_t>(), target.numel(), vocab_total,
-                                   guard.host(), flag.data_ptr<int32_t>(), st),
-        "nmce_validate_targets_once");
-  if (hipEventRecord(guard.event(), st) != hipSuccess) {
-    // The check may still write the slot's word: let it finish first.
-    (void)hipStreamSynchronize(st);
-    TORCH_CHECK(false, "nmce: hipEventRecord failed");
-  }
-  guard.recorded();
+  const std::unique_ptr<CheckGuard> guard = launch_check(target, vocab_total, flag, st);
   at::Tensor loss = OnePassMean::apply(logits, target, hint,
                                        reinterpret_cast<int64_t>(flag.data_ptr<int32_t>()),
                                        inplace, vocab_start);
-  if (guard.wait() != 0)
+  if (guard->wait() != 0)
     throw pybind11::value_error("target token id is outside the model vocabulary");
   return loss;
 }
@@ -394,6 +445,11 @@ PYBIND11_MODULE(_nmce_autograd, m) {
   m.def("one_pass_mean", &one_pass_mean, "mean one-pass loss (forward + backward in C++)");
   m.def("one_pass_mean_checked", &one_pass_mean_checked,
         "one_pass_mean after the target check; ValueError on a target outside the vocabulary");
+  pybind11::class_<TargetCheck>(m, "TargetCheck",
+                                "a target check in flight on the targets' current stream")
+      .def(pybind11::init<const at::Tensor&, int64_t>())
+      .def("query", &TargetCheck::query, "whether the check is over")
+      .def("wait", &TargetCheck::wait, "wait for it; the count of bad targets");
   m.def("assumed_of", &assumed_of, "the assumed upstream value saved by a one-pass loss");
   m.def("set_timing", &set_timing, "time every launch with HIP events while on");
   m.def("take_timeline", &take_timeline, "(name, ms) of the launches timed since the last call");

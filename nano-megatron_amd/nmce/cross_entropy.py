@@ -63,7 +63,6 @@ must be built; anything else raises.
 from __future__ import annotations
 
 import sys
-import threading
 
 import torch
 import torch.distributed as dist
@@ -150,60 +149,20 @@ def _check_inputs(logits: torch.Tensor, target: torch.Tensor, vocab_start: int,
             f"[{vocab_start}, {vocab_end}) has {vocab_end - vocab_start}")
 
 
-# Event queries (about a microsecond each) before the target check falls back
-# to a blocking wait.
-_CHECK_POLLS = 200
-
-
-# Pinned count buffers and their events, per device, reused once a check is
-# over (allocating them cost a few microseconds per call, which a small batch
-# pays every step).
-_check_free: dict[int, list] = {}
-_check_lock = threading.Lock()
-
-
-def _check_slot(dev_index: int, slots: int):
-    with _check_lock:
-        free = _check_free.setdefault(dev_index, [])
-        for i, (host, event) in enumerate(free):
-            if host.numel() >= slots:
-                return free.pop(i)
-    cap = 1 << max(slots - 1, 0).bit_length()
-    return torch.empty(cap, dtype=torch.int32, pin_memory=True), torch.cuda.Event()
-
-
 class _PendingCheck:
-    """Bad-target counts on their way to pinned host memory.
+    """A target check in flight: its kernel writes the count of bad targets
+    straight into a pooled pinned word, which goes back to its pool once the
+    check is over. Every caller ends with ``raise_if_bad()`` or, when it leaves
+    early on an exception, ``wait()``. ``event.query()`` tells whether the
+    check is over."""
 
-    The check kernel writes the counts straight into ``host`` (pinned memory
-    is mapped into the device's address space at its host address), so the
-    buffer must not be reused until ``event`` has completed: every caller ends
-    with ``raise_if_bad()`` or, when it leaves early on an exception,
-    ``wait()``, which return the buffer and the event to the per-device pool.
-    """
-
-    def __init__(self, dev_index: int, host: torch.Tensor, event: torch.cuda.Event, slots: int):
-        self.dev_index = dev_index
-        self.host = host
+    def __init__(self, event):
         self.event = event
-        self.slots = slots
         self.bad = None
 
     def wait(self) -> None:
-        if self.bad is not None:
-            return
-        # The counts usually reach the host within microseconds of the call:
-        # poll first, so that a blocking wait's wake-up latency (tens of
-        # microseconds, per step of a small batch) is paid only by long waits.
-        event = self.event
-        for _ in range(_CHECK_POLLS):
-            if event.query():
-                break
-        else:
-            event.synchronize()
-        self.bad = bool(self.host.numpy()[:self.slots].any())
-        with _check_lock:
-            _check_free.setdefault(self.dev_index, []).append((self.host, self.event))
+        if self.bad is None:
+            self.bad = self.event.wait() != 0
 
     def raise_if_bad(self) -> None:
         self.wait()
@@ -211,49 +170,23 @@ class _PendingCheck:
             raise ValueError("target token id is outside the model vocabulary")
 
 
-_side_streams: dict[int, torch.cuda.Stream] = {}
-
-
-def _side_stream(device: torch.device) -> torch.cuda.Stream:
-    """A per-device stream (default priority) for the target check."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    stream = _side_streams.get(idx)
-    if stream is None:
-        stream = torch.cuda.Stream(device=idx)
-        _side_streams[idx] = stream
-    return stream
-
-
 def launch_target_check(target: torch.Tensor, vocab_size: int) -> _PendingCheck | None:
     """Start the target check of cross_entropy.py:79-81 without blocking.
 
-    One kernel counts targets outside ``[0, vocab_size)`` straight into pinned
-    host memory, on a side stream ordered after the work already queued on the
-    current stream; ``raise_if_bad()`` on the result waits for that kernel
-    alone. The loss kernels go on the current stream meanwhile, so the check
-    adds nothing to the loss stream's timeline. (The one-pass path runs its
-    check on the loss stream, with a device word its kernel reads, inside the
-    C++ call: ``_nmce_autograd.one_pass_mean_checked``.)
+    One workgroup counts the targets outside ``[0, vocab_size)`` on the
+    current stream, in front of the loss kernels that the caller enqueues
+    next; ``raise_if_bad()`` on the result waits for that kernel alone. It is
+    one call into the C++ module: a check on a side stream, with its events and
+    stream switches in Python, cost the host 60 us a call, a third of what the
+    fused loss of a few hundred tokens takes, where the check itself takes the
+    loss stream 2-4 us.
     """
-    lib = _lib.load()
     t = target.reshape(-1)
     if not t.is_contiguous():
         t = t.contiguous()
-    n = t.numel()
-    if n == 0:
+    if t.numel() == 0:
         return None
-    slots = lib.nmce_validate_slots(n)
-    dev_index = t.device.index if t.device.index is not None else torch.cuda.current_device()
-    host, event = _check_slot(dev_index, slots)
-    main = torch.cuda.current_stream(t.device)
-    side = _side_stream(t.device)
-    side.wait_stream(main)  # the targets are complete in the current stream's order
-    with torch.cuda.stream(side):
-        _launch("nmce_validate_targets", lib.nmce_validate_targets, t.data_ptr(), n,
-                vocab_size, host.data_ptr(), side.cuda_stream)
-        event.record(side)
-    t.record_stream(side)  # keep the targets' memory until the side stream is done
-    return _PendingCheck(dev_index, host, event, slots)
+    return _PendingCheck(_lib.autograd_ext().TargetCheck(t, vocab_size))
 
 
 def validate_targets(target: torch.Tensor, vocab_size: int) -> None:
