@@ -118,7 +118,8 @@ constexpr float kMaxFloorL = -1.0e38f;
 constexpr int kPartialRows = kWaveM;
 
 // A wave's 128 x 128 results: c[i][j] is the 16 x 16 block of rows 16 i and
-// columns 16 j; lane l holds column l % 16, rows 4 (l / 16) + e of it.
+// columns 16 j; lane l holds column l % 16, rows 4 (l / 16) + e of it, or,
+// from a main loop with kRows, row l % 16, columns 4 (l / 16) + e.
 struct Acc {
   f32x4_t c[kF][kF];
 };
@@ -321,7 +322,11 @@ struct Frags {
 // sub-step of kt; its B into stage kt's buffer, after the barrier at which every
 // wave has read the last of stage kt. That barrier waits for all but the wave's
 // newest eight loads (stage kt + 2's A).
-template <bool kAMN, bool kBMN>
+//
+// kRows hands the MFMA its operands the other way round, which gives the lane
+// four columns of one row instead of four rows of one column (the same sums):
+// what an epilogue wants that stores rows.
+template <bool kAMN, bool kBMN, bool kRows = false>
 __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda,
                                               int64_t M, const uint16_t* __restrict__ B,
                                               int64_t ldb, int64_t N, int64_t K, int64_t m0,
@@ -400,13 +405,19 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   // MFMAs that no read follows: an MFMA's 16 cycles hide about three other
   // instructions.
   constexpr int kLoadGap = 6;
+  auto mma = [&](int i, int j, const Set& f) {
+    if constexpr (kRows)
+      mfma_16x16x32(acc.c[i][j], f.b[j], f.a[i]);
+    else
+      mfma_16x16x32(acc.c[i][j], f.a[i], f.b[j]);
+  };
   auto step = [&](const char* pa, const char* pb, int s, Set& next, const Set& cur, auto loads,
                   auto&& load) {
     constexpr int kLoads = decltype(loads)::value;
 #pragma unroll
     for (int x = 0; x < kF * kF; ++x) {
       const int i = x / kF, j = (i & 1) ? kF - 1 - x % kF : x % kF;
-      mfma_16x16x32(acc.c[i][j], cur.a[i], cur.b[j]);
+      mma(i, j, cur);
       if (x % 3 != 0 && x / 3 < 2 * kF) read(pa, pb, s, next, x / 3, x % 3 - 1);
       if (x % kLoadGap == 0 && x / kLoadGap < kLoads) load(x / kLoadGap);
       if (kAMN || kBMN || x % 3 == 2) __builtin_amdgcn_sched_barrier(0);
@@ -460,7 +471,7 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   }
   step(lds + a_cur, lds_b + (kt & 1) * kStage, 1, f1, f0, NoLoads{}, none);
 #pragma unroll
-  for (int x = 0; x < kF * kF; ++x) mfma_16x16x32(acc.c[x / kF][x % kF], f1.a[x / kF], f1.b[x % kF]);
+  for (int x = 0; x < kF * kF; ++x) mma(x / kF, x % kF, f1);
   // The compiler does not know the MFMAs' latency: let the last ones finish
   // before anything reads the accumulators.
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -493,21 +504,6 @@ __device__ __forceinline__ uint32_t* stage_word(uint32_t* P, int wm, int i, int 
   const int lane_swz = ((g & 1) << 4) | ((g >> 1) << 5);
   const int block_swz = ((i & 3) << 2) | ((i >> 2) << 4);
   return P + (wm * (kWaveM / 2) + 2 * g) * kBN + (8 * i + h) * kBN + ((c ^ lane_swz) ^ block_swz);
-}
-
-// Stage the wave's results as bf16.
-__device__ __forceinline__ void stage_bf16(const Acc& acc, uint32_t* P, int wm, int wn, int lane) {
-  const int g = lane >> 4;
-#pragma unroll
-  for (int j = 0; j < kF; ++j) {
-    const int c = wn * kWaveN + 16 * j + (lane & 15);
-#pragma unroll
-    for (int i = 0; i < kF; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        *stage_word(P, wm, i, g, h, c) =
-            pack_bf16x2(acc.c[i][j][2 * h], acc.c[i][j][2 * h + 1]);
-  }
 }
 
 // 8 columns t0 .. t0 + 7 of staged rows 2 vp (lo) and 2 vp + 1 (hi), bf16.
@@ -905,14 +901,22 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
   }
 }
 
+// The stored products' epilogues take the results row by row (kRows): lane l
+// holds, of each 16x16 block, row l % 16 and columns 4 g .. 4 g + 3 (g = l /
+// 16), and stages them through the freed LDS, so that whole row segments of
+// 512 bytes (bf16) or 1 KiB (fp32) leave. Stored straight from the registers
+// they are segments of 64 bytes: 1358 against 1415 TFLOP/s with fp32 out on
+// 128256 x 4096 x 4096, 1457 against 1485 with bf16.
+//
 // The fp32 epilogues (modes 1-3 of gemm_store_kernel). The 256x256 fp32 tile
 // goes through the freed LDS in two passes of 128 rows: pass q takes row
 // blocks i = 4q .. 4q + 3 of every wave, i.e. tile rows 64 q .. 64 q + 63
 // and 128 + 64 q .. 128 + 64 q + 63, so each pass reads its own half of the
 // accumulator registers. Staged row r (1 KiB) is tile row
-// 128 (r >> 6) + 64 q + (r & 63); its 16-byte chunk c sits at c ^ 4 ((r >> 2)
-// & 3), which puts the four rows one ds_write_b32 covers (r, r + 4, r + 8,
-// r + 12) on the four 16-bank groups. Every thread then moves 32 chunks:
+// 128 (r >> 6) + 64 q + (r & 63); its 16-byte chunk c sits at c ^ (r & 15),
+// which puts the 16 rows that 16 lanes write on distinct 16-byte bank groups
+// (the lane's four columns of a block are one chunk). Every thread then moves
+// 32 chunks:
 // staged row 4 p + wave, chunk lane, so a wave's access is one 1 KiB row
 // segment of Cf (or 512 bytes of C).
 // kVec (N % 4 == 0, ldc % 4 == 0, Cf 16-byte and C 8-byte aligned, 512 rows
@@ -978,21 +982,18 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
       }
     }
 #pragma unroll
-    for (int j = 0; j < kF; ++j) {
-      const int c = wn * kWaveN + 16 * j + (lane & 15);
+    for (int j = 0; j < kF; ++j)
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = wm * 64 + 16 * f + 4 * g + e;
-          S[r * kBN + (c ^ (g << 4))] = acc.c[4 * q + f][j][e];
-        }
-    }
+      for (int f = 0; f < 4; ++f) {
+        const int r = wm * 64 + 16 * f + (lane & 15);
+        const int c = (wn * (kWaveN / 4) + 4 * j + g) ^ (lane & 15);
+        *reinterpret_cast<f32x4_t*>(S + r * kBN + 4 * c) = acc.c[4 * q + f][j];
+      }
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
       const int r = p * kRowsPerPass + wave;
-      const u32x4 sv = *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ ((p & 3) << 2)) << 2));
+      const u32x4 sv = *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ ((4 * p + wave) & 15)) << 2));
       if constexpr (!kVec) {
         const int64_t row = row0 + row_off(p);
         const float sf[4] = {__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z),
@@ -1040,55 +1041,65 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
   }
 }
 
-// bf16 out through the freed LDS, as lmhead_p_kernel stages P^T: words of two
-// rows (vp = row / 2) per column, then 16-byte stores of 512-byte row
-// segments. Tiles that reach past N, and outputs that are not 16-byte
-// aligned, store element by element.
+// bf16 out: rows of 512 bytes whose 16-byte chunk c sits at c ^ (row & 15):
+// the 16 rows of a block that 32 lanes write 8 bytes of each are on distinct
+// 16-byte bank groups. The stores are non-temporal: the product is read by a
+// later kernel, if at all, and its lines would take L2 from the next tiles'
+// operands. Against words of two rows, unscrambled on the way out, and cached
+// stores: K = 512 875 -> 1030 TFLOP/s, K = 1600 1166 -> 1247, K = 4096 1445 ->
+// 1459. Tiles that reach past M or N, and outputs that are not 16-byte
+// aligned, test every row and column.
 __device__ __forceinline__ void store_bf16_tile(const Acc& acc, char* lds,
                                                 uint16_t* __restrict__ C, int64_t ldc, int64_t M,
                                                 int64_t N, int64_t m0, int64_t n0) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
+  const int g = lane >> 4, c = lane & 15;
   const bool vec_ok = (ldc & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   __syncthreads();  // every wave is done with the operand buffers
-  uint32_t* P = reinterpret_cast<uint32_t*>(lds);
-  stage_bf16(acc, P, wm, wn, lane);
+  char* row = lds + (wm * kWaveM + c) * (kBN * 2) + 8 * (g & 1);
+#pragma unroll
+  for (int j = 0; j < kF; ++j) {
+    char* at = row + (((wn * (kWaveN / 8) + 2 * j + (g >> 1)) ^ c) << 4);
+#pragma unroll
+    for (int i = 0; i < kF; ++i)
+      *reinterpret_cast<u32x2*>(at + i * (16 * kBN * 2)) =
+          u32x2{pack_bf16x2(acc.c[i][j][0], acc.c[i][j][1]),
+                pack_bf16x2(acc.c[i][j][2], acc.c[i][j][3])};
+  }
   __syncthreads();
-  const int vp0 = static_cast<int>(threadIdx.x) / (kBN / 8);
-  const int c0 = 8 * (static_cast<int>(threadIdx.x) % (kBN / 8));
-  constexpr int kVpStep = kThreads / (kBN / 8);
+  constexpr int kRowStep = kThreads / (kBN / 8);  // 8 rows of 32 chunks at a time
+  constexpr int kIters = kBM / kRowStep;
+  const int r0 = static_cast<int>(threadIdx.x) / (kBN / 8);
+  const int q = static_cast<int>(threadIdx.x) % (kBN / 8);
+  auto staged = [&](int it) {
+    const int r = r0 + it * kRowStep;
+    return *reinterpret_cast<const u32x4*>(lds + r * (kBN * 2) + ((q ^ (r & 15)) << 4));
+  };
   if (vec_ok && m0 + kBM <= M && n0 + kBN <= N) {  // every store in bounds: no tests
-    uint16_t* dst = C + (m0 + 2 * vp0) * ldc + n0 + c0;
-#pragma unroll 4
-    for (int it = 0; it < kStagedIters; ++it) {
-      u32x4 lo, hi;
-      staged_rows(P, vp0 + it * kVpStep, c0, lo, hi);
-      *reinterpret_cast<u32x4*>(dst) = lo;
-      *reinterpret_cast<u32x4*>(dst + ldc) = hi;
-      dst += 2 * kVpStep * ldc;
+    uint16_t* dst = C + (m0 + r0) * ldc + n0 + 8 * q;
+#pragma unroll 8
+    for (int it = 0; it < kIters; ++it) {
+      store_stream(reinterpret_cast<u32x4*>(dst), staged(it));
+      dst += kRowStep * ldc;
     }
     return;
   }
+  const int64_t col = n0 + 8 * q;
 #pragma unroll 2
-  for (int it = 0; it < kStagedIters; ++it) {
-    const int vp = vp0 + it * kVpStep;
-    u32x4 lo, hi;
-    staged_rows(P, vp, c0, lo, hi);
-    const int64_t col0 = n0 + c0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t row = m0 + 2 * vp + h;
-      if (row >= M || col0 >= N) continue;
-      const u32x4 w = h ? hi : lo;
-      uint16_t* dst = C + row * ldc + col0;
-      if (vec_ok && col0 + 8 <= N) {
-        *reinterpret_cast<u32x4*>(dst) = w;
-      } else {
-        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-        for (int e = 0; e < 8 && col0 + e < N; ++e)
-          dst[e] = static_cast<uint16_t>(e & 1 ? ws[e >> 1] >> 16 : ws[e >> 1] & 0xffffu);
-      }
+  for (int it = 0; it < kIters; ++it) {
+    const u32x4 w = staged(it);
+    const int64_t r = m0 + r0 + it * kRowStep;
+    if (r >= M || col >= N) continue;
+    uint16_t* dst = C + r * ldc + col;
+    if (vec_ok && col + 8 <= N) {
+      store_stream(reinterpret_cast<u32x4*>(dst), w);
+    } else {
+      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+      for (int e = 0; e < 8 && col + e < N; ++e)
+        dst[e] = static_cast<uint16_t>(e & 1 ? ws[e >> 1] >> 16 : ws[e >> 1] & 0xffffu);
     }
   }
 }
@@ -1104,8 +1115,7 @@ __device__ __forceinline__ void store_bf16_tile(const Acc& acc, char* lds,
 // partial product to Cf + s * split_stride. Copies are numbered as extra tile
 // rows (split-major), so the XCD bands keep tiles of one K range together.
 // kVec (modes 1-3): the output meets store_f32_tile's conditions for 16-byte
-// accesses (the host checks them); otherwise the half tiles leave element by
-// element.
+// accesses (the host checks them); otherwise it leaves element by element.
 // ---------------------------------------------------------------------------
 template <int kMode, bool kAMN = false, bool kBMN = false, bool kVec = true>
 __global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
@@ -1129,8 +1139,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
   const uint16_t* Bs = kBMN ? B + k0 * ldb : B + k0;
   Cf += split * split_stride;
   Acc acc;
-  gemm_mainloop<kAMN, kBMN>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc, ka_rows - k0,
-                            kb_rows - k0);
+  gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
+                                            ka_rows - k0, kb_rows - k0);
   if constexpr (kMode != 0)
     store_f32_tile<kMode, kVec>(acc, lds, Cf, C, ldc, M, N, m0, n0);
   else
