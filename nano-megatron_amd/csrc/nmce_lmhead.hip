@@ -326,12 +326,23 @@ struct Frags {
 // kRows hands the MFMA its operands the other way round, which gives the lane
 // four columns of one row instead of four rows of one column (the same sums):
 // what an epilogue wants that stores rows.
-template <bool kAMN, bool kBMN, bool kRows = false>
+//
+// touch(i), i = 0 .. kTouches - 1, is called in every second one of the last K
+// steps that load a whole stage (as many as there are): a load whose value
+// nobody needs, that brings a part of what the epilogue will read nearer
+// (TouchTile). It is issued behind the step's A loads, so that step's wait
+// leaves nine in flight and it has a whole K step to come back.
+constexpr int kTouches = 8;
+struct NoTouch {
+  __device__ __forceinline__ uint32_t operator()(int) const { return 0; }
+};
+template <bool kAMN, bool kBMN, bool kRows = false, typename Touch = NoTouch>
 __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda,
                                               int64_t M, const uint16_t* __restrict__ B,
                                               int64_t ldb, int64_t N, int64_t K, int64_t m0,
                                               int64_t n0, char* lds, Acc& acc,
-                                              int64_t ka_rows = 0, int64_t kb_rows = 0) {
+                                              int64_t ka_rows = 0, int64_t kb_rows = 0,
+                                              Touch touch = {}) {
   const int lane = threadIdx.x & 63;
   // The wave index is uniform across the wave; say so, so that the load
   // bases and LDS destinations below live in scalar registers.
@@ -441,13 +452,19 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   const int full_a = la.full_stages(kt_n), full_b = lb.full_stages(kt_n);
   const int full = full_a < full_b ? full_a : full_b;
   int kt = 0;
-  for (; kt + 2 < full; ++kt) {
+  auto k_step = [&](auto touching, int i) {
     const int a_nxt = next_a(a_cur);
     const int b_cur = (kt & 1) * kStage;
     char* da = lds + prev_a(a_cur) + lds_w;
     la.at(kt + 2);
     step(lds + a_cur, lds_b + b_cur, 1, f1, f0, Loads{}, [&](int l) { la.load(da, l); });
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    uint32_t t = 0;
+    if constexpr (touching.value) {
+      t = touch(i);
+      asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     char* db = lds_b + b_cur + lds_w;
@@ -455,6 +472,21 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
     step(lds + a_nxt, lds_b + (kStage - b_cur), 0, f0, f1, Loads{},
          [&](int l) { lb.load(db, l); });
     a_cur = a_nxt;
+    return t;
+  };
+  constexpr bool kTouch = !std::is_same<Touch, NoTouch>::value;
+  for (; kt + 2 + (kTouch ? 2 * kTouches : 0) < full; ++kt) k_step(std::false_type{}, 0);
+  if constexpr (kTouch) {
+    for (int i = 0; kt + 3 < full; ++kt, ++i) {
+      const uint32_t t = k_step(std::true_type{}, i);
+      ++kt;
+      k_step(std::false_type{}, 0);
+      asm volatile("" ::"v"(t));  // back since this step's wait
+    }
+    if (kt + 2 < full) {
+      k_step(std::false_type{}, 0);
+      ++kt;
+    }
   }
   static_assert(kBlocksPerWave == 8, "the loop's wait leaves one stage's A loads in flight");
   for (; kt + 1 < kt_n; ++kt) {
@@ -1041,6 +1073,34 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
   }
 }
 
+// A part of the fp32 tile that store_f32_tile will add to, read ahead: touch i
+// reads one value of each of 2048 / kTouches 128-byte lines (a thread each) of
+// the tile's rows 32 i .. 32 i + 31. The lines come from HBM while the matrix
+// units work, and the epilogue's loads, all compute units' at once, find them
+// in the caches: [16384, 4096] x [128256, 4096] in four chunks 38.36 -> 38.21
+// ms, in eight consecutive steps as in every second one. Offsets past the matrix are out of the resource's range (no
+// access); the columns past N of a row before the last are the next row's.
+// The caller has checked that 512 rows lie within 32-bit offsets.
+struct TouchTile {
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off, step;
+  __device__ __forceinline__ void init(const float* Cf, int64_t ldc, int64_t M, int64_t N,
+                                       int64_t m0, int64_t n0) {
+    const int64_t rows = (M - m0) < kBM ? (M - m0) : kBM;
+    const int64_t cols = (N - n0) < kBN ? (N - n0) : kBN;
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Cf) + m0 * ldc + n0, 0,
+                                             static_cast<int>(((rows - 1) * ldc + cols) * 4),
+                                             0x00020000);
+    const uint32_t row_bytes = static_cast<uint32_t>(ldc * 4);
+    off = (threadIdx.x >> 3) * row_bytes + (threadIdx.x & 7) * 128u;
+    step = (kThreads / 8) * row_bytes;
+  }
+  __device__ __forceinline__ uint32_t operator()(int i) const {
+    return __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + static_cast<uint32_t>(i) * step, 0, 0);
+  }
+};
+static_assert(kTouches * (kThreads / 8) == kBM && kBN * 4 == 8 * 128, "the touches cover a tile");
+
 // bf16 out: rows of 512 bytes whose 16-byte chunk c sits at c ^ (row & 15):
 // the 16 rows of a block that 32 lanes write 8 bytes of each are on distinct
 // 16-byte bank groups. The stores are non-temporal: the product is read by a
@@ -1139,8 +1199,15 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
   const uint16_t* Bs = kBMN ? B + k0 * ldb : B + k0;
   Cf += split * split_stride;
   Acc acc;
-  gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
-                                            ka_rows - k0, kb_rows - k0);
+  if constexpr (kMode >= 2 && kVec) {
+    TouchTile touch;
+    touch.init(Cf, ldc, M, N, m0, n0);
+    gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
+                                              ka_rows - k0, kb_rows - k0, touch);
+  } else {
+    gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
+                                              ka_rows - k0, kb_rows - k0);
+  }
   if constexpr (kMode != 0)
     store_f32_tile<kMode, kVec>(acc, lds, Cf, C, ldc, M, N, m0, n0);
   else

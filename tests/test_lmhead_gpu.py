@@ -778,7 +778,7 @@ def test_one_pass_fused_many_k_ranges(n, h, v):
     check_grad(wd.grad.float().cpu().numpy(), rdw, "dW")
 
 
-@pytest.mark.parametrize("n,chunk", [(2048, 2048), (2000, 512)])
+@pytest.mark.parametrize("n,chunk", [(2048, 2048), (2000, 512), (3700, 1280)])
 def test_fused_dw_product_is_bit_identical(n, chunk):
     """The one-pass path's dW product of each token chunk (V = 33000, 129
     tile rows with a ragged last one, x H = 1024) equals the GEMM core's own
@@ -786,7 +786,8 @@ def test_fused_dw_product_is_bit_identical(n, chunk):
     one chunk (bf16 out) nmce_gemm_mn_bf16's product; with four chunks, the
     last one short (fp32 accumulation, rounded to bf16 by the last), the
     core's fp32 products of the chunks (nmce_gemm_nt_bf16 on X_c^T, zero past
-    the chunk's tokens) summed in chunk order and rounded once. Compared as
+    the chunk's tokens) summed in chunk order and rounded once. Chunks of 1280
+    have more K steps (20) than those that read the accumulator ahead (16). Compared as
     values (the two may differ in the sign of a zero only). The fp32
     read-add-store epilogue checked here is where a VALU write of a 16-byte
     store's data registers right after the store corrupts the first dword of
