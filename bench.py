@@ -459,13 +459,13 @@ def run_fused(args, name: str, steps: int, warmup: int, one_pass: bool = True,
         del dst
 
     gemm_flops = 2.0 * n * v * h   # one product over every token
-    # Algorithmic flops per step of each C entry: the one-pass statistics call
+    # Algorithmic flops per step of each C entry: the one-pass chunk's loss call
     # is the forward GEMM of its chunk, the gradients call the dX and dW
     # GEMMs of its chunk; the recomputing path's statistics call is the
     # forward GEMM and its backward call the three GEMMs of the backward
     # (the recomputation counted as executed, not as algorithmic work).
     entry_flops = {
-        "nmce_lmhead_ce_fused_chunk_stats": gemm_flops,
+        "nmce_lmhead_ce_fused_chunk_loss": gemm_flops,
         "nmce_lmhead_ce_fused_chunk_grads": 2 * gemm_flops,
         "nmce_lmhead_ce_fwd_stats": gemm_flops,
         "nmce_lmhead_ce_bwd": 3 * gemm_flops,
@@ -476,7 +476,7 @@ def run_fused(args, name: str, steps: int, warmup: int, one_pass: bool = True,
     flops_per_launch = entry_flops[dominant] / per_step
     achieved = flops_per_launch / (avg_ms[dominant] * 1e-3) / 1e12
     alg_flops = 3 * gemm_flops      # forward GEMM + the dX and dW GEMMs
-    on_one_pass = "nmce_lmhead_ce_fused_chunk_stats" in avg_ms
+    on_one_pass = "nmce_lmhead_ce_fused_chunk_loss" in avg_ms
     exe_flops = alg_flops if on_one_pass else 4 * gemm_flops
     vpad = (v + 255) // 256 * 256
     pt_bytes = vpad * ((min(chunk, n) + 63) // 64 * 64) * 2 if on_one_pass else None

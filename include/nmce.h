@@ -236,7 +236,17 @@ int nmce_ce_grad_rescale_unless(void* grad, int dtype, int64_t n_rows, int64_t v
                                 float* observed, void* stream);
 
 /*
- * The two calls above for rows of any width and alignment: `vocab` up to the
+ * The same for two contiguous gradients of one backward, count_a and count_b
+ * elements (multiples of 16 bytes' elements; 16-byte aligned; either may be
+ * empty), in one launch.
+ */
+int nmce_ce_grad_rescale_pair_unless(void* grad_a, int64_t count_a, void* grad_b, int64_t count_b,
+                                     int dtype, const float* grad_output, const float* assumed,
+                                     float* observed, void* stream);
+
+/*
+ * The two one-pass calls above (nmce_ce_fwd_bwd, nmce_ce_grad_rescale_unless)
+ * for rows of any width and alignment: `vocab` up to the
  * same limit, logits and grad aligned to their element. In
  * nmce_ce_fwd_bwd_ragged every grad row must share its logits row's offset
  * from a 16-byte boundary (logits - grad a multiple of 16 bytes, ld - ld_grad
@@ -437,6 +447,20 @@ int nmce_lmhead_ce_fused_chunk_stats(const void* hidden, const void* weight, int
                                      int64_t token_chunk, int64_t chunk_index, float* row_max,
                                      float* row_sumexp_m1, float* target_logit, void* workspace,
                                      int64_t workspace_bytes, void* stream);
+
+/*
+ * The same where the shard is the whole vocabulary (target ids from 0): the
+ * chunk's statistics are then the final ones, and its per-token loss is
+ * written with them, as nmce_ce_combine over one shard would. `assumed`
+ * (unless NULL) gets what nmce_hint_assume(hint, assumed) writes.
+ */
+int nmce_lmhead_ce_fused_chunk_loss(const void* hidden, const void* weight, int dtype,
+                                    int64_t n_rows, int64_t hidden_size, int64_t vocab,
+                                    const int64_t* target, int64_t token_chunk,
+                                    int64_t chunk_index, float* loss, float* g_max,
+                                    float* g_sumexp_m1, float* target_logit, const float* hint,
+                                    float* assumed, void* workspace, int64_t workspace_bytes,
+                                    void* stream);
 
 /*
  * Chunk c's gradients, given the combined statistics g_max / g_sumexp_m1 of

@@ -884,6 +884,44 @@ __global__ __launch_bounds__(kBlock) void ce_grad_rescale_kernel(
   }
 }
 
+// The same for two contiguous gradients that one backward hands out (the fused
+// head's), of vec_a and vec_b vectors: on a hit, one launch instead of two.
+template <typename T>
+__global__ __launch_bounds__(kRescaleBlock) void ce_grad_rescale_pair_kernel(
+    T* a, uint64_t vec_a, T* b, uint64_t vec_b, const float* __restrict__ gout,
+    const float* __restrict__ assumed, float* __restrict__ observed) {
+  using E = Elem<T>;
+  constexpr int EPV = E::kPerVec;
+  constexpr int kUnroll = kRescaleUnroll;
+  const float gv = gout[0];
+  if (observed && blockIdx.x == 0 && threadIdx.x == 0) observed[0] = gv;
+  const float was = assumed[0];
+  if (gv == was) return;
+  const float ratio = gv / was;
+  const uint64_t total = vec_a + vec_b;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kRescaleBlock;
+  auto at = [&](uint64_t f) {
+    return reinterpret_cast<u32x4*>(f < vec_a ? a + f * EPV : b + (f - vec_a) * EPV);
+  };
+  for (uint64_t f0 = static_cast<uint64_t>(blockIdx.x) * kRescaleBlock + threadIdx.x; f0 < total;
+       f0 += stride * kUnroll) {
+    u32x4 v[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)
+      if (f0 + u * stride < total) v[u] = load_stream(at(f0 + u * stride));
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      if (f0 + u * stride < total) {
+        float f[EPV];
+        E::unpack(v[u], f);
+#pragma unroll
+        for (int k = 0; k < EPV; ++k) f[k] *= ratio;
+        store_stream(at(f0 + u * stride), E::pack(f));
+      }
+    }
+  }
+}
+
 // The same for rows of any width and alignment (kRagged's): each stretch of
 // contiguous elements (the whole slab when ldg == V, else one row) as the
 // 16-byte-aligned body's vectors, and the elements around it one by one.
@@ -1349,6 +1387,32 @@ int nmce_ce_grad_rescale_unless(void* grad, int dtype, int64_t n_rows, int64_t v
     hipLaunchKernelGGL(ce_grad_rescale_kernel<uint16_t>, grid, block, 0, st,
                        static_cast<uint16_t*>(grad), n_rows, vocab, ld_grad, grad_output, assumed,
                        observed);
+  return launch_status();
+}
+
+int nmce_ce_grad_rescale_pair_unless(void* grad_a, int64_t count_a, void* grad_b, int64_t count_b,
+                                     int dtype, const float* grad_output, const float* assumed,
+                                     float* observed, void* stream) {
+  if (dtype != NMCE_F32 && dtype != NMCE_BF16) return NMCE_EINVAL_DTYPE;
+  const int64_t epv = dtype == NMCE_F32 ? 4 : 8;
+  if (count_a < 0 || count_b < 0 || count_a % epv || count_b % epv) return NMCE_EINVAL_SHAPE;
+  if (count_a == 0 && count_b == 0) return NMCE_OK;
+  if ((count_a && !grad_a) || (count_b && !grad_b) || !grad_output || !assumed)
+    return NMCE_EINVAL_PTR;
+  if (reinterpret_cast<uintptr_t>(grad_a) % 16 || reinterpret_cast<uintptr_t>(grad_b) % 16)
+    return NMCE_EINVAL_ALIGN;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint64_t va = static_cast<uint64_t>(count_a / epv), vb = static_cast<uint64_t>(count_b / epv);
+  const int64_t blocks = static_cast<int64_t>((va + vb + kRescaleBlock - 1) / kRescaleBlock);
+  const dim3 grid(after_one_pass_grid(blocks)), block(kRescaleBlock);
+  if (dtype == NMCE_F32)
+    hipLaunchKernelGGL(ce_grad_rescale_pair_kernel<float>, grid, block, 0, st,
+                       static_cast<float*>(grad_a), va, static_cast<float*>(grad_b), vb,
+                       grad_output, assumed, observed);
+  else
+    hipLaunchKernelGGL(ce_grad_rescale_pair_kernel<uint16_t>, grid, block, 0, st,
+                       static_cast<uint16_t*>(grad_a), va, static_cast<uint16_t*>(grad_b), vb,
+                       grad_output, assumed, observed);
   return launch_status();
 }
 

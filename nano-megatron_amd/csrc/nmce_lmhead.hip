@@ -771,13 +771,24 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_stats_kernel(
 // max, sum exp relative to it minus one, and the target logit (0 when not in
 // the shard). A workgroup takes 16 tokens; 16 slices of its threads stride
 // over the blocks with a running (max, sum - 1) each, then merge through LDS.
+// kWhole: the shard is the whole vocabulary, so the merged statistics are the
+// final ones and the loss is formed here (ce_combine_kernel's expression for
+// one shard), where a combine launch would read them back; assumed (unless
+// NULL) gets the upstream value the gradients are written for
+// (hint_assume_kernel's). Each of those launches took 5 and 2 us of a small
+// batch's 200.
 constexpr int kRedTokens = 16;
 constexpr int kRedSlices = 16;
 
+template <bool kWhole>
 __global__ __launch_bounds__(kRedTokens * kRedSlices) void lmhead_reduce_partials_kernel(
     const float* __restrict__ pmax, const float* __restrict__ psum1,
     const float* __restrict__ ptgt, int64_t nb, int64_t N, float* __restrict__ row_max,
-    float* __restrict__ row_sumexp_m1, float* __restrict__ target_logit) {
+    float* __restrict__ row_sumexp_m1, float* __restrict__ target_logit,
+    float* __restrict__ loss, const float* __restrict__ hint, float* __restrict__ assumed) {
+  if constexpr (kWhole) {
+    if (assumed && blockIdx.x == 0 && threadIdx.x == 0) assumed[0] = usable_hint(hint[0]);
+  }
   __shared__ float sm[kRedSlices][kRedTokens], ss[kRedSlices][kRedTokens],
       st[kRedSlices][kRedTokens];
   const int tl = threadIdx.x % kRedTokens;
@@ -823,6 +834,7 @@ __global__ __launch_bounds__(kRedTokens * kRedSlices) void lmhead_reduce_partial
     row_max[t] = gm;
     row_sumexp_m1[t] = gs;
     target_logit[t] = gt;
+    if constexpr (kWhole) loss[t] = log1pf(gs) - (gt - gm);
   }
 }
 
@@ -1281,14 +1293,83 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_p_kernel(
 // formed once. Rows past V and blocks past nb come out 0 (pt holds 0 there).
 // blockIdx.x walks the token tiles, so consecutive workgroups cover whole
 // rows of pt (measured 2.5% faster than walking the row blocks first).
+//
+// The grid's rows past row_blocks transpose the chunk's hidden rows for the dW
+// product (X_c [N, H] to xt [H, ldt], zero past N): work of its own that a
+// launch by itself took 5 us for at [512, 768] and 14 at [4096, 4096], nearly
+// all of it the launch.
 // ---------------------------------------------------------------------------
 constexpr int kRsRows = kPartialRows;  // 128: one block of partial statistics
 constexpr int kRsToks = 256;
+constexpr int kTrTile = 64;            // transpose tiles: 64 x 64
+
+// bf16 transpose with zero padding, the 64 x 64 tile at rows r0 and columns c0
+// of `in`: out[c * ldo + r] = in[r * ldi + c] for r < R, c < C; out[c * ldo +
+// r] = 0 for R <= r < ldo. Through LDS; interior tiles move 16 bytes per load
+// and per store (vec_ok: ldi, ldo and the base pointers 16-byte aligned), edge
+// tiles go element by element. 256 lanes.
+__device__ __forceinline__ void transpose_tile(uint16_t (*t)[kTrTile + 2],
+                                               const uint16_t* __restrict__ in, int64_t R,
+                                               int64_t C, int64_t ldi, uint16_t* __restrict__ out,
+                                               int64_t ldo, bool vec_ok, int64_t r0, int64_t c0) {
+  const int tid = threadIdx.x;
+  const bool interior = vec_ok && r0 + 64 <= R && c0 + 64 <= C && r0 + 64 <= ldo;
+  if (interior) {
+    // in: 64 rows x 8 vectors of 8 elements
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = tid / 8 + 32 * i;
+      const int cv = (tid % 8) * 8;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(in + (r0 + row) * ldi + c0 + cv);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        t[row][cv + 2 * e] = static_cast<uint16_t>(w[e] & 0xffffu);
+        t[row][cv + 2 * e + 1] = static_cast<uint16_t>(w[e] >> 16);
+      }
+    }
+    __syncthreads();
+    // out: 64 rows (c) x 8 vectors of 8 elements (r)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int col = tid / 8 + 32 * i;
+      const int rv = (tid % 8) * 8;
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[e] = static_cast<uint32_t>(t[rv + 2 * e][col]) |
+               (static_cast<uint32_t>(t[rv + 2 * e + 1][col]) << 16);
+      *reinterpret_cast<u32x4*>(out + (c0 + col) * ldo + r0 + rv) = u32x4{w[0], w[1], w[2], w[3]};
+    }
+    return;
+  }
+  const int tx = tid & 63, ty = tid >> 6;
+  for (int i = ty; i < 64; i += 4) {
+    const int64_t r = r0 + i, c = c0 + tx;
+    t[i][tx] = (r < R && c < C) ? in[r * ldi + c] : static_cast<uint16_t>(0);
+  }
+  __syncthreads();
+  for (int i = ty; i < 64; i += 4) {
+    const int64_t c = c0 + i, r = r0 + tx;
+    if (c < C && r < ldo) out[c * ldo + r] = t[tx][i];
+  }
+}
+
 __global__ __launch_bounds__(256) void lmhead_dz_rescale_kernel(
     uint16_t* __restrict__ pt, int64_t ldt, int64_t V, int64_t N, const float* __restrict__ pmax,
     int64_t nb, const float* __restrict__ gmax, const float* __restrict__ gsum1,
     const float* __restrict__ tlogit, const int64_t* __restrict__ target, int64_t vstart,
-    const float* __restrict__ gout, int64_t gstride, float gdiv) {
+    const float* __restrict__ gout, int64_t gstride, float gdiv, int row_blocks,
+    const uint16_t* __restrict__ x, int64_t H, uint16_t* __restrict__ xt) {
+  if (static_cast<int>(blockIdx.y) >= row_blocks) {
+    __shared__ uint16_t tile[kTrTile][kTrTile + 2];
+    const int64_t id = static_cast<int64_t>(blockIdx.y - row_blocks) * gridDim.x + blockIdx.x;
+    const int64_t across = (H + kTrTile - 1) / kTrTile;
+    const int64_t r0 = id / across * kTrTile;
+    if (r0 >= ldt) return;
+    transpose_tile(tile, x, N, H, H, xt, ldt, true, r0, id % across * kTrTile);
+    return;
+  }
   __shared__ float s_scale[kRsToks];
   __shared__ float s_dt[kRsToks];
   __shared__ int s_tv[kRsToks];
@@ -1384,58 +1465,15 @@ __global__ __launch_bounds__(256) void split_sum_bf16_kernel(const float* __rest
                                                        pack_bf16x2(a[2], a[3])};
 }
 
-// bf16 transpose with zero padding: out[c * ldo + r] = in[r * ldi + c] for
-// r < R, c < C; out[c * ldo + r] = 0 for R <= r < ldo. 64x64 tiles through
-// LDS; interior tiles move 16 bytes per load and per store (ldi, ldo and the
-// base pointers 16-byte aligned), edge tiles go element by element.
+// The transpose of transpose_tile by itself.
 __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __restrict__ in,
                                                              int64_t R, int64_t C, int64_t ldi,
                                                              uint16_t* __restrict__ out,
                                                              int64_t ldo, int vec_ok) {
-  __shared__ uint16_t t[64][64 + 2];
-  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64;  // over ldo (padded R)
-  const int64_t c0 = static_cast<int64_t>(blockIdx.x) * 64;
-  const int tid = threadIdx.x;
-  const bool interior = vec_ok && r0 + 64 <= R && c0 + 64 <= C && r0 + 64 <= ldo;
-  if (interior) {
-    // in: 64 rows x 8 vectors of 8 elements
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = tid / 8 + 32 * i;
-      const int cv = (tid % 8) * 8;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(in + (r0 + row) * ldi + c0 + cv);
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        t[row][cv + 2 * e] = static_cast<uint16_t>(w[e] & 0xffffu);
-        t[row][cv + 2 * e + 1] = static_cast<uint16_t>(w[e] >> 16);
-      }
-    }
-    __syncthreads();
-    // out: 64 rows (c) x 8 vectors of 8 elements (r)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int col = tid / 8 + 32 * i;
-      const int rv = (tid % 8) * 8;
-      uint32_t w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        w[e] = static_cast<uint32_t>(t[rv + 2 * e][col]) |
-               (static_cast<uint32_t>(t[rv + 2 * e + 1][col]) << 16);
-      *reinterpret_cast<u32x4*>(out + (c0 + col) * ldo + r0 + rv) = u32x4{w[0], w[1], w[2], w[3]};
-    }
-    return;
-  }
-  const int tx = tid & 63, ty = tid >> 6;
-  for (int i = ty; i < 64; i += 4) {
-    const int64_t r = r0 + i, c = c0 + tx;
-    t[i][tx] = (r < R && c < C) ? in[r * ldi + c] : static_cast<uint16_t>(0);
-  }
-  __syncthreads();
-  for (int i = ty; i < 64; i += 4) {
-    const int64_t c = c0 + i, r = r0 + tx;
-    if (c < C && r < ldo) out[c * ldo + r] = t[tx][i];
-  }
+  __shared__ uint16_t t[kTrTile][kTrTile + 2];
+  transpose_tile(t, in, R, C, ldi, out, ldo, vec_ok != 0,
+                 static_cast<int64_t>(blockIdx.y) * kTrTile,  // over ldo (padded R)
+                 static_cast<int64_t>(blockIdx.x) * kTrTile);
 }
 
 inline int launch_status() {
@@ -1712,10 +1750,10 @@ int launch_fwd_stats(const uint16_t* X, const uint16_t* W, int64_t n, int64_t H,
                      kLdsBytes, s, W, X, V, n, H, target, vstart, pmax, psum1, ptgt);
   int st = launch_status();
   if (st) return st;
-  hipLaunchKernelGGL(lmhead_reduce_partials_kernel,
+  hipLaunchKernelGGL(lmhead_reduce_partials_kernel<false>,
                      dim3(static_cast<unsigned>((n + kRedTokens - 1) / kRedTokens)),
                      dim3(kRedTokens * kRedSlices), 0, s, pmax, psum1, ptgt, nb, n, row_max,
-                     row_sumexp_m1, target_logit);
+                     row_sumexp_m1, target_logit, nullptr, nullptr, nullptr);
   return launch_status();
 }
 
@@ -2016,12 +2054,19 @@ int nmce_hint_assume(const float* hint, float* assumed, void* stream) {
   return launch_status();
 }
 
-int nmce_lmhead_ce_fused_chunk_stats(const void* hidden, const void* weight, int dtype,
-                                     int64_t n_rows, int64_t hidden_size, int64_t vocab_local,
-                                     const int64_t* target, int64_t vocab_start,
-                                     int64_t token_chunk, int64_t chunk_index, float* row_max,
-                                     float* row_sumexp_m1, float* target_logit, void* workspace,
-                                     int64_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+namespace nmce {
+namespace {
+
+// A chunk's statistics; with `loss` the shard is the whole vocabulary and
+// they are final.
+int fused_chunk_stats(const void* hidden, const void* weight, int dtype, int64_t n_rows,
+                      int64_t hidden_size, int64_t vocab_local, const int64_t* target,
+                      int64_t vocab_start, int64_t token_chunk, int64_t chunk_index, float* loss,
+                      float* row_max, float* row_sumexp_m1, float* target_logit,
+                      const float* hint, float* assumed, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
   FusedLayout L;
   int st = check_fused_args(hidden, weight, dtype, n_rows, hidden_size, vocab_local, token_chunk,
                             workspace, workspace_bytes, L);
@@ -2044,11 +2089,46 @@ int nmce_lmhead_ce_fused_chunk_stats(const void* hidden, const void* weight, int
                      vocab_start, pmax, psum1, ptgt, reinterpret_cast<uint16_t*>(ws + L.off_pt),
                      L.ldt);
   if ((st = launch_status())) return st;
-  hipLaunchKernelGGL(lmhead_reduce_partials_kernel,
-                     dim3(static_cast<unsigned>((nc + kRedTokens - 1) / kRedTokens)),
-                     dim3(kRedTokens * kRedSlices), 0, s, pmax, psum1, ptgt, L.nb, nc,
-                     row_max + t0, row_sumexp_m1 + t0, target_logit + t0);
+  const dim3 grid(static_cast<unsigned>((nc + kRedTokens - 1) / kRedTokens));
+  const dim3 block(kRedTokens * kRedSlices);
+  if (loss)
+    hipLaunchKernelGGL(lmhead_reduce_partials_kernel<true>, grid, block, 0, s, pmax, psum1, ptgt,
+                       L.nb, nc, row_max + t0, row_sumexp_m1 + t0, target_logit + t0, loss + t0,
+                       hint, assumed);
+  else
+    hipLaunchKernelGGL(lmhead_reduce_partials_kernel<false>, grid, block, 0, s, pmax, psum1, ptgt,
+                       L.nb, nc, row_max + t0, row_sumexp_m1 + t0, target_logit + t0, nullptr,
+                       nullptr, nullptr);
   return launch_status();
+}
+
+}  // namespace
+}  // namespace nmce
+
+extern "C" {
+
+int nmce_lmhead_ce_fused_chunk_stats(const void* hidden, const void* weight, int dtype,
+                                     int64_t n_rows, int64_t hidden_size, int64_t vocab_local,
+                                     const int64_t* target, int64_t vocab_start,
+                                     int64_t token_chunk, int64_t chunk_index, float* row_max,
+                                     float* row_sumexp_m1, float* target_logit, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  return fused_chunk_stats(hidden, weight, dtype, n_rows, hidden_size, vocab_local, target,
+                           vocab_start, token_chunk, chunk_index, nullptr, row_max, row_sumexp_m1,
+                           target_logit, nullptr, nullptr, workspace, workspace_bytes, stream);
+}
+
+int nmce_lmhead_ce_fused_chunk_loss(const void* hidden, const void* weight, int dtype,
+                                    int64_t n_rows, int64_t hidden_size, int64_t vocab,
+                                    const int64_t* target, int64_t token_chunk,
+                                    int64_t chunk_index, float* loss, float* g_max,
+                                    float* g_sumexp_m1, float* target_logit, const float* hint,
+                                    float* assumed, void* workspace, int64_t workspace_bytes,
+                                    void* stream) {
+  if (n_rows > 0 && (!loss || (assumed && !hint))) return NMCE_EINVAL_PTR;
+  return fused_chunk_stats(hidden, weight, dtype, n_rows, hidden_size, vocab, target, 0,
+                           token_chunk, chunk_index, loss, g_max, g_sumexp_m1, target_logit, hint,
+                           assumed, workspace, workspace_bytes, stream);
 }
 
 int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int dtype,
@@ -2078,13 +2158,23 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
   const auto* W = static_cast<const uint16_t*>(weight);
   auto* pt = reinterpret_cast<uint16_t*>(ws + L.off_pt);
   const float* pmax = reinterpret_cast<const float*>(ws + L.off_part);
-  // dZ^T of the chunk, in place of P^T.
+  // dZ^T of the chunk, in place of P^T, and X_c^T beside it (by itself where
+  // the grid has no rows left for it).
+  auto* xt = reinterpret_cast<uint16_t*>(ws + L.off_xt);
+  const int64_t across = (L.ldt + kRsToks - 1) / kRsToks;
+  const int64_t row_blocks = L.vpad / kRsRows;
+  const int64_t tr_tiles = (L.ldt / kTrTile) * ((H + kTrTile - 1) / kTrTile);
+  int64_t tr_rows = (tr_tiles + across - 1) / across;
+  if (row_blocks + tr_rows > 65535) {
+    if ((st = launch_transpose(X + t0 * H, nc, H, H, xt, L.ldt, s))) return st;
+    tr_rows = 0;
+  }
   hipLaunchKernelGGL(lmhead_dz_rescale_kernel,
-                     dim3(static_cast<unsigned>((L.ldt + kRsToks - 1) / kRsToks),
-                          static_cast<unsigned>(L.vpad / kRsRows)),
+                     dim3(static_cast<unsigned>(across),
+                          static_cast<unsigned>(row_blocks + tr_rows)),
                      dim3(256), 0, s, pt, L.ldt, V, nc, pmax, L.nb, g_max + t0, g_sumexp_m1 + t0,
                      target_logit + t0, target + t0, vocab_start, grad_output + t0 * gout_stride,
-                     gout_stride, gout_div);
+                     gout_stride, gout_div, static_cast<int>(row_blocks), X + t0 * H, H, xt);
   if ((st = launch_status())) return st;
   // dX rows of the chunk = dZ_c W: both operands read as they lie, k-row
   // (vocabulary) major: dZ^T [vpad, ldt] and W [V, H] (K = the padded
@@ -2107,7 +2197,7 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
     if ((st = launch_status())) return st;
   }
   // dW (+)= dZ_c^T X_c: A = dZ^T (K = the chunk's padded tokens contiguous),
-  // B = X_c^T [H, ldt], the chunk's hidden rows transposed first (zero past
+  // B = X_c^T [H, ldt], the chunk's hidden rows transposed above (zero past
   // the chunk's tokens), so that both operands are K-contiguous: measured
   // 0.14 ms faster per chunk of 4096 tokens at H = 4096 than reading X as it
   // lies (MN-contiguous), for a transpose of 32 MB. The same products, bit
@@ -2118,8 +2208,6 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
   else if (chunk_index == 0) mode = 1;
   else if (chunk_index + 1 < L.n_chunks) mode = 2;
   else mode = 3;
-  auto* xt = reinterpret_cast<uint16_t*>(ws + L.off_xt);
-  if ((st = launch_transpose(X + t0 * H, nc, H, H, xt, L.ldt, s))) return st;
   return launch_gemm_store(mode, pt, L.ldt, V, xt, L.ldt, H, L.ldt,
                            static_cast<uint16_t*>(grad_weight),
                            reinterpret_cast<float*>(ws + L.off_acc), H, s);

@@ -48,6 +48,7 @@ SIGNATURES: dict[str, tuple] = {
     "nmce_ce_grad_rescale_unless": (_c_int, [_p, _c_int, _i64, _i64, _i64, _p, _p, _p, _p]),
     "nmce_ce_fwd_bwd_ragged": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p,
                                         _p, _p, ctypes.c_float, _p]),
+    "nmce_ce_grad_rescale_pair_unless": (_c_int, [_p, _i64, _p, _i64, _c_int, _p, _p, _p, _p]),
     "nmce_ce_grad_rescale_unless_ragged": (_c_int, [_p, _c_int, _i64, _i64, _i64, _p, _p, _p,
                                                     _p]),
     "nmce_lmhead_ce_fwd_workspace_bytes": (_i64, [_i64, _i64, _i64]),
@@ -62,6 +63,8 @@ SIGNATURES: dict[str, tuple] = {
     "nmce_hint_assume": (_c_int, [_p, _p, _p]),
     "nmce_lmhead_ce_fused_chunk_stats": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _p, _i64,
                                                   _i64, _i64, _p, _p, _p, _p, _i64, _p]),
+    "nmce_lmhead_ce_fused_chunk_loss": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _p, _i64, _i64,
+                                                 _p, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "nmce_lmhead_ce_fused_chunk_grads": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _p, _i64,
                                                   _i64, _i64, _p, _p, _p, _p, _i64,
                                                   ctypes.c_float, _p, _p, _p, _i64, _p]),

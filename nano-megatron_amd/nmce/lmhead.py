@@ -201,8 +201,12 @@ class _LMHeadVocabParallelCrossEntropyMean(torch.autograd.Function):
         ws = _workspace(L["total"], dev)
         args = (x.data_ptr(), w.data_ptr(), _lib.NMCE_BF16, n, hp, V)
         assumed = torch.empty(1, dtype=torch.float32, device=dev)
-        _launch("nmce_hint_assume", lib.nmce_hint_assume, hint.data_ptr(), assumed.data_ptr(),
-                stream)
+        # One rank's shard from id 0 is the whole vocabulary: its statistics
+        # need no exchange and no combine.
+        whole = world_size == 1 and vocab_start == 0
+        if not whole:
+            _launch("nmce_hint_assume", lib.nmce_hint_assume, hint.data_ptr(),
+                    assumed.data_ptr(), stream)
         local = torch.empty((3, n), dtype=torch.float32, device=dev)  # max, sum - 1, target z
         out = torch.empty((3, n), dtype=torch.float32, device=dev)    # loss, max, sum - 1
         dx = torch.empty((n, hp), dtype=torch.bfloat16, device=dev)
@@ -211,18 +215,25 @@ class _LMHeadVocabParallelCrossEntropyMean(torch.autograd.Function):
         for c in range(L["n_chunks"]):
             t0 = c * step
             nc = min(step, n - t0)
-            _launch("nmce_lmhead_ce_fused_chunk_stats", lib.nmce_lmhead_ce_fused_chunk_stats,
-                    *args, tgt.data_ptr(), vocab_start, chunk, c, local[0].data_ptr(),
-                    local[1].data_ptr(), local[2].data_ptr(), ws.data_ptr(), ws.numel(), stream)
-            if world_size == 1:
-                base, stride = local.data_ptr() + 4 * t0, 3 * n
+            if whole:
+                _launch("nmce_lmhead_ce_fused_chunk_loss", lib.nmce_lmhead_ce_fused_chunk_loss,
+                        *args, tgt.data_ptr(), chunk, c, out[0].data_ptr(), out[1].data_ptr(),
+                        out[2].data_ptr(), local[2].data_ptr(), hint.data_ptr(),
+                        assumed.data_ptr() if c == 0 else None, ws.data_ptr(), ws.numel(), stream)
             else:
-                stats = _exchange_stats(local[:, t0:t0 + nc], group, world_size)
-                base, stride = stats.data_ptr(), 3 * nc
-            _launch("nmce_ce_combine", lib.nmce_ce_combine, base, base + 4 * (stride // 3),
-                    base + 8 * (stride // 3), world_size, stride, nc,
-                    out[0].data_ptr() + 4 * t0, out[1].data_ptr() + 4 * t0,
-                    out[2].data_ptr() + 4 * t0, stream)
+                _launch("nmce_lmhead_ce_fused_chunk_stats", lib.nmce_lmhead_ce_fused_chunk_stats,
+                        *args, tgt.data_ptr(), vocab_start, chunk, c, local[0].data_ptr(),
+                        local[1].data_ptr(), local[2].data_ptr(), ws.data_ptr(), ws.numel(),
+                        stream)
+                if world_size == 1:
+                    base, stride = local.data_ptr() + 4 * t0, 3 * n
+                else:
+                    stats = _exchange_stats(local[:, t0:t0 + nc], group, world_size)
+                    base, stride = stats.data_ptr(), 3 * nc
+                _launch("nmce_ce_combine", lib.nmce_ce_combine, base, base + 4 * (stride // 3),
+                        base + 8 * (stride // 3), world_size, stride, nc,
+                        out[0].data_ptr() + 4 * t0, out[1].data_ptr() + 4 * t0,
+                        out[2].data_ptr() + 4 * t0, stream)
             _launch("nmce_lmhead_ce_fused_chunk_grads", lib.nmce_lmhead_ce_fused_chunk_grads,
                     *args, tgt.data_ptr(), vocab_start, chunk, c, out[1].data_ptr(),
                     out[2].data_ptr(), local[2].data_ptr(), assumed.data_ptr(), 0, float(n),
@@ -252,12 +263,9 @@ class _LMHeadVocabParallelCrossEntropyMean(torch.autograd.Function):
                                      DEFAULT_VOCAB_CHUNK, dw)
         else:
             stream = _lib.stream_handle(x.device)
-            _launch("nmce_ce_grad_rescale_unless", lib.nmce_ce_grad_rescale_unless,
-                    dx.data_ptr(), _lib.NMCE_BF16, n, hp, hp, go.data_ptr(), assumed.data_ptr(),
-                    ctx.hint.data_ptr(), stream)
-            _launch("nmce_ce_grad_rescale_unless", lib.nmce_ce_grad_rescale_unless,
-                    dw.data_ptr(), _lib.NMCE_BF16, V, hp, hp, go.data_ptr(), assumed.data_ptr(),
-                    None, stream)
+            _launch("nmce_ce_grad_rescale_pair_unless", lib.nmce_ce_grad_rescale_pair_unless,
+                    dx.data_ptr(), n * hp, dw.data_ptr(), V * hp, _lib.NMCE_BF16, go.data_ptr(),
+                    assumed.data_ptr(), ctx.hint.data_ptr(), stream)
             ctx.handed_out = True
         H = ctx.H
         if hp != H:

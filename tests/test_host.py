@@ -128,6 +128,21 @@ def test_lmhead_argument_errors_before_launch(lib):
     # and the vocabulary is padded to 256: 8388352 rows fit, one more does not.
     assert stats(p, p, 1, 16, 64, 8388352, p, 0, 0, 0, p, p, p, p, 16, None) == -6
     assert stats(p, p, 1, 16, 64, 8388353, p, 0, 0, 0, p, p, p, p, ws, None) == -2
+    loss = lib.nmce_lmhead_ce_fused_chunk_loss
+    assert loss(p, p, 0, 16, 64, 100, p, 0, 0, p, p, p, p, p, p, p, ws, None) == -1
+    assert loss(p, p, 1, 16, 64, 100, p, 0, 1, p, p, p, p, p, p, p, ws, None) == -2
+    assert loss(p, p, 1, 16, 64, 100, p, 0, 0, None, p, p, p, p, p, p, ws, None) == -4
+    assert loss(p, p, 1, 16, 64, 100, p, 0, 0, p, p, p, p, None, p, p, ws, None) == -4  # no hint
+    assert loss(p, p, 1, 16, 64, 100, p, 0, 0, p, p, p, None, p, p, p, ws, None) == -4
+    assert loss(p, p, 1, 16, 64, 100, p, 0, 0, p, p, p, p, p, p, p, 16, None) == -6
+    pair = lib.nmce_ce_grad_rescale_pair_unless
+    assert pair(p, 8, p, 8, 5, p, p, None, None) == -1
+    assert pair(p, 12, p, 8, 1, p, p, None, None) == -2   # a part of a 16-byte vector
+    assert pair(p, 8, p, -8, 1, p, p, None, None) == -2
+    assert pair(p, 8, p + 8, 8, 1, p, p, None, None) == -3
+    assert pair(p, 8, None, 8, 1, p, p, None, None) == -4
+    assert pair(p, 8, p, 8, 1, None, p, None, None) == -4
+    assert pair(None, 0, None, 0, 1, None, None, None, None) == 0
     grads = lib.nmce_lmhead_ce_fused_chunk_grads
     assert grads(p, p, 1, 16, 64, 100, p, 0, 0, 0, p, p, p, p, 0, 0.0, p, p, p, ws,
                  None) == -2  # gout_div must be positive

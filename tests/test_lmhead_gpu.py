@@ -847,6 +847,98 @@ def test_fused_dw_product_is_bit_identical(n, chunk):
     assert dw.float().abs().sum().item() > 0
 
 
+@pytest.mark.parametrize("n,h,v,chunk", [(1, 64, 100, 0), (700, 320, 1900, 256),
+                                         (515, 64, 1001, 0)])
+def test_fused_chunk_loss_is_the_calls_it_replaces(n, h, v, chunk):
+    """nmce_lmhead_ce_fused_chunk_loss writes the bits of chunk_stats followed
+    by nmce_ce_combine over one shard and nmce_hint_assume, for every chunk
+    (one chunk, three with a short last one), and the gradients call leaves the
+    chunk's hidden rows transposed in the workspace, zero past its tokens."""
+    from nmce import _lib as L
+    from nmce import lmhead
+    lib = L.load()
+    print(f"[gpu] chunk loss n={n} h={h} v={v} chunk={chunk}", flush=True)
+    x, w, t = make_inputs(n, h, v, seed=5, w_std=0.5)
+    xd, wd, td = x.to(DEV), w.to(DEV), t.to(DEV)
+    stream = L.stream_handle(torch.device(DEV))
+    lay = lmhead._fused_layout(lib, n, h, v, chunk)
+    args = (xd.data_ptr(), wd.data_ptr(), L.NMCE_BF16, n, h, v)
+    hint = torch.full((1,), 0.0, device=DEV)  # not usable: 1.0 is assumed
+    dx = torch.empty((n, h), dtype=torch.bfloat16, device=DEV)
+    dw = torch.empty((v, h), dtype=torch.bfloat16, device=DEV)
+    results = []
+    for whole in (False, True):
+        ws = torch.zeros(lay["total"], dtype=torch.uint8, device=DEV)
+        local = torch.zeros((3, n), device=DEV)
+        out = torch.zeros((3, n), device=DEV)
+        assumed = torch.zeros(1, device=DEV)
+        if not whole:
+            L.check(lib.nmce_hint_assume(hint.data_ptr(), assumed.data_ptr(), stream), "hint")
+        for c in range(lay["n_chunks"]):
+            t0 = c * lay["chunk"]
+            nc = min(lay["chunk"], n - t0)
+            if whole:
+                L.check(lib.nmce_lmhead_ce_fused_chunk_loss(
+                    *args, td.data_ptr(), chunk, c, out[0].data_ptr(), out[1].data_ptr(),
+                    out[2].data_ptr(), local[2].data_ptr(), hint.data_ptr(),
+                    assumed.data_ptr() if c == 0 else None, ws.data_ptr(), ws.numel(), stream),
+                    "chunk loss")
+            else:
+                L.check(lib.nmce_lmhead_ce_fused_chunk_stats(
+                    *args, td.data_ptr(), 0, chunk, c, local[0].data_ptr(), local[1].data_ptr(),
+                    local[2].data_ptr(), ws.data_ptr(), ws.numel(), stream), "chunk stats")
+                base = local.data_ptr() + 4 * t0
+                L.check(lib.nmce_ce_combine(base, base + 4 * n, base + 8 * n, 1, 3 * n, nc,
+                                            out[0].data_ptr() + 4 * t0, out[1].data_ptr() + 4 * t0,
+                                            out[2].data_ptr() + 4 * t0, stream), "combine")
+            L.check(lib.nmce_lmhead_ce_fused_chunk_grads(
+                *args, td.data_ptr(), 0, chunk, c, out[1].data_ptr(), out[2].data_ptr(),
+                local[2].data_ptr(), assumed.data_ptr(), 0, float(n), dx.data_ptr(),
+                dw.data_ptr(), ws.data_ptr(), ws.numel(), stream), "chunk grads")
+            xt = ws[lay["off_xt"]:lay["off_xt"] + h * lay["ldt"] * 2].view(torch.bfloat16)
+            want = torch.zeros((h, lay["ldt"]), dtype=torch.bfloat16, device=DEV)
+            want[:, :nc] = xd[t0:t0 + nc].t()
+            assert torch.equal(xt.view(h, lay["ldt"]), want)
+        results.append((out, local[2], assumed, dx.clone(), dw.clone()))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    assert results[1][2].item() == 1.0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("na,nb", [(8, 0), (0, 4096), (8 * 777, 8 * 70001), (1 << 20, 24)])
+def test_grad_rescale_pair_is_two_rescales(dtype, na, nb):
+    """nmce_ce_grad_rescale_pair_unless leaves both gradients alone on a hit and
+    scales them as nmce_ce_grad_rescale_unless does each, bit for bit, on a
+    miss; the value it saw goes to observed either way. The larger pair is more
+    than one sweep of the grid."""
+    from nmce import _lib as L
+    lib = L.load()
+    print(f"[gpu] rescale pair {dtype} {na} {nb}", flush=True)
+    code = L.dtype_code(dtype)
+    stream = L.stream_handle(torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(na + nb)
+    a0 = torch.randn(na, device=DEV, generator=g).to(dtype)
+    b0 = torch.randn(nb, device=DEV, generator=g).to(dtype)
+    assumed = torch.full((1,), 0.7, device=DEV)
+    for value in (0.7, 1.3):
+        go = torch.full((1,), value, device=DEV)
+        seen = torch.zeros(1, device=DEV)
+        a, b = a0.clone(), b0.clone()
+        L.check(lib.nmce_ce_grad_rescale_pair_unless(
+            a.data_ptr(), na, b.data_ptr(), nb, code, go.data_ptr(), assumed.data_ptr(),
+            seen.data_ptr(), stream), "pair")
+        for got, was in ((a, a0), (b, b0)):
+            want = was.clone()
+            if want.numel():
+                L.check(lib.nmce_ce_grad_rescale_unless(
+                    want.data_ptr(), code, 1, want.numel(), want.numel(), go.data_ptr(),
+                    assumed.data_ptr(), None, stream), "one")
+            assert torch.equal(got, want)
+            assert not want.numel() or torch.equal(want, was) == (value == 0.7)
+        assert seen.item() == go.item()
+
+
 def test_one_pass_fused_follows_the_upstream_value():
     """A loss scaled by 0.25 each step: the first backward rescales the forward's
     gradients (a power-of-two ratio, so exactly) and records 0.25, after which
