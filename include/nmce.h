@@ -339,6 +339,9 @@ int64_t nmce_lmhead_ce_bwd_workspace_bytes(int64_t n_rows, int64_t hidden_size,
  *   [8] byte offset of dZ    bf16 [n_rows, chunk] of the current chunk
  *   [9] byte offset of the fp32 [n_rows, hidden_size] accumulator of
  *       nmce_lmhead_ce_bwd (present when n_chunks > 1)
+ * for the caller-driven steps below. nmce_lmhead_ce_bwd by itself arranges the
+ * same bytes as it needs them: X^T, one chunk's dZ^T and, where they fit, fp32
+ * partial sums of grad_hidden in the place of W^T, dZ and the accumulator.
  */
 #define NMCE_LMHEAD_LAYOUT_FIELDS 10
 int nmce_lmhead_ce_bwd_layout(int64_t n_rows, int64_t hidden_size, int64_t vocab_local,

@@ -15,10 +15,13 @@
 //             partial (max, sum exp, target logit); this statistics-only form
 //             stores nothing of Z.
 //   backward  per vocabulary chunk of Vc rows:
-//             dZ^T_c = recompute(W_c X^T) -> (softmax - onehot) * g, written as
-//                      bf16 in both layouts [Vc, tokens] and [tokens, Vc]
+//             dZ^T_c = recompute(W_c X^T) -> (softmax - onehot) * g, bf16 [Vc,
+//                      tokens] (and [tokens, Vc] for callers that form the
+//                      products themselves)
 //             dW_c   = dZ^T_c X      (M = Vc, N = hidden, K = tokens; B = X^T)
-//             dX    += dZ_c W_c      (M = tokens, N = hidden, K = Vc; B = W^T)
+//             dX    += dZ_c W_c      (M = tokens, N = hidden, K = Vc; both read
+//                                     vocabulary-row major, split over K when
+//                                     the tiles are few)
 //
 // The one-pass path (the drop-in's default) computes Z once, per chunk of
 // tokens (the caller's choice; the drop-in takes a quarter of the tokens):
@@ -844,8 +847,9 @@ __global__ __launch_bounds__(kRedTokens * kRedSlices) void lmhead_reduce_partial
 // (cross_entropy.py:53-65) as bf16 into dzt[v * ldt + t] and dz[t * ldz + v].
 // Rows v >= Mvalid and tokens t >= N are written as 0 (they pad the K extents
 // of the two GEMMs that follow). The tile goes through LDS so that both
-// layouts leave as coalesced 16-byte stores.
+// layouts leave as coalesced 16-byte stores. kBoth = false writes dzt only.
 // ---------------------------------------------------------------------------
+template <bool kBoth>
 __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
     const uint16_t* __restrict__ Wc, const uint16_t* __restrict__ X, int64_t Mvalid,
     int64_t Mpad, int64_t N, int64_t H, const int64_t* __restrict__ target, int64_t vfirst,
@@ -917,7 +921,7 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
   // dz [N, ldz]: 32 lanes per token row, each 8 consecutive vocabulary rows
   // (16 bytes), so one store instruction writes two 512-byte row segments.
 #pragma unroll 4
-  for (int it = 0; it < kBN * (kBM / 8) / kThreads; ++it) {
+  for (int it = 0; kBoth && it < kBN * (kBM / 8) / kThreads; ++it) {
     const int lin = it * kThreads + static_cast<int>(threadIdx.x);
     const int t = lin / (kBM / 8);
     const int L = lin % (kBM / 8);  // vocabulary rows 8L .. 8L+7, pairs 4L .. 4L+3
@@ -1491,7 +1495,8 @@ int configure_lds() {
   if (lds_configured) return NMCE_OK;
   const void* kernels[] = {
       reinterpret_cast<const void*>(&lmhead_stats_kernel),
-      reinterpret_cast<const void*>(&lmhead_dz_kernel),
+      reinterpret_cast<const void*>(&lmhead_dz_kernel<true>),
+      reinterpret_cast<const void*>(&lmhead_dz_kernel<false>),
       reinterpret_cast<const void*>(&lmhead_p_kernel),
   };
   for (const void* k : kernels) {
@@ -1614,6 +1619,16 @@ BwdLayout bwd_layout(int64_t n, int64_t h, int64_t v, int64_t chunk) {
   return L;
 }
 
+// The carve-up of the same bytes by a backward whose dX product reads dZ^T and
+// the weight as they lie (bwd_direct): X^T stays where BwdLayout has it, dZ^T of
+// one chunk follows, and what W^T, dZ and the accumulator would take holds fp32
+// partials of dX, [n, h] each, one per K range of every chunk.
+struct DirectLayout {
+  int64_t off_dzt, off_part;
+  int64_t splits;  // K ranges of a chunk's dX product; 0: the partials do not fit
+  int64_t ks;      // their length
+};
+
 int64_t fwd_partial_blocks(int64_t v) { return (v + kPartialRows - 1) / kPartialRows; }
 
 // Compute units of the current device (256 if the query fails).
@@ -1686,6 +1701,25 @@ int choose_splits(int64_t tiles, int64_t out, int64_t K, int64_t k_valid, int cu
   }
   *ks = best == 1 ? K : round_up((K + best - 1) / best, kBK);
   return best;
+}
+
+// The K ranges are choose_splits' for a whole chunk, and no more than fit. One
+// range a chunk is enough to run (the chunks' partials take the accumulator's
+// place); where even that does not fit (many tokens in many small chunks), the
+// accumulating products on W^T remain.
+DirectLayout direct_layout(const BwdLayout& L, int64_t n, int64_t h, int cus) {
+  DirectLayout D{};
+  D.off_dzt = L.off_wt;
+  D.off_part = D.off_dzt + align256(L.chunk * L.ldt * 2);
+  const int64_t fit = (L.total - D.off_part) / (n * h * 4) / L.n_chunks;
+  if (fit < 1) return D;
+  const int64_t tiles = ((n + kBM - 1) / kBM) * ((h + kBN - 1) / kBN);
+  D.splits = choose_splits(tiles, n * h, L.chunk, L.chunk, cus, &D.ks);
+  if (D.splits > fit) {
+    D.splits = fit;
+    D.ks = round_up((L.chunk + fit - 1) / fit, kBK);
+  }
+  return D;
 }
 
 // Workspace of the one-pass fused loss (all offsets 256-byte aligned).
@@ -1886,16 +1920,64 @@ int bwd_prepare(const uint16_t* X, const uint16_t* W, int64_t n_rows, int64_t H,
 int bwd_dz(const uint16_t* X, const uint16_t* W, int64_t n_rows, int64_t H, int64_t V,
            const int64_t* target, int64_t vocab_start, const float* g_max,
            const float* g_sumexp_m1, const float* grad_output, int64_t gout_stride, int64_t c,
-           const BwdLayout& L, char* ws, hipStream_t s) {
+           const BwdLayout& L, uint16_t* dzt, uint16_t* dz, hipStream_t s) {
   const int64_t v0 = c * L.chunk;
   const int64_t mvalid = (V - v0) < L.chunk ? (V - v0) : L.chunk;
   const int64_t mpad = round_up(mvalid, kBM);
   const int64_t tiles = (mpad / kBM) * ((L.ldt + kBN - 1) / kBN);
-  hipLaunchKernelGGL(lmhead_dz_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads),
+  hipLaunchKernelGGL(dz ? lmhead_dz_kernel<true> : lmhead_dz_kernel<false>,
+                     dim3(static_cast<unsigned>(tiles)), dim3(kThreads),
                      kLdsBytes, s, W + v0 * H, X, mvalid, mpad, n_rows, H, target,
-                     vocab_start + v0, g_max, g_sumexp_m1, grad_output, gout_stride,
-                     reinterpret_cast<uint16_t*>(ws + L.off_dzt), L.ldt,
-                     reinterpret_cast<uint16_t*>(ws + L.off_dz), L.chunk);
+                     vocab_start + v0, g_max, g_sumexp_m1, grad_output, gout_stride, dzt, L.ldt,
+                     dz, L.chunk);
+  return launch_status();
+}
+
+// The backward's products with nothing transposed but X: dX = dZ W of each
+// chunk reads dZ^T and W vocabulary-row major, as they lie, in K ranges where
+// its tiles leave compute units idle, and the ranges' partials of all chunks
+// are summed at the end. Against both layouts of dZ, a W^T and an fp32
+// accumulator (BwdLayout), in the same workspace: no transpose of the weight
+// and half of dZ's stores, and the few tiles of a small batch no longer walk
+// the whole chunk serially. Forward and backward: [64, 1024] x
+// [50304, 1024] 994 -> 257 us, [660, 1536] x [151936, 1536] 3.83 -> 1.44 ms,
+// [2048, 2048] x [32000, 2048] 1.26 -> 0.86, [4564, 3456] x [64128, 3456] 6.06
+// -> 5.82, [12288, 4096] x [128256, 4096] 35.9 -> 35.0.
+int bwd_direct(const uint16_t* X, const uint16_t* W, int64_t n_rows, int64_t H, int64_t V,
+               const int64_t* target, int64_t vocab_start, const float* g_max,
+               const float* g_sumexp_m1, const float* grad_output, int64_t gout_stride,
+               const BwdLayout& L, const DirectLayout& D, char* ws, uint16_t* dX, uint16_t* dW,
+               hipStream_t s) {
+  auto* xt = reinterpret_cast<uint16_t*>(ws + L.off_xt);
+  auto* dzt = reinterpret_cast<uint16_t*>(ws + D.off_dzt);
+  auto* part = reinterpret_cast<float*>(ws + D.off_part);
+  int st = launch_transpose(X, n_rows, H, H, xt, L.ldt, s);
+  if (st) return st;
+  int parts = 0;
+  for (int64_t c = 0; c < L.n_chunks; ++c) {
+    const int64_t v0 = c * L.chunk;
+    const int64_t mvalid = (V - v0) < L.chunk ? (V - v0) : L.chunk;
+    const int64_t mpad = round_up(mvalid, kBM);
+    if ((st = bwd_dz(X, W, n_rows, H, V, target, vocab_start, g_max, g_sumexp_m1, grad_output,
+                     gout_stride, c, L, dzt, nullptr, s)))
+      return st;
+    if ((st = launch_gemm_store(0, dzt, L.ldt, mvalid, xt, L.ldt, H, L.ldt, dW + v0 * H, nullptr,
+                                H, s)))
+      return st;
+    if (L.n_chunks == 1 && D.splits == 1)
+      return launch_gemm_store(0, dzt, L.ldt, n_rows, W, H, H, mpad, dX, nullptr, H, s, true, true,
+                               mpad, mvalid);
+    // Ranges that begin inside the shard; a last chunk may have fewer.
+    const int ranges = D.splits == 1 ? 1 : static_cast<int>((mvalid + D.ks - 1) / D.ks);
+    if ((st = launch_gemm_store(1, dzt, L.ldt, n_rows, W + v0 * H, H, H, mpad, nullptr,
+                                part + parts * n_rows * H, H, s, true, true, mpad, mvalid, ranges,
+                                D.ks, n_rows * H)))
+      return st;
+    parts += ranges;
+  }
+  const int64_t quads = n_rows * H / 4;
+  hipLaunchKernelGGL(split_sum_bf16_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)),
+                     dim3(256), 0, s, part, parts, n_rows, H, dX, H);
   return launch_status();
 }
 
@@ -1941,10 +2023,11 @@ int nmce_lmhead_ce_bwd_dz(const void* hidden, const void* weight, int dtype, int
   if (!target || !g_max || !g_sumexp_m1 || !grad_output) return NMCE_EINVAL_PTR;
   if (gout_stride < 0 || chunk_index < 0 || chunk_index >= L.n_chunks) return NMCE_EINVAL_SHAPE;
   if ((st = configure_lds())) return st;
+  char* ws = static_cast<char*>(workspace);
   return bwd_dz(static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(weight), n_rows,
                 hidden_size, vocab_local, target, vocab_start, g_max, g_sumexp_m1, grad_output,
-                gout_stride, chunk_index, L, static_cast<char*>(workspace),
-                static_cast<hipStream_t>(stream));
+                gout_stride, chunk_index, L, reinterpret_cast<uint16_t*>(ws + L.off_dzt),
+                reinterpret_cast<uint16_t*>(ws + L.off_dz), static_cast<hipStream_t>(stream));
 }
 
 int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_t n_rows,
@@ -1966,8 +2049,8 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
   char* ws = static_cast<char*>(workspace);
   const uint16_t* xt = reinterpret_cast<const uint16_t*>(ws + L.off_xt);
   const uint16_t* wt = reinterpret_cast<const uint16_t*>(ws + L.off_wt);
-  const uint16_t* dzt = reinterpret_cast<const uint16_t*>(ws + L.off_dzt);
-  const uint16_t* dz = reinterpret_cast<const uint16_t*>(ws + L.off_dz);
+  uint16_t* dzt = reinterpret_cast<uint16_t*>(ws + L.off_dzt);
+  uint16_t* dz = reinterpret_cast<uint16_t*>(ws + L.off_dz);
   float* acc = reinterpret_cast<float*>(ws + L.off_acc);
   const auto* X = static_cast<const uint16_t*>(hidden);
   const auto* W = static_cast<const uint16_t*>(weight);
@@ -1975,6 +2058,10 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
   auto* dW = static_cast<uint16_t*>(grad_weight);
   const int64_t H = hidden_size;
 
+  const DirectLayout D = direct_layout(L, n_rows, H, device_cus());
+  if (D.splits > 0)
+    return bwd_direct(X, W, n_rows, H, vocab_local, target, vocab_start, g_max, g_sumexp_m1,
+                      grad_output, gout_stride, L, D, ws, dX, dW, s);
   if ((st = bwd_prepare(X, W, n_rows, H, vocab_local, L, ws, s))) return st;
   for (int64_t c = 0; c < L.n_chunks; ++c) {
     const int64_t v0 = c * L.chunk;
@@ -1982,7 +2069,7 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
     const int64_t mpad = round_up(mvalid, kBM);
     // dZ of this chunk, both layouts.
     if ((st = bwd_dz(X, W, n_rows, H, vocab_local, target, vocab_start, g_max, g_sumexp_m1,
-                     grad_output, gout_stride, c, L, ws, s)))
+                     grad_output, gout_stride, c, L, dzt, dz, s)))
       return st;
     // dW rows [v0, v0 + mvalid) = dZ^T_c X  (K = tokens, padded with zeros).
     if ((st = launch_gemm_store(0, dzt, L.ldt, mvalid, xt, L.ldt, H, L.ldt, dW + v0 * H, nullptr, H,

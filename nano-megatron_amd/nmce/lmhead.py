@@ -15,8 +15,8 @@ respect to ``x`` and ``W`` are those of the two-step reference, but the
 ``[tokens, V/tp]`` logits are never stored: the one-pass path holds the
 bf16 exponentials of one chunk of tokens at a time (by default at most 2 GiB,
 and at most a quarter of the tokens unless every token at once takes no more
-memory), the recomputing path two bf16 copies of one vocabulary chunk's logit
-gradient.
+memory), the recomputing path one vocabulary chunk's logit gradient (its
+workspace has room for two bf16 copies of it).
 
 When a gradient is wanted (grad mode on, ``x`` or ``W`` requiring grad) the
 wrapper takes the one-pass path: the forward goes through the tokens in
@@ -58,9 +58,9 @@ from .mappings import (
 )
 from .parallel import divide
 
-# Default vocabulary rows per chunk of the recomputing backward: the chunk's
-# logit gradient is held twice in bf16 (4 * tokens * chunk bytes), so no
-# tensor the size of the full logits ever exists. A chunk covering the whole
+# Default vocabulary rows per chunk of the recomputing backward: its workspace
+# has room for the chunk's logit gradient twice in bf16 (4 * tokens * chunk
+# bytes), so no tensor the size of the full logits ever exists. A chunk covering the whole
 # shard needs no fp32 accumulation of dX, at the price of a full-size dZ.
 DEFAULT_VOCAB_CHUNK = 32768
 

@@ -284,6 +284,23 @@ def test_fused_chunked_backward_matches(chunk):
     check_grad(dx1, rdx, "dH one chunk")
 
 
+@pytest.mark.parametrize("n,h,v,chunk", [(77, 64, 9000, 4096), (300, 192, 20000, None),
+                                         (1, 64, 2305, 1024), (515, 320, 5001, 2048),
+                                         (1000, 64, 3000, 256)])
+def test_fused_backward_k_ranges(n, h, v, chunk):
+    """The recomputing backward's dX = dZ W with dZ^T and W read as they lie: a
+    chunk's vocabulary rows in several K ranges, a last chunk with fewer of
+    them that ends in padding, one chunk of many ranges, chunks of one range
+    each whose partials fill the workspace, and chunks too many for it (the
+    accumulating products on W^T), against the fp64 closed form."""
+    print(f"[gpu] backward K ranges n={n} h={h} v={v} chunk={chunk}", flush=True)
+    x, w, t = make_inputs(n, h, v, seed=n + v, w_std=0.5)
+    _, dx, dw = run_fused(x, w, t, vchunk=chunk)
+    _, _, rdx, rdw = fp64_reference(x, w, t)
+    check_grad(dx, rdx, f"dH chunk {chunk}")
+    check_grad(dw, rdw, f"dW chunk {chunk}")
+
+
 def test_bwd_dz_buffers():
     """The recomputed logit gradient itself, read back from the workspace after
     ``nmce_lmhead_ce_bwd_dz`` for both chunks of a ragged shard (300 tokens,
