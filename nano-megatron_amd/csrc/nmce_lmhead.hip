@@ -137,13 +137,12 @@ __device__ __forceinline__ void mfma_16x16x32(f32x4_t& c, const bf16x8_t& a, con
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 
-// Tile index for this workgroup. The dispatcher deals workgroups to the 8 XCDs
+// Tile index for workgroup b. The dispatcher deals workgroups to the 8 XCDs
 // round-robin (block b runs on XCD b % 8); give each XCD a contiguous band of
 // tile ids, and inside the band walk groups of kGroupM tile rows column by
 // column, so the tiles that run together on one L2 share A and B stripes.
-__device__ __forceinline__ void tile_coords(int tiles_m, int tiles_n, int& tm, int& tn) {
+__device__ __forceinline__ void tile_coords(int b, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int total = tiles_m * tiles_n;
-  const int b = blockIdx.x;
   const int xcd = b % kXcds;
   const int q = total / kXcds, r = total % kXcds;
   const int tid = xcd * q + (xcd < r ? xcd : r) + b / kXcds;
@@ -756,7 +755,7 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_stats_kernel(
   const int tiles_m = static_cast<int>((V + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(tiles_m, tiles_n, tm, tn);
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
   gemm_mainloop<false, false>(W, H, V, X, H, N, H, m0, n0, lds, acc);
@@ -860,7 +859,7 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
   const int tiles_m = static_cast<int>(Mpad / kBM);
   const int tiles_n = static_cast<int>((ldt + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(tiles_m, tiles_n, tm, tn);
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
   gemm_mainloop<false, false>(Wc, H, Mvalid, X, H, N, H, m0, n0, lds, acc);
@@ -1193,17 +1192,16 @@ __device__ __forceinline__ void store_bf16_tile(const Acc& acc, char* lds,
 // kVec (modes 1-3): the output meets store_f32_tile's conditions for 16-byte
 // accesses (the host checks them); otherwise it leaves element by element.
 // ---------------------------------------------------------------------------
-template <int kMode, bool kAMN = false, bool kBMN = false, bool kVec = true>
-__global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
-    const uint16_t* __restrict__ A, int64_t lda, int64_t M, const uint16_t* __restrict__ B,
-    int64_t ldb, int64_t N, int64_t K, uint16_t* __restrict__ C, float* __restrict__ Cf,
-    int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits, int64_t ks,
+template <int kMode, bool kAMN, bool kBMN, bool kVec>
+__device__ __forceinline__ void gemm_store_tile(
+    int block, char* lds, const uint16_t* __restrict__ A, int64_t lda, int64_t M,
+    const uint16_t* __restrict__ B, int64_t ldb, int64_t N, int64_t K, uint16_t* __restrict__ C,
+    float* __restrict__ Cf, int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits, int64_t ks,
     int64_t split_stride) {
-  extern __shared__ __align__(16) char lds[];
   const int tiles_m = static_cast<int>((M + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tmv, tn;
-  tile_coords(tiles_m * splits, tiles_n, tmv, tn);
+  tile_coords(block, tiles_m * splits, tiles_n, tmv, tn);
   const int split = tmv / tiles_m;
   const int tm = tmv - split * tiles_m;
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
@@ -1230,6 +1228,53 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
     store_bf16_tile(acc, lds, C, ldc, M, N, m0, n0);
 }
 
+template <int kMode, bool kAMN = false, bool kBMN = false, bool kVec = true>
+__global__ __launch_bounds__(kThreads, 1) void gemm_store_kernel(
+    const uint16_t* __restrict__ A, int64_t lda, int64_t M, const uint16_t* __restrict__ B,
+    int64_t ldb, int64_t N, int64_t K, uint16_t* __restrict__ C, float* __restrict__ Cf,
+    int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits, int64_t ks,
+    int64_t split_stride) {
+  extern __shared__ __align__(16) char lds[];
+  gemm_store_tile<kMode, kAMN, kBMN, kVec>(blockIdx.x, lds, A, lda, M, B, ldb, N, K, C, Cf, ldc,
+                                           ka_rows, kb_rows, splits, ks, split_stride);
+}
+
+// One chunk's two backward products in one grid: dX = dZ W (kSplit: K ranges'
+// fp32 partials; else bf16) by the first x_blocks workgroups, then dW = dZ^T X
+// in bf16. dX's tiles are few and long, dW's many and short, so dW's fill the
+// compute units that dX's one round leaves idle or frees early, and one last
+// round is left partly empty instead of two. Steps: [512, 768] x [50304, 768]
+// 225 -> 204 us, [135, 960] x [111313, 960] 269 -> 256, [1548, 3904] x [256000,
+// 3904] 8.23 -> 8.06 ms; where dW alone has tens of rounds there is no
+// difference ([4096, 4096] x [128256, 4096] 9.48 ms either way). Chunks that
+// accumulate dW in fp32 keep two launches: their dW is long, and its epilogue
+// another.
+struct PairArgs {
+  const uint16_t* dzt;  // [vpad, ldt]
+  int64_t ldt, vpad;
+  const uint16_t* W;    // [V, H]
+  int64_t V, H;
+  const uint16_t* xt;   // [H, ldt]
+  int64_t n;            // tokens
+  uint16_t* dx;         // [n, H]
+  float* part;          // [splits][n][H]
+  uint16_t* dw;         // [V, H]
+  int64_t ks;
+  int splits, x_blocks;
+};
+template <bool kSplit>
+__global__ __launch_bounds__(kThreads, 1) void gemm_pair_kernel(PairArgs p) {
+  extern __shared__ __align__(16) char lds[];
+  const int b = blockIdx.x;
+  if (b < p.x_blocks)
+    gemm_store_tile<kSplit ? 1 : 0, true, true, true>(b, lds, p.dzt, p.ldt, p.n, p.W, p.H, p.H,
+                                                      p.vpad, p.dx, p.part, p.H, p.vpad, p.V,
+                                                      p.splits, p.ks, p.n * p.H);
+  else
+    gemm_store_tile<0, false, false, true>(b - p.x_blocks, lds, p.dzt, p.ldt, p.V, p.xt, p.ldt,
+                                           p.H, p.ldt, p.dw, nullptr, p.H, 0, 0, 1, p.ldt, 0);
+}
+
 // ---------------------------------------------------------------------------
 // One-pass fused loss, step 1 (per chunk of tokens): the statistics GEMM of
 // lmhead_stats_kernel whose epilogue also keeps the exponentials it forms,
@@ -1249,7 +1294,7 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_p_kernel(
   const int tiles_m = static_cast<int>((V + kBM - 1) / kBM);
   const int tiles_n = static_cast<int>((N + kBN - 1) / kBN);
   int tm, tn;
-  tile_coords(tiles_m, tiles_n, tm, tn);
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
   Acc acc;
   gemm_mainloop<false, false>(W, H, V, X, H, N, H, m0, n0, lds, acc);
@@ -1582,6 +1627,34 @@ int launch_gemm_store(int mode, const uint16_t* A, int64_t lda, int64_t M, const
   return launch_status();
 }
 
+// Both products write 16-byte vectors at 32-bit offsets (launch_gemm_store's
+// `vec`, for row strides of H, a multiple of 64).
+inline bool pair_ok(int64_t h) { return h * 4 * 512 < (int64_t{1} << 32); }
+
+template <bool kSplit>
+int launch_pair_as(const PairArgs& p, int64_t blocks, hipStream_t s) {
+  static bool lds_set = false;  // the attribute is set once per process and kernel
+  if (!lds_set) {
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<kSplit>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    if (e != hipSuccess) return static_cast<int>(e);
+    lds_set = true;
+  }
+  hipLaunchKernelGGL(gemm_pair_kernel<kSplit>, dim3(static_cast<unsigned>(blocks)),
+                     dim3(kThreads), kLdsBytes, s, p);
+  return launch_status();
+}
+
+// Fills in x_blocks.
+int launch_pair(PairArgs p, bool split, hipStream_t s) {
+  const int64_t h_tiles = (p.H + kBN - 1) / kBN;
+  const int64_t x_blocks = ((p.n + kBM - 1) / kBM) * h_tiles * p.splits;
+  p.x_blocks = static_cast<int>(x_blocks);
+  const int64_t blocks = x_blocks + ((p.V + kBM - 1) / kBM) * h_tiles;
+  return split ? launch_pair_as<true>(p, blocks, s) : launch_pair_as<false>(p, blocks, s);
+}
+
 int launch_transpose(const uint16_t* in, int64_t R, int64_t C, int64_t ldi, uint16_t* out,
                      int64_t ldo, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((C + 63) / 64), static_cast<unsigned>((ldo + 63) / 64));
@@ -1712,7 +1785,7 @@ DirectLayout direct_layout(const BwdLayout& L, int64_t n, int64_t h, int cus) {
   D.off_dzt = L.off_wt;
   D.off_part = D.off_dzt + align256(L.chunk * L.ldt * 2);
   const int64_t fit = (L.total - D.off_part) / (n * h * 4) / L.n_chunks;
-  if (fit < 1) return D;
+  if (fit < 1 || !pair_ok(h)) return D;
   const int64_t tiles = ((n + kBM - 1) / kBM) * ((h + kBN - 1) / kBN);
   D.splits = choose_splits(tiles, n * h, L.chunk, L.chunk, cus, &D.ks);
   if (D.splits > fit) {
@@ -1961,18 +2034,12 @@ int bwd_direct(const uint16_t* X, const uint16_t* W, int64_t n_rows, int64_t H, 
     if ((st = bwd_dz(X, W, n_rows, H, V, target, vocab_start, g_max, g_sumexp_m1, grad_output,
                      gout_stride, c, L, dzt, nullptr, s)))
       return st;
-    if ((st = launch_gemm_store(0, dzt, L.ldt, mvalid, xt, L.ldt, H, L.ldt, dW + v0 * H, nullptr,
-                                H, s)))
-      return st;
-    if (L.n_chunks == 1 && D.splits == 1)
-      return launch_gemm_store(0, dzt, L.ldt, n_rows, W, H, H, mpad, dX, nullptr, H, s, true, true,
-                               mpad, mvalid);
     // Ranges that begin inside the shard; a last chunk may have fewer.
     const int ranges = D.splits == 1 ? 1 : static_cast<int>((mvalid + D.ks - 1) / D.ks);
-    if ((st = launch_gemm_store(1, dzt, L.ldt, n_rows, W + v0 * H, H, H, mpad, nullptr,
-                                part + parts * n_rows * H, H, s, true, true, mpad, mvalid, ranges,
-                                D.ks, n_rows * H)))
-      return st;
+    const bool split = L.n_chunks > 1 || D.splits > 1;
+    const PairArgs p{dzt, L.ldt, mpad, W + v0 * H, mvalid, H, xt, n_rows, dX,
+                     part + parts * n_rows * H, dW + v0 * H, ranges == 1 ? mpad : D.ks, ranges, 0};
+    if ((st = launch_pair(p, split, s)) || !split) return st;
     parts += ranges;
   }
   const int64_t quads = n_rows * H / 4;
@@ -2268,6 +2335,17 @@ int nmce_lmhead_ce_fused_chunk_grads(const void* hidden, const void* weight, int
   // vocabulary; dZ^T is zero past V, so W's k-rows stop at V). A chunk with
   // too few tiles to fill the device splits K and sums the fp32 partials.
   uint16_t* dx_rows = static_cast<uint16_t*>(grad_hidden) + t0 * H;
+  if (L.n_chunks == 1 && pair_ok(H)) {
+    const PairArgs p{pt, L.ldt, L.vpad, W, V, H, xt, nc, dx_rows,
+                     reinterpret_cast<float*>(ws + L.off_dxp),
+                     static_cast<uint16_t*>(grad_weight),
+                     L.dx_splits == 1 ? L.vpad : L.dx_ks, static_cast<int>(L.dx_splits), 0};
+    if ((st = launch_pair(p, L.dx_splits > 1, s)) || L.dx_splits == 1) return st;
+    const int64_t quads = nc * H / 4;
+    hipLaunchKernelGGL(split_sum_bf16_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)),
+                       dim3(256), 0, s, p.part, p.splits, nc, H, dx_rows, H);
+    return launch_status();
+  }
   if (L.dx_splits == 1) {
     if ((st = launch_gemm_store(0, pt, L.ldt, nc, W, H, H, L.vpad, dx_rows, nullptr, H, s,
                                 true, true, L.vpad, V)))
