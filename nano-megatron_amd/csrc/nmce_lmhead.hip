@@ -7,7 +7,7 @@
 // vocabulary chunk's gradient, at a time.
 //
 // Every product is one bf16 GEMM core, C[m, n] = sum_k A[m, k] * B[n, k] on
-// v_mfma_f32_32x32x16_bf16, each operand K-contiguous or MN-contiguous
+// v_mfma_f32_16x16x32_bf16, each operand K-contiguous or MN-contiguous
 // (gemm_mainloop):
 //
 //   forward   Z^T = W X^T    (M = vocab, N = tokens, K = hidden). The epilogue
@@ -133,6 +133,10 @@ struct Acc {
 // back (360 moves per K step, 1055-1200 instead of 1440 TFLOP/s). The 16 x 16
 // form moves half the accumulator bytes per product that the 32 x 32 x 16 form
 // does, with the same sums: 1440 against 1240 TFLOP/s in the same loop.
+// The compiler puts no wait states around an instruction that it does not know
+// for an MFMA: its fragments come from LDS reads, whose waits it counts, and
+// nothing else touches the accumulators within the loop (gemm_mainloop waits
+// before the first and after the last; a test looks at the generated code).
 __device__ __forceinline__ void mfma_16x16x32(f32x4_t& c, const bf16x8_t& a, const bf16x8_t& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }

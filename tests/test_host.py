@@ -449,6 +449,60 @@ def test_one_pass_ragged_route(lib):
     assert rs(p, 1, 4, 9, 9, None, p, None, None) == -4
 
 
+def test_gemm_mfmas_keep_their_wait_states(tmp_path):
+    """The GEMM core's MFMAs are inline asm, around which the compiler puts no
+    wait states. In the generated code no VALU instruction writes a source of
+    an MFMA within two wait states before it, and none touches the registers
+    that one wrote within 16 wait states after it."""
+    import re
+    import subprocess
+
+    from nmce import _build
+    asm = tmp_path / "lmhead.s"
+    subprocess.run([_build.hipcc(), *_build.HIPCC_FLAGS, "-S", "--cuda-device-only",
+                    str(_build.CSRC_DIR / "nmce_lmhead.hip"), "-o", str(asm)], check=True,
+                   capture_output=True)
+
+    def regs(token):
+        m = re.match(r"([va])(?:\[(\d+):(\d+)\]|(\d+))$", token)
+        if not m:
+            return set()
+        lo, hi = (m[2], m[3]) if m[2] else (m[4], m[4])
+        return {(m[1], i) for i in range(int(lo), int(hi) + 1)}
+
+    recent = []   # (wait states, VALU destination) of the last instructions
+    pending = []  # (registers an MFMA writes, wait states since it)
+    mfmas = 0
+    for line in asm.read_text().splitlines():
+        if re.match(r"_Z\w+:", line):
+            recent, pending = [], []
+        op, _, rest = line.split(";")[0].strip().partition(" ")
+        if not op or op.startswith(".") or op.endswith(":"):
+            continue
+        tokens = [t.strip() for t in re.split(r",(?![^\[]*\])", rest)]
+        states = int(tokens[0]) + 1 if op == "s_nop" else 1
+        if op.startswith("v_mfma"):
+            mfmas += 1
+            sources = set().union(*map(regs, tokens[1:4]))
+            waited = 0
+            for n, written in reversed(recent):
+                if waited >= 2:
+                    break
+                assert not written & sources, line
+                waited += n
+            recent.append((1, set()))
+        else:
+            used = set().union(*map(regs, tokens))
+            for written, _ in pending:
+                assert not written & used, line
+            recent.append((states, regs(tokens[0]) if op.startswith("v_") else set()))
+        recent = recent[-3:]
+        pending = [(w, n + states) for w, n in pending if n + states < 16]
+        if op.startswith("v_mfma"):
+            pending.append((regs(tokens[0]), 0))
+    assert mfmas > 1000
+
+
 def test_wide_buffer_stores_go_through_the_helper():
     """Buffer stores wider than 8 bytes are issued only by buffer_store_b128,
     which keeps the scalar offset the constant 0: with a register scalar
