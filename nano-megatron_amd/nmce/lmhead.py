@@ -71,9 +71,8 @@ DEFAULT_VOCAB_CHUNK = 32768
 # tiles; every token only when there are at most 256) and at most
 # CHUNK_BUDGET_BYTES, so nothing the size of the [tokens, V] logits is
 # allocated. dW is then accumulated in fp32 across the chunks by the GEMM
-# epilogue (measured on one MI355X: [16384, 4096] x [128256, 4096] 3.4% slower
-# in four chunks of 4096 tokens than in one chunk, [16384, 3072] x
-# [256000, 3072] 1.6%). The accumulator is 4 V H bytes whatever the tokens, so
+# epilogue (measured on one MI355X: [16384, 4096] x [128256, 4096] 38.55 ms in
+# four chunks of 4096 tokens, 36.97 in one). The accumulator is 4 V H bytes whatever the tokens, so
 # with few tokens per unit of H it outgrows every token's exponentials: then
 # one chunk, which needs no accumulator, is the smaller workspace and the
 # faster pass (one_pass_token_chunk).
@@ -103,8 +102,9 @@ def one_pass_token_chunk(n_tokens: int, hidden: int, vocab_local: int) -> int:
     line everywhere, since each further chunk reads and writes the accumulator
     and shortens dW's K to the chunk ([4096, 4096] x [128256, 4096]: 12.9 ms
     in four chunks, 10.7 in one; [2103, 1600] x [50257, 1600]: 1.60 ms in
-    three, 1.13 in one; [512, 768] x [50304, 768]: 0.54 in two, 0.32 in one). The line depends on sizes alone, so every tensor-parallel rank
-    takes the same chunks."""
+    three, 1.13 in one; [512, 768] x [50304, 768]: 0.54 in two, 0.32 in one).
+    The line depends on sizes alone, so every tensor-parallel rank takes the
+    same chunks."""
     chunk = default_token_chunk(n_tokens, vocab_local)
     more = (n_tokens - chunk) * (2 * vocab_local + 12 * -(-vocab_local // 128) + 2 * hidden)
     if more <= 4 * vocab_local * hidden and 2 * vocab_local * n_tokens <= CHUNK_BUDGET_BYTES:
