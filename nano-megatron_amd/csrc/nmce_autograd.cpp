@@ -334,7 +334,15 @@ at::Tensor unread_word(const at::Tensor& like) {
 // is over) and the slot back; so does the end of its life.
 class TargetCheck {
  public:
+  // Any tensor may come here (validate_targets is public): the kernel reads it
+  // at its device address, as int64 and without strides.
   TargetCheck(const at::Tensor& target, int64_t vocab_total) {
+    TORCH_CHECK_VALUE(target.is_cuda(), "nmce: targets must be on a ROCm device, got ",
+                      target.device());
+    TORCH_CHECK_TYPE(target.scalar_type() == at::kLong, "nmce: target must be int64, got ",
+                     target.scalar_type());
+    TORCH_CHECK_VALUE(target.is_contiguous() && target.numel() > 0,
+                      "nmce: the target check takes a non-empty contiguous tensor");
     const c10::DeviceGuard device_guard(target.device());
     hipStream_t st = stream_of(target);
     guard_ = launch_check(target, vocab_total, unread_word(target), st);

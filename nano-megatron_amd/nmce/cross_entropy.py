@@ -181,11 +181,15 @@ def launch_target_check(target: torch.Tensor, vocab_size: int) -> _PendingCheck 
     fused loss of a few hundred tokens takes, where the check itself takes the
     loss stream 2-4 us.
     """
+    if target.numel() == 0:
+        return None
+    if not target.is_cuda:
+        raise ValueError(f"nmce: targets must be on a ROCm device, got {target.device}")
+    if target.dtype != torch.int64:
+        raise TypeError(f"nmce: target must be int64, got {target.dtype}")
     t = target.reshape(-1)
     if not t.is_contiguous():
         t = t.contiguous()
-    if t.numel() == 0:
-        return None
     return _PendingCheck(_lib.autograd_ext().TargetCheck(t, vocab_size))
 
 

@@ -44,6 +44,24 @@ def test_autograd_extension_loads(lib):
     assert ext.take_timeline() == []
 
 
+@pytest.mark.parametrize("target,error", [
+    (torch.zeros(4, dtype=torch.int64), ValueError),
+    (torch.zeros(2, 3, dtype=torch.int64).t(), ValueError),
+    (torch.zeros(4, dtype=torch.int64, device="meta"), ValueError),
+    (torch.zeros(4, dtype=torch.int32), (TypeError, ValueError))])
+def test_target_check_refuses_other_devices(lib, target, error):
+    """The public target check and the C++ check under it refuse a tensor that
+    is not on the GPU before anything is launched: its kernel would be handed
+    a host address. Nothing to check is nothing to refuse."""
+    import nmce
+    from nmce import _lib as L
+    with pytest.raises(error, match="on a ROCm device|int64"):
+        nmce.validate_targets(target, 10)
+    with pytest.raises(error, match="on a ROCm device|int64"):
+        L.autograd_ext().TargetCheck(target, 10)
+    nmce.validate_targets(target[:0], 10)
+
+
 def test_head_output_node():
     """The measurements' stand-in for the LM-head node: the logits come back as
     a non-leaf alias (same storage) with a C++ grad_fn, and its backward hands
