@@ -431,6 +431,15 @@ int nmce_lmhead_ce_bwd(const void* hidden, const void* weight, int dtype, int64_
 int nmce_lmhead_ce_fused_layout(int64_t n_rows, int64_t hidden_size, int64_t vocab_local,
                                 int64_t token_chunk, int64_t* layout);
 
+/*
+ * layout[0] above on a device of `compute_units` compute units (0: the current
+ * device's count), or -1 for arguments that the layout refuses. Callers whose
+ * ranks must agree on a chunk by its workspace ask for one count everywhere.
+ */
+int64_t nmce_lmhead_ce_fused_workspace_bytes(int64_t n_rows, int64_t hidden_size,
+                                             int64_t vocab_local, int64_t token_chunk,
+                                             int compute_units);
+
 /* assumed[0] = hint[0], or 1.0 when hint[0] is zero, subnormal, infinite or
  * NaN (a gradient written for such a value could not be rescaled). Both are
  * device pointers to one float. */

@@ -1813,7 +1813,7 @@ struct FusedLayout {
   int64_t off_xt;     // the chunk's hidden rows transposed, X_c^T [h, ldt] bf16
 };
 
-FusedLayout fused_layout(int64_t n, int64_t h, int64_t v, int64_t token_chunk) {
+FusedLayout fused_layout(int64_t n, int64_t h, int64_t v, int64_t token_chunk, int cus) {
   FusedLayout L{};
   L.chunk = (token_chunk <= 0 || token_chunk >= n) ? n : round_up(token_chunk, kBN);
   if (L.chunk > n) L.chunk = n;
@@ -1822,7 +1822,7 @@ FusedLayout fused_layout(int64_t n, int64_t h, int64_t v, int64_t token_chunk) {
   L.vpad = round_up(v, kBM);
   L.nb = fwd_partial_blocks(v);
   const int64_t dx_tiles = ((L.chunk + kBM - 1) / kBM) * ((h + kBN - 1) / kBN);
-  L.dx_splits = choose_splits(dx_tiles, L.chunk * h, L.vpad, v, device_cus(), &L.dx_ks);
+  L.dx_splits = choose_splits(dx_tiles, L.chunk * h, L.vpad, v, cus, &L.dx_ks);
   int64_t off = 0;
   L.off_pt = off; off += align256(L.vpad * L.ldt * 2);
   L.off_part = off; off += align256(3 * L.nb * L.chunk * 4);
@@ -2176,7 +2176,7 @@ int check_fused_args(const void* hidden, const void* weight, int dtype, int64_t 
   if (n_rows > (int64_t{1} << 30) || vocab_local > (int64_t{1} << 30)) return NMCE_EINVAL_SHAPE;
   if (!operand_ok(hidden, hidden_size) || !operand_ok(weight, hidden_size))
     return NMCE_EINVAL_ALIGN;
-  L = fused_layout(n_rows, hidden_size, vocab_local, token_chunk);
+  L = fused_layout(n_rows, hidden_size, vocab_local, token_chunk, device_cus());
   // Per-lane offsets are 32-bit: 256 rows of P^T (dW's K-contiguous A) and 64
   // k-rows of P^T, W and X (MN-contiguous operands) must stay below 2 GiB;
   // ldt < 2^22 covers P^T, and operand_ok above bounds H.
@@ -2197,12 +2197,20 @@ int nmce_lmhead_ce_fused_layout(int64_t n_rows, int64_t hidden_size, int64_t voc
                                 int64_t token_chunk, int64_t* layout) {
   if (!layout) return NMCE_EINVAL_PTR;
   if (n_rows < 1 || hidden_size < 1 || vocab_local < 1) return NMCE_EINVAL_SHAPE;
-  const FusedLayout L = fused_layout(n_rows, hidden_size, vocab_local, token_chunk);
+  const FusedLayout L = fused_layout(n_rows, hidden_size, vocab_local, token_chunk, device_cus());
   const int64_t v[NMCE_LMHEAD_FUSED_LAYOUT_FIELDS] = {
       L.total,  L.chunk,    L.n_chunks, L.ldt,     L.vpad,      L.nb,
       L.off_pt, L.off_part, L.off_acc,  L.off_dxp, L.dx_splits, L.off_xt};
   for (int i = 0; i < NMCE_LMHEAD_FUSED_LAYOUT_FIELDS; ++i) layout[i] = v[i];
   return NMCE_OK;
+}
+
+int64_t nmce_lmhead_ce_fused_workspace_bytes(int64_t n_rows, int64_t hidden_size,
+                                             int64_t vocab_local, int64_t token_chunk,
+                                             int compute_units) {
+  if (n_rows < 1 || hidden_size < 1 || vocab_local < 1 || compute_units < 0) return -1;
+  return fused_layout(n_rows, hidden_size, vocab_local, token_chunk,
+                      compute_units > 0 ? compute_units : device_cus()).total;
 }
 
 int nmce_hint_assume(const float* hint, float* assumed, void* stream) {

@@ -60,6 +60,7 @@ SIGNATURES: dict[str, tuple] = {
     "nmce_lmhead_ce_bwd": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _i64,
                                     _p, _p, _i64, _p, _i64, _p]),
     "nmce_lmhead_ce_fused_layout": (_c_int, [_i64, _i64, _i64, _i64, _p]),
+    "nmce_lmhead_ce_fused_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _c_int]),
     "nmce_hint_assume": (_c_int, [_p, _p, _p]),
     "nmce_lmhead_ce_fused_chunk_stats": (_c_int, [_p, _p, _c_int, _i64, _i64, _i64, _p, _i64,
                                                   _i64, _i64, _p, _p, _p, _p, _i64, _p]),

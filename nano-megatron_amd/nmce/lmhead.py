@@ -14,7 +14,7 @@ LM head's vocabulary shard ``[V/tp, H]``. The loss and its gradients with
 respect to ``x`` and ``W`` are those of the two-step reference, but the
 ``[tokens, V/tp]`` logits are never stored: the one-pass path holds the
 bf16 exponentials of one chunk of tokens at a time (by default at most 2 GiB,
-and at most a quarter of the tokens unless every token at once takes no more
+and a quarter of the tokens unless every token's at once take no more
 memory), the recomputing path one vocabulary chunk's logit gradient (its
 workspace has room for two bf16 copies of it).
 
@@ -67,15 +67,15 @@ DEFAULT_VOCAB_CHUNK = 32768
 # The one-pass path goes through the tokens in chunks. A chunk's
 # exponentials, turned into its dZ^T in place, take 2 * V * chunk bytes
 # (bf16), so the chunk bounds what the fused loss holds of the logits: by
-# default at most a quarter of the tokens (rounded up to whole 256-token
-# tiles; every token only when there are at most 256) and at most
-# CHUNK_BUDGET_BYTES, so nothing the size of the [tokens, V] logits is
-# allocated. dW is then accumulated in fp32 across the chunks by the GEMM
-# epilogue (measured on one MI355X: [16384, 4096] x [128256, 4096] 38.55 ms in
-# four chunks of 4096 tokens, 36.97 in one). The accumulator is 4 V H bytes whatever the tokens, so
+# default a quarter of the tokens (rounded up to whole 256-token tiles; every
+# token when there are at most 256), and at most CHUNK_BUDGET_BYTES. dW is then
+# accumulated in fp32 across the chunks by the GEMM epilogue (measured on one
+# MI355X: [16384, 4096] x [128256, 4096] 38.55 ms in four chunks of 4096
+# tokens, 36.97 in one). The accumulator is 4 V H bytes whatever the tokens, so
 # with few tokens per unit of H it outgrows every token's exponentials: then
-# one chunk, which needs no accumulator, is the smaller workspace and the
-# faster pass (one_pass_token_chunk).
+# one chunk, which holds exponentials the size of the bf16 logits but needs no
+# accumulator, is the smaller workspace and the faster pass
+# (one_pass_token_chunk).
 CHUNK_BUDGET_BYTES = 2 << 30
 CHUNK_FRACTION = 4
 
@@ -90,26 +90,44 @@ def default_token_chunk(n_tokens: int, vocab_local: int) -> int:
     return min(chunk, fit, max(n_tokens, 1))
 
 
+# The compute units that one_pass_token_chunk counts with on every device: the
+# workspace holds the partials of dX's K ranges, whose number follows from the
+# device's count (256 on an MI355X), and ranks that took different chunks would
+# meet in different collectives.
+_RULE_COMPUTE_UNITS = 256
+
+
 def one_pass_token_chunk(n_tokens: int, hidden: int, vocab_local: int) -> int:
     """The chunk the one-pass path takes when the caller names none: every
-    token where that workspace is no larger than the one of
-    ``default_token_chunk``'s chunks, and else those chunks.
+    token where that workspace (nmce_lmhead_ce_fused_workspace_bytes, on 256
+    compute units) is no larger than the one of ``default_token_chunk``'s
+    chunks and its exponentials fit ``CHUNK_BUDGET_BYTES``, and else those
+    chunks. ``hidden`` is the padded hidden size.
 
     Against chunks of ``c`` tokens, one chunk of all ``n`` holds ``n - c`` more
     tokens' exponentials (2 V bytes each), partial statistics (12 bytes per 128
     vocabulary rows) and transposed hidden rows (2 H), and saves the fp32 dW
-    accumulator (4 V H): about n <= 2.6 H. It is also the faster side of the
-    line everywhere, since each further chunk reads and writes the accumulator
+    accumulator (4 V H): about n <= 2.6 H. Where its dX tiles do not fill the
+    device, it also holds their K ranges' fp32 partials (4 n H bytes each, up
+    to 8 ranges, more for few tiles), so some smaller n keep the chunks too:
+    [8653, 3584] x [50304, 3584] would take 1.88 GB against 1.00. One chunk is
+    the faster side, since each further chunk reads and writes the accumulator
     and shortens dW's K to the chunk ([4096, 4096] x [128256, 4096]: 12.9 ms
     in four chunks, 10.7 in one; [2103, 1600] x [50257, 1600]: 1.60 ms in
-    three, 1.13 in one; [512, 768] x [50304, 768]: 0.54 in two, 0.32 in one).
-    The line depends on sizes alone, so every tensor-parallel rank takes the
+    three, 1.13 in one; [512, 768] x [50304, 768]: 0.54 in two, 0.32 in one;
+    [8653, 3584] x [50304, 3584] 7.88 in four, 7.20 in one).
+    The rule depends on sizes alone, so every tensor-parallel rank takes the
     same chunks."""
     chunk = default_token_chunk(n_tokens, vocab_local)
-    more = (n_tokens - chunk) * (2 * vocab_local + 12 * -(-vocab_local // 128) + 2 * hidden)
-    if more <= 4 * vocab_local * hidden and 2 * vocab_local * n_tokens <= CHUNK_BUDGET_BYTES:
-        return max(n_tokens, 1)
-    return chunk
+    if chunk >= n_tokens or 2 * vocab_local * n_tokens > CHUNK_BUDGET_BYTES:
+        return chunk
+    lib = _lib.load()
+
+    def held(c):
+        return lib.nmce_lmhead_ce_fused_workspace_bytes(n_tokens, hidden, vocab_local, c,
+                                                        _RULE_COMPUTE_UNITS)
+
+    return n_tokens if held(n_tokens) <= held(chunk) else chunk
 
 
 _ALIGN = 64  # hidden size granularity of the GEMM kernels
@@ -406,7 +424,7 @@ def lmhead_vocab_parallel_cross_entropy(
     When a gradient is wanted the forward is one pass (module docstring),
     going through ``token_chunk`` tokens at a time (default
     ``one_pass_token_chunk``: a quarter of the tokens, or all of them where
-    that takes no more memory, within ``CHUNK_BUDGET_BYTES``; pass the token
+    that whole workspace is no larger, within ``CHUNK_BUDGET_BYTES``; pass the token
     count to hold every token's exponentials at once) and assuming the upstream value held by
     ``upstream_hint`` (a one-element fp32 device tensor; default: one per
     call site). ``one_pass=False`` selects the forward that keeps only the

@@ -276,15 +276,18 @@ def test_one_pass_token_chunk_budget(lib):
                                          (4096, 4096, 128256, True), (8192, 4096, 128256, True),
                                          (8704, 4096, 128256, False),   # 2 GiB of exponentials
                                          (16384, 4096, 128256, False), (16384, 3072, 256000, False),
-                                         (2048, 512, 32000, False), (1280, 512, 32000, True),
-                                         (100, 64, 1000, True), (1, 64, 1, True)])
+                                         (2048, 512, 32000, False),
+                                         (100, 64, 1000, True), (1, 64, 1, True),
+                                         # fewer bytes of exponentials than the accumulator
+                                         # saves, but more with dX's K ranges
+                                         (1280, 512, 32000, False), (6971, 4032, 8192, False),
+                                         (7944, 3712, 32000, False), (8653, 3584, 50304, False),
+                                         (8166, 3840, 32000, False)])
 def test_one_pass_chunk_holds_every_token_where_smaller(lib, n, h, v, whole):
-    """The one-pass path's own chunk is every token exactly where that
-    workspace is no larger than the quarter chunks' (their fp32 dW accumulator
-    against the further tokens' exponentials) and its exponentials fit the
-    budget; otherwise it is default_token_chunk's. The regions are the
-    library's layout, without the split dX product's partials (their count is
-    the device's)."""
+    """The one-pass path's own chunk is every token exactly where that whole
+    workspace is no larger than the quarter chunks' and its exponentials fit
+    the budget; otherwise it is default_token_chunk's. (The layout's K ranges
+    are those of 256 compute units here, the count that the rule uses.)"""
     import ctypes
     from nmce import _lib as L
     from nmce import lmhead
@@ -292,15 +295,34 @@ def test_one_pass_chunk_holds_every_token_where_smaller(lib, n, h, v, whole):
 
     def held(chunk):
         assert lib.nmce_lmhead_ce_fused_layout(n, h, v, chunk, ctypes.addressof(buf)) == 0
-        return buf[0] - (buf[11] - buf[9])
+        for units in (0, 256):
+            assert lib.nmce_lmhead_ce_fused_workspace_bytes(n, h, v, chunk, units) == buf[0]
+        return buf[0]
 
     quarter = lmhead.default_token_chunk(n, v)
     chunk = lmhead.one_pass_token_chunk(n, h, v)
     assert chunk == (n if whole else quarter)
+    assert held(chunk) <= held(quarter)
     if chunk != quarter:
-        # the rule counts whole tokens; the layout pads them to 64
-        assert held(chunk) <= held(quarter) + 64 * (2 * v + 2 * h) + 4096
         assert 2 * v * chunk <= lmhead.CHUNK_BUDGET_BYTES
+    elif quarter < n:
+        assert held(n) > held(quarter) or 2 * v * n > lmhead.CHUNK_BUDGET_BYTES
+
+
+def test_one_pass_chunk_never_holds_more(lib):
+    """The same over drawn sizes: the workspace of the one-pass path's own chunk
+    is never larger than that of default_token_chunk's, and the chunk does not
+    depend on the device."""
+    import random
+    from nmce import lmhead
+    rng = random.Random(5)
+    size = lib.nmce_lmhead_ce_fused_workspace_bytes
+    for _ in range(2000):
+        n, h, v = rng.randint(1, 12000), 64 * rng.randint(1, 64), rng.randint(1, 256000)
+        chunk, quarter = lmhead.one_pass_token_chunk(n, h, v), lmhead.default_token_chunk(n, v)
+        assert chunk in (n, quarter)
+        assert size(n, h, v, chunk, 256) <= size(n, h, v, quarter, 256), (n, h, v)
+    assert size(0, 64, 100, 0, 256) == size(16, 64, 0, 0, 256) == size(16, 64, 100, 0, -1) == -1
 
 
 def test_fused_dx_split_choice(lib):
