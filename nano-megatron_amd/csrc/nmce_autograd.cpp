@@ -236,7 +236,8 @@ at::Tensor flag_word(const at::Tensor& like, hipStream_t st) {
 
 // Pinned count words with their events, pooled per device (an event belongs
 // to one) and reused once a check has been waited for (the kernel writes the
-// word through its host mapping).
+// words through their host mapping). The pool holds as many as were ever in
+// flight at once, each with the words of the largest check it served.
 struct CheckSlot {
   at::Tensor host;
   hipEvent_t event = nullptr;
@@ -245,22 +246,31 @@ struct CheckSlot {
 std::mutex g_slot_lock;
 std::map<int, std::vector<CheckSlot>> g_slots;
 
-// The caller has made `device` the current one.
-CheckSlot take_slot(int device) {
+// A slot of at least `words` words. The caller has made `device` the current one.
+CheckSlot take_slot(int device, int64_t words) {
+  CheckSlot s;
+  s.device = device;
   {
     std::lock_guard<std::mutex> g(g_slot_lock);
     std::vector<CheckSlot>& free = g_slots[device];
     if (!free.empty()) {
-      CheckSlot s = free.back();
+      s = std::move(free.back());
       free.pop_back();
-      return s;
     }
   }
-  CheckSlot s;
-  s.device = device;
-  s.host = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  TORCH_CHECK(hipEventCreateWithFlags(&s.event, hipEventDisableTiming) == hipSuccess,
-              "nmce: hipEventCreateWithFlags failed");
+  if (!s.event)
+    TORCH_CHECK(hipEventCreateWithFlags(&s.event, hipEventDisableTiming) == hipSuccess,
+                "nmce: hipEventCreateWithFlags failed");
+  if (!s.host.defined() || s.host.numel() < words) {
+    int64_t room = 1;
+    while (room < words) room *= 2;
+    try {
+      s.host = at::empty({room}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    } catch (...) {
+      (void)hipEventDestroy(s.event);
+      throw;
+    }
+  }
   return s;
 }
 
@@ -268,13 +278,13 @@ CheckSlot take_slot(int device) {
 // the pinned word until then), and gives the slot back.
 class CheckGuard {
  public:
-  explicit CheckGuard(CheckSlot s) : slot_(std::move(s)) {}
+  CheckGuard(CheckSlot s, int64_t words) : slot_(std::move(s)), words_(words) {}
   int32_t* host() { return slot_.host.data_ptr<int32_t>(); }
   hipEvent_t event() const { return slot_.event; }
   void recorded() { recorded_ = true; }
   // The count, once the check has finished. Polls first (the count is
   // usually there within microseconds of the launch), then blocks.
-  int32_t wait() {
+  int64_t wait() {
     if (recorded_) {
       pybind11::gil_scoped_release nogil;
       const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
@@ -286,7 +296,10 @@ class CheckGuard {
       TORCH_CHECK(q == hipSuccess, "nmce: waiting for the target check failed: ",
                   hipGetErrorString(q));
     }
-    return *static_cast<volatile int32_t*>(slot_.host.data_ptr<int32_t>());
+    const volatile int32_t* word = slot_.host.data_ptr<int32_t>();
+    int64_t count = 0;
+    for (int64_t i = 0; i < words_; ++i) count += word[i];
+    return count;
   }
   ~CheckGuard() {
     if (recorded_) (void)hipEventSynchronize(slot_.event);
@@ -296,20 +309,29 @@ class CheckGuard {
 
  private:
   CheckSlot slot_;
+  int64_t words_;
   bool recorded_ = false;
 };
 
 // The check of flat contiguous targets on the current stream of their device,
-// its event recorded behind it; `flag` is that stream's device word.
+// its event recorded behind it. With `flag`, that stream's device word, one
+// workgroup counts into it and one host word; without, as many workgroups as
+// there are slots of targets count into a host word each: 3.5 us at any of 64
+// to a million targets, where the one workgroup takes 3.8 at 16384, 16 at
+// 131072 and 126 at a million.
 std::unique_ptr<CheckGuard> launch_check(const at::Tensor& target, int64_t vocab_total,
-                                         const at::Tensor& flag, hipStream_t st) {
-  auto guard = std::make_unique<CheckGuard>(take_slot(target.device().index()));
-  timed("nmce_validate_targets_once", st, [&] {
-    return nmce_validate_targets_once(target.data_ptr<int64_t>(), target.numel(), vocab_total,
-                                      guard->host(), flag.data_ptr<int32_t>(), st);
+                                         const at::Tensor* flag, hipStream_t st) {
+  const int64_t n = target.numel();
+  const int64_t words = flag ? 1 : nmce_validate_slots(n);
+  auto guard = std::make_unique<CheckGuard>(take_slot(target.device().index(), words), words);
+  timed(flag ? "nmce_validate_targets_once" : "nmce_validate_targets", st, [&] {
+    return flag ? nmce_validate_targets_once(target.data_ptr<int64_t>(), n, vocab_total,
+                                             guard->host(), flag->data_ptr<int32_t>(), st)
+                : nmce_validate_targets(target.data_ptr<int64_t>(), n, vocab_total,
+                                        guard->host(), st);
   });
   if (hipEventRecord(guard->event(), st) != hipSuccess) {
-    // The check may still write the slot's word: let it finish first.
+    // The check may still write the slot's words: let it finish first.
     (void)hipStreamSynchronize(st);
     TORCH_CHECK(false, "nmce: hipEventRecord failed");
   }
@@ -317,20 +339,9 @@ std::unique_ptr<CheckGuard> launch_check(const at::Tensor& target, int64_t vocab
   return guard;
 }
 
-// The device word of checks that no kernel reads the result of (their callers
-// write nothing until the host has it), one per device: apart from the words
-// that one-pass kernels read, which another thread's check on the same stream
-// must not touch.
-at::Tensor unread_word(const at::Tensor& like) {
-  static std::map<int, at::Tensor> words;
-  std::lock_guard<std::mutex> g(g_flag_lock);
-  at::Tensor& w = words[static_cast<int>(like.device().index())];
-  if (!w.defined()) w = at::empty({1}, like.options().dtype(at::kInt));
-  return w;
-}
-
 // A target check in flight, for the callers that launch their loss kernels
-// from Python meanwhile: wait() gives the count of bad targets (once the check
+// from Python meanwhile (they write nothing that a bad target must not touch
+// until the host has the count, so no kernel reads it): wait() gives the count of bad targets (once the check
 // is over) and the slot back; so does the end of its life.
 class TargetCheck {
  public:
@@ -345,10 +356,10 @@ class TargetCheck {
                       "nmce: the target check takes a non-empty contiguous tensor");
     const c10::DeviceGuard device_guard(target.device());
     hipStream_t st = stream_of(target);
-    guard_ = launch_check(target, vocab_total, unread_word(target), st);
+    guard_ = launch_check(target, vocab_total, nullptr, st);
   }
   bool query() const { return !guard_ || hipEventQuery(guard_->event()) == hipSuccess; }
-  int32_t wait() {
+  int64_t wait() {
     if (guard_) {
       count_ = guard_->wait();
       guard_.reset();
@@ -358,7 +369,7 @@ class TargetCheck {
 
  private:
   std::unique_ptr<CheckGuard> guard_;
-  int32_t count_ = 0;
+  int64_t count_ = 0;
 };
 
 at::Tensor one_pass_mean(const at::Tensor& logits, const at::Tensor& target,
@@ -379,7 +390,7 @@ at::Tensor one_pass_mean_checked(const at::Tensor& logits, const at::Tensor& tar
   const c10::DeviceGuard device_guard(logits.device());
   hipStream_t st = stream_of(logits);
   const at::Tensor flag = flag_word(logits, st);
-  const std::unique_ptr<CheckGuard> guard = launch_check(target, vocab_total, flag, st);
+  const std::unique_ptr<CheckGuard> guard = launch_check(target, vocab_total, &flag, st);
   at::Tensor loss = OnePassMean::apply(logits, target, hint,
                                        reinterpret_cast<int64_t>(flag.data_ptr<int32_t>()),
                                        inplace, vocab_start);

@@ -151,7 +151,7 @@ def _check_inputs(logits: torch.Tensor, target: torch.Tensor, vocab_start: int,
 
 class _PendingCheck:
     """A target check in flight: its kernel writes the count of bad targets
-    straight into a pooled pinned word, which goes back to its pool once the
+    straight into pooled pinned words, which go back to their pool once the
     check is over. Every caller ends with ``raise_if_bad()`` or, when it leaves
     early on an exception, ``wait()``. ``event.query()`` tells whether the
     check is over."""
@@ -173,13 +173,14 @@ class _PendingCheck:
 def launch_target_check(target: torch.Tensor, vocab_size: int) -> _PendingCheck | None:
     """Start the target check of cross_entropy.py:79-81 without blocking.
 
-    One workgroup counts the targets outside ``[0, vocab_size)`` on the
-    current stream, in front of the loss kernels that the caller enqueues
-    next; ``raise_if_bad()`` on the result waits for that kernel alone. It is
-    one call into the C++ module: a check on a side stream, with its events and
-    stream switches in Python, cost the host 60 us a call, a third of what the
-    fused loss of a few hundred tokens takes, where the check itself takes the
-    loss stream 2-4 us.
+    One kernel counts the targets outside ``[0, vocab_size)`` on the current
+    stream, a workgroup and a word per 1024 of them, in front of the loss
+    kernels that the caller enqueues next; ``raise_if_bad()`` on the result
+    waits for that kernel alone. It is one call into the C++ module: a check on
+    a side stream, with its events and stream switches in Python, cost the host
+    60 us a call, a third of what the fused loss of a few hundred tokens takes,
+    where the check itself takes the loss stream 3-4 us, up to millions of
+    targets.
     """
     if target.numel() == 0:
         return None

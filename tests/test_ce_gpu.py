@@ -394,6 +394,44 @@ def test_out_of_vocabulary_target_raises():
     nmce.validate_targets(t, ctx.tp_size * 16)
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 70001, 1 << 20])
+def test_target_check_slots(n):
+    """The check that the two-pass and the fused path start from Python: a count
+    per 1024 targets by nmce_validate_targets (one workgroup walking a million
+    of them would hold the loss stream for over 100 us), bad ones at the ends
+    of the first, a middle and the last slot, and the pooled words good for the
+    next check, of another size."""
+    import nmce
+    from nmce import _lib as L
+    lib, ext = L.load(), L.autograd_ext()
+    print(f"[gpu] target check n={n}", flush=True)
+    slots = lib.nmce_validate_slots(n)
+    t = torch.randint(0, 1000, (n,), device=DEV)
+    counts = torch.full((slots + 1,), -7, dtype=torch.int32, device=DEV)
+    ext.take_timeline()
+    for at in ((), (0,), (n - 1,), (0, min(1023, n - 1), n // 2 // 1024 * 1024, n - 1)):
+        bad = t.clone()
+        for k, i in enumerate(sorted(set(at))):
+            bad[i] = (1000, -1, 1 << 40)[k % 3]
+        want = torch.zeros(slots * 1024, dtype=torch.int32, device=DEV)
+        want[:n] = ((bad < 0) | (bad >= 1000)).int()
+        L.check(lib.nmce_validate_targets(bad.data_ptr(), n, 1000, counts.data_ptr(),
+                                          L.stream_handle(torch.device(DEV))), "validate")
+        assert torch.equal(counts[:slots], want.view(slots, 1024).sum(1).int())
+        assert counts[slots].item() == -7  # no word past the last slot
+        ext.set_timing(True)
+        check = ext.TargetCheck(bad, 1000)
+        ext.set_timing(False)
+        assert check.wait() == check.wait() == len(set(at))
+        assert check.query()
+        assert [name for name, _ in ext.take_timeline()] == ["nmce_validate_targets"]
+        if at:
+            with pytest.raises(ValueError, match="outside the model vocabulary"):
+                nmce.validate_targets(bad, 1000)
+        nmce.validate_targets(bad[1:2] if n > 2 else t, 1000)
+    assert ext.TargetCheck(t, 1).wait() == int((t > 0).sum())
+
+
 def test_target_check_waits_when_the_loss_raises(monkeypatch):
     """The check kernel writes its counts straight into a pinned host buffer,
     so a loss call that leaves on an exception must still wait for it before
