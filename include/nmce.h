@@ -282,6 +282,8 @@ int nmce_stream_copy(const void* src, void* dst, int64_t bytes, void* stream);
  * the tied embedding, tp_layers.py:108) is [vocab_local, hidden_size], both
  * row-major with row stride hidden_size, 16-byte aligned; hidden_size must be
  * a multiple of 64. Logits are accumulated in fp32 and not rounded to bf16.
+ * The gradients that the entries below write, grad_hidden and grad_weight, need
+ * be aligned to their element only (16-byte aligned ones leave faster).
  * --------------------------------------------------------------------------- */
 
 /* Device workspace bytes needed by nmce_lmhead_ce_fwd_stats. */

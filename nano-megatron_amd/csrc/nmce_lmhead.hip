@@ -1492,10 +1492,12 @@ __global__ __launch_bounds__(256) void lmhead_dz_rescale_kernel(
 }
 
 // A product split over K (gemm_store_kernel, splits > 1) summed into bf16:
-// out[r * ldo + c] = bf16(sum_s part[s][r][c]) for r < M, c < N (N % 4 == 0),
+// out[r * ldo + c] = bf16(sum_s part[s][r][c]) for r < M, c < N (N, ldo % 4 == 0),
 // with the partials [splits][M][N] fp32 contiguous. The splits are added in
 // order, so the result does not depend on how the GEMM was scheduled; eight
-// ranges' loads are in flight at a time (up to 256 ranges are summed).
+// ranges' loads are in flight at a time. One token chunk has at most one round
+// of ranges (256); the recomputing backward sums those of all its vocabulary
+// chunks, a thousand and more where a caller asks for small ones.
 __global__ __launch_bounds__(256) void split_sum_bf16_kernel(const float* __restrict__ part,
                                                              int splits, int64_t M, int64_t N,
                                                              uint16_t* __restrict__ out,
@@ -1514,8 +1516,13 @@ __global__ __launch_bounds__(256) void split_sum_bf16_kernel(const float* __rest
   }
   const int64_t r = i / N, c = i - r * N;
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  *reinterpret_cast<u32x2*>(out + r * ldo + c) = u32x2{pack_bf16x2(a[0], a[1]),
-                                                       pack_bf16x2(a[2], a[3])};
+  uint16_t* dst = out + r * ldo + c;
+  if ((reinterpret_cast<uintptr_t>(out) & 7) == 0) {
+    *reinterpret_cast<u32x2*>(dst) = u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
+  } else {  // gradients need be aligned to their element only
+#pragma unroll
+    for (int k = 0; k < 4; ++k) dst[k] = f32_to_bf16(a[k]);
+  }
 }
 
 // The transpose of transpose_tile by itself.

@@ -301,6 +301,56 @@ def test_fused_backward_k_ranges(n, h, v, chunk):
     check_grad(dw, rdw, f"dW chunk {chunk}")
 
 
+@pytest.mark.parametrize("n,h,v,chunk", [(77, 64, 9000, 4096), (300, 192, 20000, 0),
+                                         (515, 320, 5001, 2048), (1000, 64, 3000, 256)])
+def test_backward_gradients_aligned_to_their_element(n, h, v, chunk):
+    """The C backwards take gradients at any bf16 address: split dX products (of
+    the recomputing backward and of the one-pass chunk) whose summed partials
+    go to a base 2, 6 or 8 bytes past a 16-byte boundary give the bits of an
+    aligned one, and touch nothing around it."""
+    from nmce import _lib as L
+    from nmce import lmhead
+    lib = L.load()
+    print(f"[gpu] unaligned gradients n={n} h={h} v={v} chunk={chunk}", flush=True)
+    x, w, t = make_inputs(n, h, v, seed=n + v, w_std=0.5)
+    xd, wd, td = x.to(DEV), w.to(DEV), t.to(DEV)
+    stream = L.stream_handle(torch.device(DEV))
+    args = (xd.data_ptr(), wd.data_ptr(), L.NMCE_BF16, n, h, v, td.data_ptr())
+    lay = lmhead._fused_layout(lib, n, h, v, 0)
+    ws = torch.empty(lay["total"], dtype=torch.uint8, device=DEV)
+    out, tgt = torch.empty((3, n), device=DEV), torch.empty(n, device=DEV)
+    one = torch.ones(1, device=DEV)
+    bws = torch.empty(lib.nmce_lmhead_ce_bwd_workspace_bytes(n, h, v, chunk), dtype=torch.uint8,
+                      device=DEV)
+    results = []
+    for off in (0, 1, 3, 4):
+        got = []
+        for one_pass in (True, False):
+            dx = torch.full((n * h + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+            dw = torch.full((v * h + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+            px, pw = dx[off:].data_ptr(), dw[off:].data_ptr()
+            if one_pass:
+                L.check(lib.nmce_lmhead_ce_fused_chunk_loss(
+                    *args, 0, 0, out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(),
+                    tgt.data_ptr(), one.data_ptr(), None, ws.data_ptr(), ws.numel(), stream),
+                    "loss")
+                L.check(lib.nmce_lmhead_ce_fused_chunk_grads(
+                    *args, 0, 0, 0, out[1].data_ptr(), out[2].data_ptr(), tgt.data_ptr(),
+                    one.data_ptr(), 0, float(n), px, pw, ws.data_ptr(), ws.numel(), stream),
+                    "grads")
+            else:
+                L.check(lib.nmce_lmhead_ce_bwd(
+                    *args, 0, out[1].data_ptr(), out[2].data_ptr(), one.data_ptr(), 0, px, pw,
+                    chunk, bws.data_ptr(), bws.numel(), stream), "bwd")
+            for g, size in ((dx, n * h), (dw, v * h)):
+                assert (g[:off] == 7.0).all() and (g[off + size:] == 7.0).all()
+                got.append(g[off:off + size].clone())
+        results.append(got)
+    assert lay["dx_splits"] > 1 and all(g.abs().sum() > 0 for g in results[0])
+    for got in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got, results[0]))
+
+
 def test_bwd_dz_buffers():
     """The recomputed logit gradient itself, read back from the workspace after
     ``nmce_lmhead_ce_bwd_dz`` for both chunks of a ragged shard (300 tokens,
