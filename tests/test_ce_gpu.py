@@ -843,15 +843,18 @@ RAGGED_WIDTHS = {torch.bfloat16: (1, 7, 9, 1001, 8191, 32767, 50257, 65535, 6553
                  torch.float32: (1, 3, 5, 1001, 4095, 16385, 32767, 32769, 50257, 65535)}
 
 
+@pytest.mark.parametrize("infinite", [False, True])
 @pytest.mark.parametrize("inplace", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_one_pass_ragged_rows(dtype, inplace):
+def test_one_pass_ragged_rows(dtype, inplace, infinite):
     """Rows of odd widths (every row starts at another offset from a 16-byte
     boundary) through the one-pass kernel's ragged form, both sides of each
     register-slot count and of the wide kernel, against the two-pass path: the
     loss and the gradient for upstream 1.0 bit for bit; a miss (0.5, a
     power-of-two ratio) too. Targets at the row's first and last columns (the
-    edge elements) and at the body's ends."""
+    edge elements) and at the body's ends. Every value finite, so that the mean
+    loss is one and compares; and with infinities in two rows' edge elements,
+    where the mean is NaN and the other rows' gradients compare."""
     import nmce
     ctx = nmce.ParallelContext.single()
     for v in RAGGED_WIDTHS[dtype]:
@@ -863,7 +866,8 @@ def test_one_pass_ragged_rows(dtype, inplace):
         ends = torch.tensor([0, v - 1, min(7, v - 1), max(0, v - 8), min(8, v - 1)], device=DEV)
         t[:min(n, 30)] = ends[torch.arange(min(n, 30), device=DEV) % 5]
         x[1, :] = -1.0e30  # a row far below any floor's neighbourhood
-        x[2, 0], x[3, v - 1] = float("-inf"), float("inf") if v > 1 else 0.0
+        if infinite:
+            x[2, 0], x[3, v - 1] = float("-inf"), float("inf") if v > 1 else 0.0
         hint = torch.ones(1, device=DEV)
         for upstream in (1.0, 0.5):
             got = []
@@ -878,9 +882,42 @@ def test_one_pass_ragged_rows(dtype, inplace):
                 (loss * upstream).backward()
                 got.append((loss.detach(), leaf.grad))
             (l1, g1), (l2, g2) = got
+            assert l1.isfinite() == (not infinite), (v, l1)
             assert torch.equal(l1, l2) or (l1.isnan() and l2.isnan()), (v, upstream)
             ok = ((g1 == g2) | (g1.isnan() & g2.isnan())).all()
             assert ok, f"gradient differs at v={v} upstream={upstream}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_pass_ragged_token_losses(dtype):
+    """nmce_ce_fwd_bwd_ragged's per-token loss, maximum and sum are nmce_ce_fwd's
+    bit for bit at the same widths, which a mean over the rows could hide:
+    targets at every edge element and around the body's ends, and rows with
+    infinities and of nothing but -inf beside the finite ones."""
+    from nmce import _lib as L
+    lib = L.load()
+    stream = L.stream_handle(torch.device(DEV))
+    code = L.dtype_code(dtype)
+    one, assumed = torch.ones(1, device=DEV), torch.empty(1, device=DEV)
+    for v in RAGGED_WIDTHS[dtype]:
+        n = 40
+        print(f"[gpu] ragged token losses v={v} {dtype}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(v + 1)
+        x = (torch.randn(n, v, device=DEV, generator=g) * 3.0).to(dtype)
+        k = torch.arange(n, device=DEV)
+        t = torch.where(k < 20, k, v - 1 - (k - 20)).clamp(0, v - 1)
+        inf = float("inf")
+        x[1], x[2, 0], x[3, v - 1], x[4] = -1.0e30, -inf, inf, -inf
+        got, want = torch.full((3, n), 7.0, device=DEV), torch.full((3, n), 7.0, device=DEV)
+        grad = torch.empty_like(x)
+        rows = (x.data_ptr(), code, n, v, v, t.data_ptr())
+        L.check(lib.nmce_ce_fwd(*rows, *(o.data_ptr() for o in want), stream), "fwd")
+        L.check(lib.nmce_ce_fwd_bwd_ragged(x.data_ptr(), grad.data_ptr(), code, n, v, v, v,
+                                           t.data_ptr(), *(o.data_ptr() for o in got),
+                                           one.data_ptr(), assumed.data_ptr(), None, float(n),
+                                           stream), "ragged")
+        assert want[0, 5:].isfinite().all() and want[0, :2].isfinite().all()
+        assert ((got == want) | (got.isnan() & want.isnan())).all(), v
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
