@@ -493,54 +493,47 @@ def test_gemm_mfmas_keep_their_wait_states(tmp_path):
     """The GEMM core's MFMAs are inline asm, around which the compiler puts no
     wait states. In the generated code no VALU instruction writes a source of
     an MFMA within two wait states before it, and none touches the registers
-    that one wrote within 16 wait states after it."""
-    import re
+    that one wrote within 16 wait states after it, along every path (a loop's
+    back edge is where a compiler would move a fragment's registers)."""
     import subprocess
 
+    from _util import mfma_hazards
     from nmce import _build
     asm = tmp_path / "lmhead.s"
     subprocess.run([_build.hipcc(), *_build.HIPCC_FLAGS, "-S", "--cuda-device-only",
                     str(_build.CSRC_DIR / "nmce_lmhead.hip"), "-o", str(asm)], check=True,
                    capture_output=True)
-
-    def regs(token):
-        m = re.match(r"([va])(?:\[(\d+):(\d+)\]|(\d+))$", token)
-        if not m:
-            return set()
-        lo, hi = (m[2], m[3]) if m[2] else (m[4], m[4])
-        return {(m[1], i) for i in range(int(lo), int(hi) + 1)}
-
-    recent = []   # (wait states, VALU destination) of the last instructions
-    pending = []  # (registers an MFMA writes, wait states since it)
-    mfmas = 0
-    for line in asm.read_text().splitlines():
-        if re.match(r"_Z\w+:", line):
-            recent, pending = [], []
-        op, _, rest = line.split(";")[0].strip().partition(" ")
-        if not op or op.startswith(".") or op.endswith(":"):
-            continue
-        tokens = [t.strip() for t in re.split(r",(?![^\[]*\])", rest)]
-        states = int(tokens[0]) + 1 if op == "s_nop" else 1
-        if op.startswith("v_mfma"):
-            mfmas += 1
-            sources = set().union(*map(regs, tokens[1:4]))
-            waited = 0
-            for n, written in reversed(recent):
-                if waited >= 2:
-                    break
-                assert not written & sources, line
-                waited += n
-            recent.append((1, set()))
-        else:
-            used = set().union(*map(regs, tokens))
-            for written, _ in pending:
-                assert not written & used, line
-            recent.append((states, regs(tokens[0]) if op.startswith("v_") else set()))
-        recent = recent[-3:]
-        pending = [(w, n + states) for w, n in pending if n + states < 16]
-        if op.startswith("v_mfma"):
-            pending.append((regs(tokens[0]), 0))
+    mfmas, offenders = mfma_hazards(asm.read_text())
     assert mfmas > 1000
+    assert not offenders, offenders[:5]
+
+
+@pytest.mark.parametrize("body,hazards", [
+    # a fragment moved at the loop's end, read at its head
+    (["v_mov_b32_e32 v9, 0", "s_nop 1", "L:", "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]",
+      "s_nop 15", "v_mov_b32_e32 v8, v20", "s_cbranch_scc1 L"], 1),
+    (["L:", "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]", "s_nop 15", "v_mov_b32_e32 v8, v20",
+      "s_nop 0", "s_cbranch_scc1 L"], 0),
+    # an accumulator read behind a taken branch, and the long way round
+    (["v_mfma a[0:3], v[0:3], v[8:11], a[0:3]", "s_cbranch_scc1 L", "s_nop 15", "L:",
+      "v_accvgpr_read_b32 v1, a3"], 1),
+    (["v_mfma a[0:3], v[0:3], v[8:11], a[0:3]", "s_branch L", "v_accvgpr_read_b32 v1, a3", "L:",
+      "s_nop 15", "v_accvgpr_read_b32 v1, a3"], 0),
+    # a source written just before, as either result of a swap too; an accumulator's block
+    # that is written anew by the next MFMA
+    (["v_add_f32_e32 v3, v1, v2", "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]"], 1),
+    (["v_permlane32_swap_b32_e32 v30, v9", "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]"], 1),
+    (["v_add_f32_e32 v4, v1, v2", "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]",
+      "v_mfma a[0:3], v[0:3], v[8:11], a[0:3]"], 0),
+    # a store of results that have not settled
+    (["v_mfma a[0:3], v[0:3], v[8:11], a[0:3]", "s_nop 14", "ds_write_b128 v7, a[0:3]"], 1),
+    (["v_mfma a[0:3], v[0:3], v[8:11], a[0:3]", "s_nop 15", "ds_write_b128 v7, a[0:3]"], 0)])
+def test_mfma_hazard_scan(body, hazards):
+    """The scan itself, on listings with and without an offender: it follows
+    branches both ways and counts wait states along each path."""
+    from _util import mfma_hazards
+    text = "\n".join(["kernel:"] + body + ["s_endpgm"])
+    assert len(mfma_hazards(text)[1]) == hazards, mfma_hazards(text)
 
 
 def test_wide_buffer_stores_go_through_the_helper():
