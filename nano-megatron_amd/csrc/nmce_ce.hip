@@ -1131,23 +1131,6 @@ int nmce_ce_bwd(const void* logits, void* grad, int dtype, int64_t n_rows, int64
 }  // extern "C"
 
 namespace {
-// Compute units of the current device (256 if the query fails).
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  int n_cu = 256;
-  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
-    if (cus[dev] == 0) {
-      int v = 0;
-      if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-          v > 0)
-        cus[dev] = v;
-    }
-    if (cus[dev] > 0) n_cu = cus[dev];
-  }
-  return n_cu;
-}
-
 // Workgroups of a kernel that walks rows with `per_cu` workgroups per compute
 // unit, capped by the rows.
 unsigned rows_grid(int64_t n_rows, int per_cu) {
@@ -1238,14 +1221,10 @@ int launch_fwdbwd(const void* logits, void* grad, int64_t n_rows, int64_t vocab,
   T* g = static_cast<T*>(grad);
   const int64_t per_lane = (vocab / Elem<T>::kPerVec + kStatsBlock - 1) / kStatsBlock;
   if (per_lane > kOnePassVecs[1]) {
-    static bool lds_ok = false;  // the attribute is set once per process and kernel
-    if (!lds_ok) {
-      const hipError_t e =
-          hipFuncSetAttribute(reinterpret_cast<const void*>(&ce_fwdbwd_wide_kernel<T, kRagged>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kWideLdsBytes);
-      if (e != hipSuccess) return static_cast<int>(e);
-      lds_ok = true;
-    }
+    static std::atomic<bool> lds_ok{false};
+    const int rc = allow_lds(reinterpret_cast<const void*>(&ce_fwdbwd_wide_kernel<T, kRagged>),
+                             kWideLdsBytes, lds_ok);
+    if (rc) return rc;
     hipLaunchKernelGGL((ce_fwdbwd_wide_kernel<T, kRagged>), dim3(rows_grid(n_rows, 1)),
                        dim3(kStatsBlock), kWideLdsBytes, st, x, g, n_rows, vocab, ld, ld_grad,
                        target, loss, g_max, g_sumexp_m1, expect, assumed, bad_flag, gout_div);

@@ -1,4 +1,4 @@
-// Device-side helpers shared by the gfx950 kernels of libnmce.
+// Helpers shared by the gfx950 kernels of libnmce and their launchers.
 //
 // Wave64 reductions use DPP (row-local butterflies, then row_bcast15/31 to
 // carry row totals up to lane 63), bf16 is unpacked by shifting into the high
@@ -10,7 +10,34 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace nmce {
+
+// Host: lets a kernel be launched with `bytes` of dynamic LDS, once per process
+// and kernel (`done` is the kernel's own flag; threads that launch it for the
+// first time together all set the same value). 0 or a hipError_t.
+inline int allow_lds(const void* kernel, int bytes, std::atomic<bool>& done) {
+  if (done.load(std::memory_order_acquire)) return 0;
+  const hipError_t e =
+      hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return static_cast<int>(e);
+  done.store(true, std::memory_order_release);
+  return 0;
+}
+
+// Host: compute units of the current device (256 if the query fails), asked
+// for once per device.
+inline int device_cus() {
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0 &&
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+    cus[dev].store(n, std::memory_order_relaxed);
+  return n > 0 ? n : 256;
+}
 
 constexpr float kLog2e = 1.4426950408889634f;  // exp(x) = exp2(x * kLog2e)
 constexpr float kNegHuge = -3.402823466e+38f;  // finite floor for running maxima

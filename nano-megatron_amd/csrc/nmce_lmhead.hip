@@ -1545,22 +1545,16 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-bool lds_configured = false;
-
 int configure_lds() {
-  if (lds_configured) return NMCE_OK;
+  static std::atomic<bool> done[4];
   const void* kernels[] = {
       reinterpret_cast<const void*>(&lmhead_stats_kernel),
       reinterpret_cast<const void*>(&lmhead_dz_kernel<true>),
       reinterpret_cast<const void*>(&lmhead_dz_kernel<false>),
       reinterpret_cast<const void*>(&lmhead_p_kernel),
   };
-  for (const void* k : kernels) {
-    const hipError_t e =
-        hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return static_cast<int>(e);
-  }
-  lds_configured = true;
+  for (int i = 0; i < 4; ++i)
+    if (const int rc = allow_lds(kernels[i], kLdsBytes, done[i])) return rc;
   return NMCE_OK;
 }
 
@@ -1578,14 +1572,11 @@ int launch_store(dim3 grid, hipStream_t stream, const uint16_t* A, int64_t lda, 
                  const uint16_t* B, int64_t ldb, int64_t N, int64_t K, uint16_t* C, float* Cf,
                  int64_t ldc, int64_t ka_rows, int64_t kb_rows, int splits,
                  int64_t ks, int64_t split_stride) {
-  static bool lds_set = false;  // the attribute is set once per process and kernel
-  if (!lds_set) {
-    const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&gemm_store_kernel<kMode, kAMN, kBMN, kVec>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return static_cast<int>(e);
-    lds_set = true;
-  }
+  static std::atomic<bool> lds_set{false};
+  if (const int rc =
+          allow_lds(reinterpret_cast<const void*>(&gemm_store_kernel<kMode, kAMN, kBMN, kVec>),
+                    kLdsBytes, lds_set))
+    return rc;
   hipLaunchKernelGGL((gemm_store_kernel<kMode, kAMN, kBMN, kVec>), grid, dim3(kThreads),
                      kLdsBytes, stream, A, lda, M, B, ldb, N, K, C, Cf, ldc, ka_rows, kb_rows,
                      splits, ks, split_stride);
@@ -1644,14 +1635,10 @@ inline bool pair_ok(int64_t h) { return h * 4 * 512 < (int64_t{1} << 32); }
 
 template <bool kSplit>
 int launch_pair_as(const PairArgs& p, int64_t blocks, hipStream_t s) {
-  static bool lds_set = false;  // the attribute is set once per process and kernel
-  if (!lds_set) {
-    const hipError_t e =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_pair_kernel<kSplit>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-    if (e != hipSuccess) return static_cast<int>(e);
-    lds_set = true;
-  }
+  static std::atomic<bool> lds_set{false};
+  if (const int rc = allow_lds(reinterpret_cast<const void*>(&gemm_pair_kernel<kSplit>), kLdsBytes,
+                               lds_set))
+    return rc;
   hipLaunchKernelGGL(gemm_pair_kernel<kSplit>, dim3(static_cast<unsigned>(blocks)),
                      dim3(kThreads), kLdsBytes, s, p);
   return launch_status();
@@ -1714,24 +1701,6 @@ struct DirectLayout {
 };
 
 int64_t fwd_partial_blocks(int64_t v) { return (v + kPartialRows - 1) / kPartialRows; }
-
-// Compute units of the current device (256 if the query fails).
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  int n_cu = 256;
-  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
-    if (cus[dev] == 0) {
-      int v = 0;
-      if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-          v > 0)
-        cus[dev] = v;
-    }
-    if (cus[dev] > 0) n_cu = cus[dev];
-  }
-  return n_cu;
-}
-
 
 // K ranges for a product of `tiles` output tiles over K (a multiple of kBK)
 // on `cus` compute units, one 256x256 tile per compute unit at a time: the

@@ -536,6 +536,21 @@ def test_mfma_hazard_scan(body, hazards):
     assert len(mfma_hazards(text)[1]) == hazards, mfma_hazards(text)
 
 
+def test_launchers_keep_no_plain_statics():
+    """What the launchers remember between calls (a kernel's LDS limit set, a
+    device's compute units) is atomic, const or behind a lock: calls come from
+    several threads at once."""
+    import re
+    csrc = ROOT / "nano-megatron_amd" / "csrc"
+    plain = re.compile(r"\s*static (?!const|std::atomic|inline|__device__)|(bool|int|int64_t) \w+ =")
+    text = ""
+    for path in sorted(csrc.glob("*.hip")) + sorted(csrc.glob("*.h")):
+        for i, line in enumerate(path.read_text().splitlines(), 1):
+            assert not plain.match(line), f"{path.name}:{i}: {line.strip()}"
+            text += line + "\n"
+    assert text.count("static std::atomic<") >= 5
+
+
 def test_wide_buffer_stores_go_through_the_helper():
     """Buffer stores wider than 8 bytes are issued only by buffer_store_b128,
     which keeps the scalar offset the constant 0: with a register scalar
