@@ -979,24 +979,28 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
 // a lane whose columns lie past N gets the resource's size as its offset: its
 // accesses are out of range (no memory access, a load reads 0, a store is
 // dropped) whether or not the row step takes part in the check. Every access
-// left is inside the matrix. In modes 2 and 3 half of the 32 loads of Cf
-// are issued before the pass is staged, so their latency runs under the
-// staging, and each of the others as an earlier row leaves. Cf is streamed (non-temporal)
-// both ways. Without kVec the pass leaves element by element.
+// left is inside the matrix. In modes 2 and 3 the 32 loads of Cf are
+// issued before the pass is staged, so that their latency runs under the
+// staging and 128 KiB are in flight. Cf is streamed (non-temporal) both ways.
+// Without kVec the pass leaves element by element.
+// kFull: all of the tile's rows exist, nothing is tested. Behind a branch the
+// compiler cannot count what is in flight and waits for everything, which with
+// each row's load issued behind an earlier row's store was a memory round trip
+// a row. Accumulating launches, us: K = 512 on [16348, 2368] 138 -> 97, on
+// [128256, 4096] 1398 -> 995; K = 4096 on [128256, 4096] 3550 -> 3391 (mode 2),
+// 3507 -> 3227 (mode 3).
 //   kMode 1: Cf = acc;  kMode 2: Cf += acc;  kMode 3: C = bf16(Cf + acc)
-template <int kMode, bool kVec>
-__device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float* __restrict__ Cf,
-                                               uint16_t* __restrict__ C, int64_t ldc, int64_t M,
-                                               int64_t N, int64_t m0, int64_t n0) {
+template <int kMode, bool kVec, bool kFull>
+__device__ __forceinline__ void store_f32_pass(const Acc& acc, int q, char* lds,
+                                               float* __restrict__ Cf, uint16_t* __restrict__ C,
+                                               int64_t ldc, int64_t M, int64_t N, int64_t m0,
+                                               int64_t n0) {
   static_assert(kMode >= 1 && kMode <= 3, "fp32 epilogue modes");
   static_assert(kBN == 256 && kWavesM == 2 && kF == 8 && 128 * kBN * 4 <= kLdsBytes,
                 "two passes of 128 rows fit the stages");
   constexpr int kRowsPerPass = kThreads / 64;  // 4
   constexpr int kPasses = 128 / kRowsPerPass;  // 32
   constexpr int kNt = 2;                       // cache policy: non-temporal
-  // Loads of Cf in flight (the staging needs registers for the accumulators
-  // it moves).
-  constexpr int kEarly = 16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / kWavesN, wn = wave % kWavesN;
@@ -1005,90 +1009,100 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
   const bool col_ok = n0 + 4 * lane < N;
   // Tile rows of staged rows 4 p + wave, relative to the pass's first row.
   auto row_off = [](int p) { return 4 * p + 64 * (p >> 4); };
-  __syncthreads();  // every wave is done with the operand buffers
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int64_t row0 = m0 + 64 * q + wave;  // tile row of staged row `wave`
-    // valid passes: a prefix, rows increase with p
-    int np = 0;
+  const int64_t row0 = m0 + 64 * q + wave;  // tile row of staged row `wave`
+  // valid passes: a prefix, rows increase with p
+  int np = kPasses;
+  if constexpr (!kFull) {
+    np = 0;
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) np += (row0 + row_off(p) < M) ? 1 : 0;
     np = __builtin_amdgcn_readfirstlane(np);
-    const int64_t lim = np == 0 ? 0 : (np < kPasses ? row_off(np) : row_off(kPasses - 1) + 1);
-    const uint32_t vf = col_ok ? static_cast<uint32_t>(lane) * 16u
-                               : static_cast<uint32_t>(lim * ldc * 4);
-    float* cf_base = Cf + (np > 0 ? row0 : 0) * ldc + n0;
-    u32x4 old[kEarly];  // row p's values of Cf in old[p % kEarly], kEarly rows ahead
-    __amdgpu_buffer_rsrc_t rf;
-    if constexpr (kVec) {
-      rf = __builtin_amdgcn_make_buffer_rsrc(cf_base, 0, static_cast<int>(lim * ldc * 4),
-                                             0x00020000);
-      if constexpr (kMode >= 2) {
+  }
+  const int64_t lim = np == 0 ? 0 : (np < kPasses ? row_off(np) : row_off(kPasses - 1) + 1);
+  const uint32_t vf = col_ok ? static_cast<uint32_t>(lane) * 16u
+                             : static_cast<uint32_t>(lim * ldc * 4);
+  float* cf_base = Cf + (np > 0 ? row0 : 0) * ldc + n0;
+  u32x4 old[kPasses];
+  __amdgpu_buffer_rsrc_t rf;
+  if constexpr (kVec) {
+    rf = __builtin_amdgcn_make_buffer_rsrc(cf_base, 0, static_cast<int>(lim * ldc * 4), 0x00020000);
+    if constexpr (kMode >= 2) {
 #pragma unroll
-        for (int p = 0; p < kEarly; ++p) {
-          if (p < np)
-            old[p] = __builtin_amdgcn_raw_buffer_load_b128(
-                rf, vf, static_cast<uint32_t>(row_off(p) * ldc * 4), kNt);
-        }
+      for (int p = 0; p < kPasses; ++p) {
+        if (kFull || p < np)
+          old[p] = __builtin_amdgcn_raw_buffer_load_b128(
+              rf, vf, static_cast<uint32_t>(row_off(p) * ldc * 4), kNt);
       }
     }
+  }
 #pragma unroll
-    for (int j = 0; j < kF; ++j)
+  for (int j = 0; j < kF; ++j)
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const int r = wm * 64 + 16 * f + (lane & 15);
-        const int c = (wn * (kWaveN / 4) + 4 * j + g) ^ (lane & 15);
-        *reinterpret_cast<f32x4_t*>(S + r * kBN + 4 * c) = acc.c[4 * q + f][j];
+    for (int f = 0; f < 4; ++f) {
+      const int r = wm * 64 + 16 * f + (lane & 15);
+      const int c = (wn * (kWaveN / 4) + 4 * j + g) ^ (lane & 15);
+      *reinterpret_cast<f32x4_t*>(S + r * kBN + 4 * c) = acc.c[4 * q + f][j];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < kPasses; ++p) {
+    const int r = p * kRowsPerPass + wave;
+    const u32x4 sv =
+        *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ ((4 * p + wave) & 15)) << 2));
+    if constexpr (!kVec) {
+      const int64_t row = row0 + row_off(p);
+      const float sf[4] = {__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z),
+                           __uint_as_float(sv.w)};
+      for (int j = 0; j < 4; ++j) {
+        const int64_t col = n0 + 4 * lane + j;
+        if (row >= M || col >= N) continue;
+        const int64_t o = row * ldc + col;
+        if constexpr (kMode == 1) Cf[o] = sf[j];
+        if constexpr (kMode == 2) Cf[o] += sf[j];
+        if constexpr (kMode == 3) C[o] = f32_to_bf16(Cf[o] + sf[j]);
       }
-    __syncthreads();
-#pragma unroll
-    for (int p = 0; p < kPasses; ++p) {
-      const int r = p * kRowsPerPass + wave;
-      const u32x4 sv = *reinterpret_cast<const u32x4*>(S + r * kBN + ((lane ^ ((4 * p + wave) & 15)) << 2));
-      if constexpr (!kVec) {
-        const int64_t row = row0 + row_off(p);
-        const float sf[4] = {__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z),
-                             __uint_as_float(sv.w)};
-        for (int j = 0; j < 4; ++j) {
-          const int64_t col = n0 + 4 * lane + j;
-          if (row >= M || col >= N) continue;
-          const int64_t o = row * ldc + col;
-          if constexpr (kMode == 1) Cf[o] = sf[j];
-          if constexpr (kMode == 2) Cf[o] += sf[j];
-          if constexpr (kMode == 3) C[o] = f32_to_bf16(Cf[o] + sf[j]);
-        }
+    } else {
+      if (!kFull && p >= np) continue;
+      const uint32_t so = static_cast<uint32_t>(row_off(p) * ldc * 4);
+      if constexpr (kMode == 1) {
+        buffer_store_b128<kNt>(sv, rf, vf + so);
       } else {
-        if (p >= np) continue;
-        const uint32_t so = static_cast<uint32_t>(row_off(p) * ldc * 4);
-        if constexpr (kMode == 1) {
-          buffer_store_b128<kNt>(sv, rf, vf + so);
+        const u32x4 o = old[p];
+        const float v0 = __uint_as_float(sv.x) + __uint_as_float(o.x);
+        const float v1 = __uint_as_float(sv.y) + __uint_as_float(o.y);
+        const float v2 = __uint_as_float(sv.z) + __uint_as_float(o.z);
+        const float v3 = __uint_as_float(sv.w) + __uint_as_float(o.w);
+        if constexpr (kMode == 2) {
+          buffer_store_b128<kNt>(
+              u32x4{__float_as_uint(v0), __float_as_uint(v1), __float_as_uint(v2),
+                    __float_as_uint(v3)},
+              rf, vf + so);
         } else {
-          const u32x4 o = old[p % kEarly];
-          if (p + kEarly < np)
-            old[p % kEarly] = __builtin_amdgcn_raw_buffer_load_b128(
-                rf, vf, static_cast<uint32_t>(row_off(p + kEarly) * ldc * 4), kNt);
-          const float v0 = __uint_as_float(sv.x) + __uint_as_float(o.x);
-          const float v1 = __uint_as_float(sv.y) + __uint_as_float(o.y);
-          const float v2 = __uint_as_float(sv.z) + __uint_as_float(o.z);
-          const float v3 = __uint_as_float(sv.w) + __uint_as_float(o.w);
-          if constexpr (kMode == 2) {
-            buffer_store_b128<kNt>(
-                u32x4{__float_as_uint(v0), __float_as_uint(v1), __float_as_uint(v2),
-                      __float_as_uint(v3)},
-                rf, vf + so);
-          } else {
-            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-            const auto rh = __builtin_amdgcn_make_buffer_rsrc(
-                C + (np > 0 ? row0 : 0) * ldc + n0, 0, static_cast<int>(lim * ldc * 2), 0x00020000);
-            __builtin_amdgcn_raw_buffer_store_b64(
-                u32x2{pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)}, rh,
-                col_ok ? static_cast<uint32_t>(lane) * 8u : static_cast<uint32_t>(lim * ldc * 2),
-                static_cast<uint32_t>(row_off(p) * ldc * 2), 0);
-          }
+          typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+          const auto rh = __builtin_amdgcn_make_buffer_rsrc(
+              C + (np > 0 ? row0 : 0) * ldc + n0, 0, static_cast<int>(lim * ldc * 2), 0x00020000);
+          __builtin_amdgcn_raw_buffer_store_b64(
+              u32x2{pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)}, rh,
+              col_ok ? static_cast<uint32_t>(lane) * 8u : static_cast<uint32_t>(lim * ldc * 2),
+              static_cast<uint32_t>(row_off(p) * ldc * 2), 0);
         }
       }
     }
-    __syncthreads();  // the next pass reuses S
+  }
+  __syncthreads();  // the next pass reuses S
+}
+
+template <int kMode, bool kVec>
+__device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float* __restrict__ Cf,
+                                               uint16_t* __restrict__ C, int64_t ldc, int64_t M,
+                                               int64_t N, int64_t m0, int64_t n0) {
+  __syncthreads();  // every wave is done with the operand buffers
+  if (kVec && m0 + kBM <= M) {
+    store_f32_pass<kMode, kVec, true>(acc, 0, lds, Cf, C, ldc, M, N, m0, n0);
+    store_f32_pass<kMode, kVec, true>(acc, 1, lds, Cf, C, ldc, M, N, m0, n0);
+  } else {
+    store_f32_pass<kMode, kVec, false>(acc, 0, lds, Cf, C, ldc, M, N, m0, n0);
+    store_f32_pass<kMode, kVec, false>(acc, 1, lds, Cf, C, ldc, M, N, m0, n0);
   }
 }
 

@@ -489,21 +489,44 @@ def test_one_pass_ragged_route(lib):
     assert rs(p, 1, 4, 9, 9, None, p, None, None) == -4
 
 
-def test_gemm_mfmas_keep_their_wait_states(tmp_path):
+@pytest.fixture(scope="module")
+def lmhead_asm(tmp_path_factory):
+    """The generated code of nmce_lmhead.hip, as the build compiles it."""
+    import subprocess
+
+    from nmce import _build
+    asm = tmp_path_factory.mktemp("asm") / "lmhead.s"
+    subprocess.run([_build.hipcc(), *_build.HIPCC_FLAGS, "-S", "--cuda-device-only",
+                    str(_build.CSRC_DIR / "nmce_lmhead.hip"), "-o", str(asm)], check=True,
+                   capture_output=True)
+    return asm.read_text()
+
+
+@pytest.mark.parametrize("mode", [2, 3])
+def test_accumulating_epilogue_keeps_its_loads_in_flight(lmhead_asm, mode):
+    """Whole tiles of the products that add to an fp32 accumulator: each of the
+    two passes issues its 32 loads of it with no branch or wait between them,
+    and the rows that leave then wait for one load at a time (a wait for all,
+    which is what the compiler writes behind a branch, costs a round trip to
+    memory a row)."""
+    import re
+    body = re.search(rf"^_Z\w*gemm_store_kernelILi{mode}ELb0ELb0ELb1E\w*:(.*?)\.end_amdhsa_kernel",
+                     lmhead_asm, re.S | re.M)[1]
+    seen = re.findall(r"^\s+(buffer_load_dwordx4 (?!.* lds)|s_cbranch|s_barrier|s_waitcnt .*"
+                      r"vmcnt\((\d+)\))", body, re.M)
+    kinds = "".join("L" if k.startswith("buffer") else "B" if k.startswith("s_b") else
+                    "C" if k.startswith("s_c") else "w" if int(n) >= 16 else "W" for k, n in seen)
+    assert len(re.findall(r"(?<!L)L{32}Bw+(?=B|L|C|$)", kinds)) == 2, kinds
+
+
+def test_gemm_mfmas_keep_their_wait_states(lmhead_asm):
     """The GEMM core's MFMAs are inline asm, around which the compiler puts no
     wait states. In the generated code no VALU instruction writes a source of
     an MFMA within two wait states before it, and none touches the registers
     that one wrote within 16 wait states after it, along every path (a loop's
     back edge is where a compiler would move a fragment's registers)."""
-    import subprocess
-
     from _util import mfma_hazards
-    from nmce import _build
-    asm = tmp_path / "lmhead.s"
-    subprocess.run([_build.hipcc(), *_build.HIPCC_FLAGS, "-S", "--cuda-device-only",
-                    str(_build.CSRC_DIR / "nmce_lmhead.hip"), "-o", str(asm)], check=True,
-                   capture_output=True)
-    mfmas, offenders = mfma_hazards(asm.read_text())
+    mfmas, offenders = mfma_hazards(lmhead_asm)
     assert mfmas > 1000
     assert not offenders, offenders[:5]
 
