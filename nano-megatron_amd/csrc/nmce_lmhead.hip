@@ -332,23 +332,12 @@ struct Frags {
 // kRows hands the MFMA its operands the other way round, which gives the lane
 // four columns of one row instead of four rows of one column (the same sums):
 // what an epilogue wants that stores rows.
-//
-// touch(i), i = 0 .. kTouches - 1, is called in every second one of the last K
-// steps that load a whole stage (as many as there are): a load whose value
-// nobody needs, that brings a part of what the epilogue will read nearer
-// (TouchTile). It is issued behind the step's A loads, so that step's wait
-// leaves nine in flight and it has a whole K step to come back.
-constexpr int kTouches = 8;
-struct NoTouch {
-  __device__ __forceinline__ uint32_t operator()(int) const { return 0; }
-};
-template <bool kAMN, bool kBMN, bool kRows = false, typename Touch = NoTouch>
+template <bool kAMN, bool kBMN, bool kRows = false>
 __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, int64_t lda,
                                               int64_t M, const uint16_t* __restrict__ B,
                                               int64_t ldb, int64_t N, int64_t K, int64_t m0,
                                               int64_t n0, char* lds, Acc& acc,
-                                              int64_t ka_rows = 0, int64_t kb_rows = 0,
-                                              Touch touch = {}) {
+                                              int64_t ka_rows = 0, int64_t kb_rows = 0) {
   const int lane = threadIdx.x & 63;
   // The wave index is uniform across the wave; say so, so that the load
   // bases and LDS destinations below live in scalar registers.
@@ -458,19 +447,13 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
   const int full_a = la.full_stages(kt_n), full_b = lb.full_stages(kt_n);
   const int full = full_a < full_b ? full_a : full_b;
   int kt = 0;
-  auto k_step = [&](auto touching, int i) {
+  for (; kt + 2 < full; ++kt) {
     const int a_nxt = next_a(a_cur);
     const int b_cur = (kt & 1) * kStage;
     char* da = lds + prev_a(a_cur) + lds_w;
     la.at(kt + 2);
     step(lds + a_cur, lds_b + b_cur, 1, f1, f0, Loads{}, [&](int l) { la.load(da, l); });
-    uint32_t t = 0;
-    if constexpr (touching.value) {
-      t = touch(i);
-      asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-    }
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     char* db = lds_b + b_cur + lds_w;
@@ -478,21 +461,6 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
     step(lds + a_nxt, lds_b + (kStage - b_cur), 0, f0, f1, Loads{},
          [&](int l) { lb.load(db, l); });
     a_cur = a_nxt;
-    return t;
-  };
-  constexpr bool kTouch = !std::is_same<Touch, NoTouch>::value;
-  for (; kt + 2 + (kTouch ? 2 * kTouches : 0) < full; ++kt) k_step(std::false_type{}, 0);
-  if constexpr (kTouch) {
-    for (int i = 0; kt + 3 < full; ++kt, ++i) {
-      const uint32_t t = k_step(std::true_type{}, i);
-      ++kt;
-      k_step(std::false_type{}, 0);
-      asm volatile("" ::"v"(t));  // back since this step's wait
-    }
-    if (kt + 2 < full) {
-      k_step(std::false_type{}, 0);
-      ++kt;
-    }
   }
   static_assert(kBlocksPerWave == 8, "the loop's wait leaves one stage's A loads in flight");
   for (; kt + 1 < kt_n; ++kt) {
@@ -976,19 +944,22 @@ __global__ __launch_bounds__(kThreads, 1) void lmhead_dz_kernel(
 // offset of the loads (the 16-byte stores take it in the per-lane offset:
 // buffer_store_b128). The hardware range check covers the per-lane offset
 // only, so rows past M (passes p >= np, uniform) are skipped explicitly, and
-// a lane whose columns lie past N gets the resource's size as its offset: its
-// accesses are out of range (no memory access, a load reads 0, a store is
-// dropped) whether or not the row step takes part in the check. Every access
-// left is inside the matrix. In modes 2 and 3 the 32 loads of Cf are
+// a lane whose columns lie past N gets the offset 2^31, more than a resource's
+// size and no row step takes it past 32 bits: its accesses are out of range (no
+// memory access, a load reads 0, a store is dropped) whether or not the row
+// step takes part in the check. (As a product of the row stride it made the
+// compiler carry the stride in a lane register and loop over its values at
+// every load.) Every access left is inside the matrix. In modes 2 and 3 the 32 loads of Cf are
 // issued before the pass is staged, so that their latency runs under the
 // staging and 128 KiB are in flight. Cf is streamed (non-temporal) both ways.
 // Without kVec the pass leaves element by element.
 // kFull: all of the tile's rows exist, nothing is tested. Behind a branch the
 // compiler cannot count what is in flight and waits for everything, which with
 // each row's load issued behind an earlier row's store was a memory round trip
-// a row. Accumulating launches, us: K = 512 on [16348, 2368] 138 -> 97, on
-// [128256, 4096] 1398 -> 995; K = 4096 on [128256, 4096] 3550 -> 3391 (mode 2),
-// 3507 -> 3227 (mode 3).
+// a row. Accumulating launches, us: K = 512 on [16348, 2368] 138 -> 95, on
+// [128256, 4096] 1383 -> 924; K = 4096 on [128256, 4096] 3531 -> 3255 (mode 2),
+// 3469 -> 3121 (mode 3). With the loads in flight, reading the tile's lines
+// ahead under the last K steps only costs: 3348 and 3197.
 //   kMode 1: Cf = acc;  kMode 2: Cf += acc;  kMode 3: C = bf16(Cf + acc)
 template <int kMode, bool kVec, bool kFull>
 __device__ __forceinline__ void store_f32_pass(const Acc& acc, int q, char* lds,
@@ -1001,6 +972,7 @@ __device__ __forceinline__ void store_f32_pass(const Acc& acc, int q, char* lds,
   constexpr int kRowsPerPass = kThreads / 64;  // 4
   constexpr int kPasses = 128 / kRowsPerPass;  // 32
   constexpr int kNt = 2;                       // cache policy: non-temporal
+  constexpr uint32_t kPast = 1u << 31;         // a lane past N: beyond every resource here
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / kWavesN, wn = wave % kWavesN;
@@ -1019,8 +991,7 @@ __device__ __forceinline__ void store_f32_pass(const Acc& acc, int q, char* lds,
     np = __builtin_amdgcn_readfirstlane(np);
   }
   const int64_t lim = np == 0 ? 0 : (np < kPasses ? row_off(np) : row_off(kPasses - 1) + 1);
-  const uint32_t vf = col_ok ? static_cast<uint32_t>(lane) * 16u
-                             : static_cast<uint32_t>(lim * ldc * 4);
+  const uint32_t vf = col_ok ? static_cast<uint32_t>(lane) * 16u : kPast;
   float* cf_base = Cf + (np > 0 ? row0 : 0) * ldc + n0;
   u32x4 old[kPasses];
   __amdgpu_buffer_rsrc_t rf;
@@ -1083,7 +1054,7 @@ __device__ __forceinline__ void store_f32_pass(const Acc& acc, int q, char* lds,
               C + (np > 0 ? row0 : 0) * ldc + n0, 0, static_cast<int>(lim * ldc * 2), 0x00020000);
           __builtin_amdgcn_raw_buffer_store_b64(
               u32x2{pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)}, rh,
-              col_ok ? static_cast<uint32_t>(lane) * 8u : static_cast<uint32_t>(lim * ldc * 2),
+              col_ok ? static_cast<uint32_t>(lane) * 8u : kPast,
               static_cast<uint32_t>(row_off(p) * ldc * 2), 0);
         }
       }
@@ -1105,34 +1076,6 @@ __device__ __forceinline__ void store_f32_tile(const Acc& acc, char* lds, float*
     store_f32_pass<kMode, kVec, false>(acc, 1, lds, Cf, C, ldc, M, N, m0, n0);
   }
 }
-
-// A part of the fp32 tile that store_f32_tile will add to, read ahead: touch i
-// reads one value of each of 2048 / kTouches 128-byte lines (a thread each) of
-// the tile's rows 32 i .. 32 i + 31. The lines come from HBM while the matrix
-// units work, and the epilogue's loads, all compute units' at once, find them
-// in the caches: [16384, 4096] x [128256, 4096] in four chunks 38.36 -> 38.21
-// ms, in eight consecutive steps as in every second one. Offsets past the matrix are out of the resource's range (no
-// access); the columns past N of a row before the last are the next row's.
-// The caller has checked that 512 rows lie within 32-bit offsets.
-struct TouchTile {
-  __amdgpu_buffer_rsrc_t rsrc;
-  uint32_t off, step;
-  __device__ __forceinline__ void init(const float* Cf, int64_t ldc, int64_t M, int64_t N,
-                                       int64_t m0, int64_t n0) {
-    const int64_t rows = (M - m0) < kBM ? (M - m0) : kBM;
-    const int64_t cols = (N - n0) < kBN ? (N - n0) : kBN;
-    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Cf) + m0 * ldc + n0, 0,
-                                             static_cast<int>(((rows - 1) * ldc + cols) * 4),
-                                             0x00020000);
-    const uint32_t row_bytes = static_cast<uint32_t>(ldc * 4);
-    off = (threadIdx.x >> 3) * row_bytes + (threadIdx.x & 7) * 128u;
-    step = (kThreads / 8) * row_bytes;
-  }
-  __device__ __forceinline__ uint32_t operator()(int i) const {
-    return __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + static_cast<uint32_t>(i) * step, 0, 0);
-  }
-};
-static_assert(kTouches * (kThreads / 8) == kBM && kBN * 4 == 8 * 128, "the touches cover a tile");
 
 // bf16 out: rows of 512 bytes whose 16-byte chunk c sits at c ^ (row & 15):
 // the 16 rows of a block that 32 lanes write 8 bytes of each are on distinct
@@ -1231,15 +1174,8 @@ __device__ __forceinline__ void gemm_store_tile(
   const uint16_t* Bs = kBMN ? B + k0 * ldb : B + k0;
   Cf += split * split_stride;
   Acc acc;
-  if constexpr (kMode >= 2 && kVec) {
-    TouchTile touch;
-    touch.init(Cf, ldc, M, N, m0, n0);
-    gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
-                                              ka_rows - k0, kb_rows - k0, touch);
-  } else {
-    gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
-                                              ka_rows - k0, kb_rows - k0);
-  }
+  gemm_mainloop<kAMN, kBMN, /*kRows=*/true>(As, lda, M, Bs, ldb, N, kl, m0, n0, lds, acc,
+                                            ka_rows - k0, kb_rows - k0);
   if constexpr (kMode != 0)
     store_f32_tile<kMode, kVec>(acc, lds, Cf, C, ldc, M, N, m0, n0);
   else
