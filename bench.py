@@ -424,7 +424,7 @@ def run_fused(args, name: str, steps: int, warmup: int, one_pass: bool = True,
     xp = x.requires_grad_(True)
     wp = w.requires_grad_(True)
     token_chunk = n if one_chunk else args.token_chunk
-    chunk = token_chunk if token_chunk is not None else lmhead.default_token_chunk(n, v)
+    chunk = token_chunk if token_chunk is not None else lmhead.one_pass_token_chunk(n, h, v)
     counter = [0]
 
     def run_steps(k):
