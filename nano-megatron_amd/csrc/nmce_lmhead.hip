@@ -2,9 +2,9 @@
 //
 // Replaces ParallelLMHead's projection Z = X @ W^T (nano_megatron/model.py:192,
 // run in bf16 under autocast, model.py:255-257) followed by the loss of
-// nano_megatron/cross_entropy.py:16-65, without ever holding Z (or anything of
-// its size) for every token: at most one chunk of tokens' exponentials, or one
-// vocabulary chunk's gradient, at a time.
+// nano_megatron/cross_entropy.py:16-65, without ever storing Z: at most one
+// chunk of tokens' bf16 exponentials (the caller's choice of chunk, up to every
+// token), or one vocabulary chunk's gradient, at a time.
 //
 // Every product is one bf16 GEMM core, C[m, n] = sum_k A[m, k] * B[n, k] on
 // v_mfma_f32_16x16x32_bf16, each operand K-contiguous or MN-contiguous
@@ -24,7 +24,8 @@
 //                                     the tiles are few)
 //
 // The one-pass path (the drop-in's default) computes Z once, per chunk of
-// tokens (the caller's choice; the drop-in takes a quarter of the tokens):
+// tokens (the caller's choice; the drop-in takes a quarter of the tokens, or all
+// of them where that whole workspace is no larger):
 //             P^T  = exp(W X^T - block max), bf16, with the partial statistics
 //             dZ^T = P^T * exp(block max - M) * g / S - onehot, in place
 //                    (once the statistics are combined)
@@ -374,6 +375,9 @@ __device__ __forceinline__ void gemm_mainloop(const uint16_t* __restrict__ A, in
 #pragma unroll
     for (int j = 0; j < kF; ++j) asm volatile("" : "+a"(acc.c[i][j]));
   asm volatile("s_nop 7" ::: "memory");
+  // Stage 0 is what the first reads need; the compiler puts a wait for nearly
+  // all loads in flight before the barrier of its own accord, stage 1's among
+  // them.
   if (kt_n > 1)
     asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
   else
@@ -652,7 +656,9 @@ __device__ __forceinline__ void column_stats(const Acc& acc, int j0, int g, int 
 }
 
 // Columns whose statistics are formed together: two columns' 64 values and
-// their exponentials fit the registers beside the accumulators.
+// their exponentials beside the 256 accumulators take all 512 registers, and the
+// compiler spills one or two more (8 bytes of scratch a lane in lmhead_p_kernel,
+// 12 in lmhead_stats_kernel).
 constexpr int kStatCols = 2;
 
 // The partial statistics of the wave's 128 rows x 128 tokens, written for the

@@ -198,7 +198,7 @@ def test_lmhead_workspace_layout(lib):
 
 
 def test_default_chunk_never_holds_full_logits(lib):
-    """The drop-in's default one-pass path at the fused workloads (c4: 16384
+    """The drop-in's own one-pass chunk at the fused workloads (c4: 16384
     tokens x 128256 rows, H 4096; c5: 16384 x 256000, H 3072) allocates no
     buffer of the [tokens, V] logits' size: the workspace's one chunk-sized
     buffer, P^T, holds a quarter of the tokens (4096), its largest buffer is
@@ -211,7 +211,7 @@ def test_default_chunk_never_holds_full_logits(lib):
     buf = (ctypes.c_int64 * L.NMCE_LMHEAD_FUSED_LAYOUT_FIELDS)()
     for n, h, v in ((16384, 4096, 128256), (16384, 3072, 256000)):
         logits_bytes = n * v * 2  # the bf16 logits
-        chunk = lmhead.default_token_chunk(n, v)
+        chunk = lmhead.one_pass_token_chunk(n, h, v)
         assert chunk == 4096
         assert lib.nmce_lmhead_ce_fused_layout(n, h, v, chunk, ctypes.addressof(buf)) == 0
         total, got_chunk, n_chunks = buf[0], buf[1], buf[2]
