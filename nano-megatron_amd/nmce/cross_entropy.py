@@ -472,21 +472,28 @@ def vocab_parallel_cross_entropy(
     ``inplace=True`` writes the gradient into the logits' storage (the call
     site at model.py:277-281 can: the LM head's output is read by nothing
     else); ``None`` (default) does so only from the two-pass backward, for
-    non-leaf logits; ``False`` never does.
+    non-leaf logits; ``False`` never does. So with ``None`` a call that takes
+    the one-pass path holds a second slab of the logits' size from its forward
+    to its backward, whatever its rows' width, where the two-pass path would
+    have reused the logits': ``inplace=True`` or ``one_pass=False`` where that
+    memory counts.
 
     At TP = 1, when a gradient is wanted (grad mode on, logits requiring grad)
     and the rows fit the one-pass kernel (at most 131072 bf16 or 65536 fp32
-    columns; without ``inplace=True`` also rows that lie as a new contiguous
-    buffer's would against 16-byte boundaries), the forward reads the logits once and also writes their gradient, for the
-    upstream value the previous backward of this call site received (1.0 at
-    first): in place with ``inplace=True`` (the logits hold the gradient once
-    the forward returns), else into a new buffer. The backward redoes it only
-    when its upstream value differs: bit-identical to the two-pass path, which
-    ``one_pass=False`` selects, for a new buffer; rescaled, within four fp32
+    columns, even or odd; without ``inplace=True`` also rows that lie as a new
+    contiguous buffer's would against 16-byte boundaries), the forward reads
+    the logits once and also writes their gradient, for the upstream value the
+    previous backward of this call site received (1.0 at first): in place with
+    ``inplace=True`` (the logits hold the gradient once the forward returns),
+    else into a new buffer. The backward redoes it only when its upstream value
+    differs: bit-identical to the two-pass path, which ``one_pass=False``
+    selects, for a new buffer; rescaled, within four fp32
     or two bf16 units in the last place, in place. ``upstream_hint`` (a
     one-element fp32 device tensor) replaces the call site's value: the
     forward assumes what it holds and the backward stores what it receives
-    there.
+    there. A call site whose upstream value changes at every step pays for a
+    gradient that the backward writes again, 1.1 to 1.5 times the two-pass
+    path's time: give it the value in ``upstream_hint``, or ``one_pass=False``.
 
     A target outside the vocabulary raises the reference's ``ValueError``
     before this returns, and the logits are left as they were: on the
