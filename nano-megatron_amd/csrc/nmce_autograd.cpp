@@ -130,7 +130,7 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
           reinterpret_cast<const int32_t*>(bad_flag), static_cast<float>(n), st);
     });
     ctx->saved_data["inplace"] = inplace;
-    ctx->saved_data["ld"] = ld;
+    ctx->saved_data["hint"] = hint;  // itself: the backward writes into it
     ctx->saved_data["vocab_start"] = vocab_start;
     ctx->saved_data["handed_out"] = false;
     ctx->saved_data["shape"] = logits.sizes().vec();
@@ -139,9 +139,10 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
       // their version check rather than read it.
       torch::autograd::impl::bump_version(logits);
       ctx->saved_data["grad_buf"] = logits.detach();
-      ctx->save_for_backward({target, row_stat, assumed, hint});
+      ctx->saved_data["ld"] = ld;
+      ctx->save_for_backward({target, row_stat, assumed});
     } else {
-      ctx->save_for_backward({rows, target, row_stat, grad, assumed, hint});
+      ctx->save_for_backward({rows, target, row_stat, grad, assumed});
     }
     return loss.mean();
   }
@@ -152,7 +153,7 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
     if (go.scalar_type() != at::kFloat) go = go.to(at::kFloat);
     go = go.contiguous();
     const bool inplace = ctx->saved_data["inplace"].toBool();
-    const int64_t ld = ctx->saved_data["ld"].toInt();
+    const at::Tensor hint = ctx->saved_data["hint"].toTensor();
     const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
     const int64_t V = shape.back();
     const variable_list saved = ctx->get_saved_variables();
@@ -163,9 +164,8 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
                   "which now hold the gradient; pass inplace=False to differentiate it twice");
       const at::Tensor& target = saved[0];
       const at::Tensor& assumed = saved[2];
-      const at::Tensor& hint = saved[3];
       at::Tensor grad = ctx->saved_data["grad_buf"].toTensor();
-      const int64_t n = target.numel();
+      const int64_t n = target.numel(), ld = ctx->saved_data["ld"].toInt();
       hipStream_t st = stream_of(grad);
       const bool ragged = is_ragged(grad, V, ld);
       timed(ragged ? "nmce_ce_grad_rescale_unless_ragged" : "nmce_ce_grad_rescale_unless", st, [&] {
@@ -178,13 +178,14 @@ struct OnePassMean : public torch::autograd::Function<OnePassMean> {
       grads[0] = grad;
       return grads;
     }
-    const at::Tensor& rows = saved[0];
+    // Saved-tensor hooks may hand back copies of other strides.
+    const at::Tensor rows = V > 1 && saved[0].stride(1) != 1 ? saved[0].contiguous() : saved[0];
     const at::Tensor& target = saved[1];
     const at::Tensor& row_stat = saved[2];
-    const at::Tensor& grad = saved[3];
+    const at::Tensor grad = saved[3].contiguous();
     const at::Tensor& assumed = saved[4];
-    const at::Tensor& hint = saved[5];
     const int64_t n = rows.size(0);
+    const int64_t ld = n > 1 ? rows.stride(0) : V;
     const int64_t vocab_start = ctx->saved_data["vocab_start"].toInt();
     const float gdiv = static_cast<float>(n > 1 ? n : 1);
     hipStream_t st = stream_of(rows);

@@ -282,7 +282,6 @@ def _ce_forward(ctx, logits, target, vocab_start, vocab_end, group, world_size, 
     ctx.inplace = bool(inplace)
     ctx.vocab_start = vocab_start
     ctx.logits_shape = logits.shape
-    ctx.ld = ld
     # `rows` aliases `logits` unless a contiguous copy was made above.
     ctx.save_for_backward(rows, tgt, row_stat, logits if ctx.inplace else None)
     return loss
@@ -361,14 +360,20 @@ def _ce_backward(ctx, go, gstride, gdiv):
     rows, tgt, row_stat, original = ctx.saved_tensors
     lib = _lib.load()
     n, V = rows.shape
-    if ctx.inplace:
-        out = rows
-        ld_out = ctx.ld
-    else:
+    # Saved-tensor hooks may hand back copies of other strides, and the rows
+    # and the logits as two of them: the gradient goes into the one returned.
+    if V > 1 and rows.stride(1) != 1:
+        rows = rows.contiguous()
+    ld = rows.stride(0) if n > 1 else V
+    out = _as_rows(original) if ctx.inplace else None
+    if ctx.inplace and out is None:
+        original = original.contiguous()
+        out = original.view(-1, V)
+    if out is None:
         out = torch.empty((n, V), dtype=rows.dtype, device=rows.device)
-        ld_out = V
+    ld_out = out.stride(0) if n > 1 else V
     _launch("nmce_ce_bwd_scaled", lib.nmce_ce_bwd_scaled,
-            rows.data_ptr(), out.data_ptr(), _lib.dtype_code(rows.dtype), n, V, ctx.ld, ld_out,
+            rows.data_ptr(), out.data_ptr(), _lib.dtype_code(rows.dtype), n, V, ld, ld_out,
             tgt.data_ptr(), ctx.vocab_start, row_stat[0].data_ptr(), row_stat[1].data_ptr(),
             go.data_ptr(), gstride, gdiv, _lib.stream_handle(rows.device))
     if ctx.inplace:

@@ -17,6 +17,8 @@ Tolerances (stated per test):
 
 from __future__ import annotations
 
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -960,6 +962,45 @@ def test_one_pass_ragged_in_place_strided(dtype):
     with pytest.raises(ValueError, match="outside the model vocabulary"):
         nmce.vocab_parallel_cross_entropy(logits, bad, 0, v, ctx, inplace=True)
     assert torch.equal(buf, store)
+
+
+@pytest.mark.parametrize("v", [1000, 999])
+@pytest.mark.parametrize("one_pass,inplace,leaf", [(True, None, True), (True, None, False),
+                                                   (True, True, False), (False, None, True),
+                                                   (False, None, False), (False, True, False)])
+def test_saved_tensor_hooks(one_pass, inplace, leaf, v):
+    """Saved-tensor hooks that hand back copies (save_on_cpu): rows of a padded
+    stride come back contiguous, and the rows and the logits as two tensors. The
+    gradient is the one without hooks, after a hit, a miss and, into a separate
+    buffer, a second backward; the value received reaches the caller's hint."""
+    import nmce
+    ctx = nmce.ParallelContext.single()
+    n, pad = 37, 24
+    print(f"[gpu] saved-tensor hooks v={v} {one_pass} {inplace} {leaf}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(v)
+    store = (torch.randn(n, v + pad, device=DEV, generator=g) * 2.0).to(torch.bfloat16)
+    t = torch.randint(0, v, (n,), device=DEV, generator=g)
+    for upstreams in ((1.0,), (0.5,), (1.0, 0.25)):
+        if len(upstreams) > 1 and (inplace or not (leaf or one_pass)):
+            continue  # logits that hold their gradient are not differentiated twice
+        grads = []
+        for hooks in (False, True):
+            hint = torch.ones(1, device=DEV)
+            rows = store.clone()[:, :v]
+            logits = rows.requires_grad_(True) if leaf else _Alias.apply(
+                torch.zeros(1, device=DEV, dtype=store.dtype, requires_grad=True), rows)
+            got = []
+            logits.register_hook(lambda g: got.append(g.clone()))
+            with torch.autograd.graph.save_on_cpu() if hooks else contextlib.nullcontext():
+                loss = nmce.vocab_parallel_cross_entropy(logits, t, 0, v, ctx, inplace=inplace,
+                                                         one_pass=one_pass, upstream_hint=hint)
+            assert ("OnePassMean" in loss.grad_fn.name()) == one_pass
+            for u in upstreams:
+                (loss * u).backward(retain_graph=len(upstreams) > 1)
+            assert hint.item() == (upstreams[0] if one_pass else 1.0)
+            grads.append(got)
+        for a, b in zip(*grads):
+            assert b.abs().sum() > 0 and torch.equal(a, b), upstreams
 
 
 class _Alias(torch.autograd.Function):
