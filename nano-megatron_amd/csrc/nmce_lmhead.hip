@@ -1663,7 +1663,9 @@ int64_t fwd_partial_blocks(int64_t v) { return (v + kPartialRows - 1) / kPartial
 // fewest ranges (at most 8, each at least 2048 long, each holding some of the
 // first `k_valid` k) whose rounds of tiles leave at most 5% of the compute
 // units idle, else the fewest with the least idle share. ks gets the range
-// length (a multiple of kBK).
+// length (a multiple of kBK). The product is counted by itself,
+// also where gemm_pair_kernel's other tiles would fill the idle units: fewer
+// ranges may do there, which has not been measured.
 //
 // Where even 8 ranges leave part of one round idle (fewer than 32 tiles on
 // 256 compute units: small batches, whose K is the whole vocabulary), the
